@@ -6,7 +6,7 @@
 // and B[k0+l/16][l%16]; accumulator item t of lane l is C[r][l%16] with r = 4*(l/16)+t for f32
 // and r = l/16 + 4t for f64.
 //
-// Two kernels share that structure:
+// Three kernels; the first and last share that structure:
 //  * gemm_dl_kernel (every launch with op(B) = B or B^T, and symmetric B when the caller
 //    supplies full copies of its diagonal blocks): buffer loads write LDS directly
 //    (buffer_load_dword ... lds), so slices need no register staging; kStages slices are in
@@ -14,12 +14,13 @@
 //    descriptors' range checks zero-fill what lies past the matrix (the range includes the
 //    scalar offset on gfx950, so every column gets a descriptor of its own).  Measured
 //    16384^3 FP64: 74 TF/s (94% of the MFMA peak).
+//  * gemm_direct_kernel (launches too small to fill the chip, direct_rows below): operands from
+//    global memory straight into MFMA registers, no LDS and no barriers.
 //  * gemm_kernel (fallback: symmetric B without diagonal copies, K x N slabs whose byte
 //    offsets would overflow 32 bits): register-staged, double-buffered LDS, the next slice's
 //    global loads issued before the current slice's MFMAs.
-// A launch with fewer than two 128-row tiles per CU (panel solves of the leaves, narrow
-// updates) uses 64-row tiles (each wave 32x64, up to 4 workgroups per CU), which doubles the
-// workgroups that fill the device.
+// A slice launch with fewer than two 128-row tiles per CU uses 64-row tiles (each wave 32x64, up
+// to 4 workgroups per CU), which doubles the workgroups that fill the device.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -470,6 +471,204 @@ __global__ void __launch_bounds__(NT, TM == 128 ? 2 : 4) gemm_dl_kernel(GemmArgs
     }
 }
 
+// 4x4 transpose between four registers and the four 16-lane rows of a wave: lane row q's
+// register t becomes lane row t's register q (gfx950 row swaps; no LDS).
+__device__ __forceinline__ void swap_rows(unsigned (&x)[4]) {
+    auto p = __builtin_amdgcn_permlane32_swap(x[0], x[2], false, false);
+    auto q = __builtin_amdgcn_permlane32_swap(x[1], x[3], false, false);
+    auto r = __builtin_amdgcn_permlane16_swap(p[0], q[0], false, false);
+    auto s = __builtin_amdgcn_permlane16_swap(p[1], q[1], false, false);
+    x[0] = r[0];
+    x[1] = r[1];
+    x[2] = s[0];
+    x[3] = s[1];
+}
+template <typename T>
+__device__ __forceinline__ void lane_rows_transpose(T& a, T& b, T& c, T& d) {
+    constexpr int W = sizeof(T) / 4;
+    unsigned v[4][W], x[4];
+    __builtin_memcpy(v[0], &a, sizeof(T));
+    __builtin_memcpy(v[1], &b, sizeof(T));
+    __builtin_memcpy(v[2], &c, sizeof(T));
+    __builtin_memcpy(v[3], &d, sizeof(T));
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+        for (int t = 0; t < 4; ++t) x[t] = v[t][w];
+        swap_rows(x);
+        for (int t = 0; t < 4; ++t) v[t][w] = x[t];
+    }
+    __builtin_memcpy(&a, v[0], sizeof(T));
+    __builtin_memcpy(&b, v[1], sizeof(T));
+    __builtin_memcpy(&c, v[2], sizeof(T));
+    __builtin_memcpy(&d, v[3], sizeof(T));
+}
+
+// Direct kernel for launches too small to hide the slice pipeline above: a K = 128 product is
+// 16 slices there, each a barrier and a share of the load latency.  Here no LDS and no barrier
+// stand between the loads and the MFMAs: every wave loads its A and op(B) fragments from global
+// memory (L2 for all but the first reader) straight into the MFMA operand registers, D chunks of
+// 16 k ahead.  An FP64 16x16x4 MFMA takes 64 cycles, so a wave's 16*WM x 32 block keeps
+// its matrix core fed from L1/L2.  The workgroup is 16*WM rows x 128 columns, its four waves side
+// by side, so an in-place product with N <= 128 needs one barrier before the stores.
+// The operands enter the MFMA swapped (op(B)^T first), so a lane holds 4 columns of one row and 16
+// lanes store 128 contiguous bytes of a column; products and their k order are those of the
+// kernel above, so both give the same bits.
+__device__ const int never_skip = 0;
+
+template <typename T, int TB, int WM, int D>
+__global__ void __launch_bounds__(NT) gemm_direct_kernel(GemmArgs<T> g) {
+    using acc_t = typename Mfma<T>::acc_t;
+    constexpr int WN = 2;              // 16-column MFMA blocks per wave
+    constexpr int TM = 16 * WM;        // rows of the C tile
+    constexpr int KS = 4;              // MFMA steps (of 4 k) per chunk
+    const GemmSeg<T> s = g.seg[blockIdx.z];
+    const int m0 = blockIdx.x * TM;
+    const int n0 = blockIdx.y * BN;
+    if (m0 >= s.M) return;
+    const bool tri = g.tri && (blockIdx.z == 0 || g.tri_all);
+    if (tri && m0 + TM - 1 + g.tri_off < n0) return;
+    // looked at before the stores only, so the products do not wait for it
+    const int skip = *(volatile const int*)(g.skip_if ? g.skip_if : &never_skip);
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int li = lane & 15, lq = lane >> 4;
+    const int K = g.K, N = g.N, M = s.M;
+    const int nw = n0 + 32 * wave;     // first column of this wave
+    const bool idle = nw >= N;         // nothing to compute, but the barrier below is shared
+    const T* Bm = s.B ? s.B : g.B;
+
+    // lane offsets within a step of 4 k (rows and columns clamped into the operands: what a
+    // clamped lane computes is not stored)
+    unsigned ao[WM], bo[WN];
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+        ao[i] = (unsigned)((min(m0 + 16 * i + li, M - 1) - m0) + lq * s.lda) * (unsigned)sizeof(T);
+#pragma unroll
+    for (int j = 0; j < WN; ++j) {
+        const int n = min(nw + 16 * j + li, N - 1) - n0;
+        bo[j] = (unsigned)(TB == 1 ? n + lq * g.ldb : n * g.ldb + KS * lq) * (unsigned)sizeof(T);
+    }
+    const T* ap = s.A + m0;
+    const T* bp = TB == 1 ? Bm + n0 : Bm + (long)n0 * g.ldb;
+    const long astep = 4 * s.lda, bstep = TB == 1 ? 4 * g.ldb : 4;
+
+    acc_t acc[WM][WN];
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int j = 0; j < WN; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
+    // the C block's old values, in flight beside the products (addresses clamped like the
+    // operands': in place, they are this tile's own rows and are read before the barrier below)
+    const T alpha = g.alpha, beta = g.beta;
+    T old[WM][WN][4];
+    if (beta != T(0) && !idle) {
+#pragma unroll
+        for (int i = 0; i < WM; ++i)
+#pragma unroll
+            for (int j = 0; j < WN; ++j)
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    old[i][j][t] = s.C[min(m0 + 16 * i + li, M - 1) +
+                                       (long)min(nw + 16 * j + Mfma<T>::row(lane, t), N - 1) * s.ldc];
+    }
+    T a[D][KS][WM], b[D][KS][WN];
+    auto load = [&](T (&av)[KS][WM], T (&bv)[KS][WN], int c) {
+#pragma unroll
+        for (int t = 0; t < KS; ++t) {
+            const char* A = (const char*)(ap + (c * KS + t) * astep);
+#pragma unroll
+            for (int i = 0; i < WM; ++i) av[t][i] = *(const T*)(A + ao[i]);
+            if (TB == 1) {
+                const char* B = (const char*)(bp + (c * KS + t) * bstep);
+#pragma unroll
+                for (int j = 0; j < WN; ++j) bv[t][j] = *(const T*)(B + bo[j]);
+            }
+        }
+        if (TB == 0) {
+            // k runs down a column: lane group lq takes k = 4 lq .. 4 lq + 3 of the chunk in one
+            // piece (a whole 128-byte line per column), exchanged in mma
+#pragma unroll
+            for (int j = 0; j < WN; ++j) {
+                T q[KS];
+                __builtin_memcpy(q, (const char*)(bp + c * KS * 4) + bo[j], sizeof(q));
+#pragma unroll
+                for (int t = 0; t < KS; ++t) bv[t][j] = q[t];
+            }
+        }
+    };
+    auto mma = [&](T (&av)[KS][WM], T (&bv)[KS][WN]) {
+        if (TB == 0)
+#pragma unroll
+            for (int j = 0; j < WN; ++j)
+                lane_rows_transpose(bv[0][j], bv[1][j], bv[2][j], bv[3][j]);
+#pragma unroll
+        for (int t = 0; t < KS; ++t)
+#pragma unroll
+            for (int i = 0; i < WM; ++i)
+#pragma unroll
+                for (int j = 0; j < WN; ++j)
+                    acc[i][j] = Mfma<T>::mac(bv[t][j], av[t][i], acc[i][j]);
+    };
+    const int nc = K / (4 * KS);  // whole chunks
+    if (!idle) {
+        if (nc > 0) {
+            // loads past the last chunk repeat it: unconditional, so the wait counts stay exact
+#pragma unroll
+            for (int d = 0; d < D - 1; ++d) load(a[d], b[d], min(d, nc - 1));
+            int c = 0;
+            for (; c + D <= nc; c += D) {
+#pragma unroll
+                for (int d = 0; d < D; ++d) {
+                    load(a[(d + D - 1) % D], b[(d + D - 1) % D], min(c + d + D - 1, nc - 1));
+                    mma(a[d], b[d]);
+                }
+            }
+#pragma unroll
+            for (int d = 0; d < D - 1; ++d)
+                if (c + d < nc) mma(a[d], b[d]);
+        }
+        for (int k0 = nc * 4 * KS; k0 < K; k0 += 4) {  // remainder: k past K enters as zero
+            const bool ok = k0 + lq < K;
+            const long back = ok ? 0 : k0 + lq - (K - 1);
+            T av[WM], bv[WN];
+#pragma unroll
+            for (int i = 0; i < WM; ++i) {
+                av[i] = *(const T*)((const char*)(ap + (k0 - back) * s.lda) + ao[i]);
+                av[i] = ok ? av[i] : T(0);
+            }
+#pragma unroll
+            for (int j = 0; j < WN; ++j) {
+                bv[j] = *(const T*)((const char*)(bp + (k0 - back) * (TB == 1 ? g.ldb : 1) -
+                                                  (TB == 1 ? 0 : (KS - 1) * lq)) + bo[j]);
+                bv[j] = ok ? bv[j] : T(0);
+            }
+#pragma unroll
+            for (int i = 0; i < WM; ++i)
+#pragma unroll
+                for (int j = 0; j < WN; ++j) acc[i][j] = Mfma<T>::mac(bv[j], av[i], acc[i][j]);
+        }
+    }
+    // in place (C == A): every wave has read the tile's rows before any wave writes them
+    if (s.C == s.A) __syncthreads();
+    if (idle || skip) return;
+#pragma unroll
+    for (int i = 0; i < WM; ++i) {
+        const int row = m0 + 16 * i + li;
+#pragma unroll
+        for (int j = 0; j < WN; ++j)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const int col = nw + 16 * j + Mfma<T>::row(lane, t);
+                if (row >= M || col >= N || (tri && row + g.tri_off < col)) continue;
+                T* c = s.C + row + (long)col * s.ldc;
+                T v = alpha * acc[i][j][t];
+                if (beta != T(0)) v += beta * old[i][j][t];
+                *c = v;
+            }
+    }
+}
+
 // Split-BF16 products.  Each FP32 operand element a is split as hi = bf16(a) and
 // lo = bf16(a - hi) (round to nearest even, v_cvt_pk_bf16_f32), and the product accumulates
 // lo*hi + hi*lo + hi*hi in FP32 on v_mfma_f32_16x16x32_bf16: about 16 significant bits per
@@ -672,6 +871,34 @@ __global__ void symdiag_kernel(const T* __restrict__ B, long ldb, int K, T* __re
     out[(long)blockIdx.y * BN * BN + idx] = r >= c ? B[gr + gc * ldb] : B[gc + gr * ldb];
 }
 
+// Rows per workgroup of the direct kernel for this product, 0 where the slice kernels are the
+// faster ones.  16-row workgroups while they fit the 256 CUs at once (then a wave's own chain of
+// MFMAs is the time, and a 16-row block's is half a 32-row block's), else 32-row workgroups up to
+// the count where the slice kernels' operand reuse through LDS wins: the direct kernel reads every
+// operand from L1/L2, and op(B) = B or FP32's twice as fast MFMA reach that limit sooner.
+// Measured, slice kernel -> direct kernel, us (M x N x K, op(B) = B^T): FP64 152 x 128 x 128
+// 19.5 -> 7.4, 1000 x 512 x 512 63 -> 19, 2400 x 1024 x 1024 147 -> 123, 5000 x 1024 x 1024
+// (1,256 workgroups) 216 -> 199, 10000 x 1024 x 1024 (2,504) 394 -> 389, 10000 x 2048 x 2048 1259
+// -> 1507; op(B) = B 152 x 128 x 128 18.6 -> 9.1, 5000 x 512 x 512 (628) 81 -> 77, 5000 x 1024 x
+// 1024 (1,256) 204 -> 231; FP32 2400 x 128 x 128 15.7 -> 6.3, 20000 x 256 x 256 (1,250) 51 -> 47,
+// 5000 x 512 x 512 (628) 57 -> 52, 10000 x 512 x 512 (1,252) 76 -> 88.
+template <typename T>
+int direct_rows(const GemmArgs<T>& g, int maxM) {
+    double cells = 0;  // C elements of the launch, trapezoids without their upper part
+    for (int i = 0; i < g.nseg; ++i) {
+        const double M = g.seg[i].M, N = g.N;
+        cells += M * N;
+        if (g.tri && (i == 0 || g.tri_all)) {
+            const double w = std::min(N, M + g.tri_off);
+            cells -= M * (N - w) + w * w / 2;
+        }
+    }
+    const double groups = cells / (16 * BN);
+    if (groups <= 256) return 16;
+    const double limit = sizeof(T) == 8 ? (g.transb == 1 ? 1500 : 640) : (g.K <= 256 ? 1500 : 640);
+    return groups / 2 <= limit ? 32 : 0;
+}
+
 template <typename T>
 int launch(const GemmArgs<T>& g, hipStream_t stream) {
     if (g.nseg == 0) return MOAO_OK;
@@ -735,6 +962,18 @@ int launch(const GemmArgs<T>& g, hipStream_t stream) {
     }
     // the K x N slab loads address 128 columns with 32-bit byte offsets
     const bool kn_offsets_fit = (long)BN * g.ldb * (long)sizeof(T) < (1L << 31);
+    if (g.transb < 2 && (g.transb == 1 || kn_offsets_fit)) {
+        if (const int rows = direct_rows(g, maxM)) {
+            grid.x = (maxM + rows - 1) / rows;
+            auto k = g.transb == 1 ? (rows == 16 ? gemm_direct_kernel<T, 1, 1, 4>
+                                                 : gemm_direct_kernel<T, 1, 2, 3>)
+                                   : (rows == 16 ? gemm_direct_kernel<T, 0, 1, 4>
+                                                 : gemm_direct_kernel<T, 0, 2, 3>);
+            hipLaunchKernelGGL(k, grid, dim3(NT), 0, stream, g);
+            MOAO_HIP_TRY(hipGetLastError());
+            return MOAO_OK;
+        }
+    }
     if (small) {
         grid.x = (maxM + 63) / 64;
         if (g.transb == 0 && kn_offsets_fit)

@@ -131,3 +131,48 @@ def test_split_bf16_gemm_matches_numpy(M, N, K, transb, beta):
           f"relative Frobenius {rel:.2e}", flush=True)
     assert rel <= 1e-4
     assert np.array_equal(out[M:], C[M:])
+
+
+@pytest.mark.parametrize("transb", [0, 1])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_few_rows_equal_the_rows_of_a_large_product(transb, dtype):
+    """Launches that leave most of the chip idle run on the direct kernel (16 or 32 rows per
+    workgroup), large ones on the slice kernels; both take every product in the same k order, so
+    a product of the first r rows has the bits of those rows in a product of 52,000: edges of the
+    16- and 32-row blocks, ragged columns, K below, at and past whole 16-k chunks, beta = 0 and 1."""
+    f = dgemm_dev if dtype == np.float64 else sgemm_dev
+    rng = np.random.default_rng(3 + transb)
+    big = 52000
+    for N, K in [(128, 128), (97, 131), (128, 7)]:
+        lda, ldb = big + 3, (N if transb == 1 else K) + 1
+        A = np.asfortranarray(rng.standard_normal((lda, K)).astype(dtype))
+        B = np.asfortranarray(rng.standard_normal((ldb, N if transb == 0 else K)).astype(dtype))
+        C = np.asfortranarray(rng.standard_normal((big, N)).astype(dtype))
+        dA, dB = DeviceArray.from_host(A), DeviceArray.from_host(B)
+        for beta in (0.0, 1.0):
+            dC = DeviceArray.from_host(C)
+            f(transb, big, N, K, -1.25, dA.ptr, lda, dB.ptr, ldb, beta, dC.ptr, big)
+            want = dC.to_host()
+            for r in (1, 15, 16, 17, 33, 300, 4097, 9000):
+                print(f"[gemm-direct] {dtype.__name__} transb={transb} N={N} K={K} rows={r}",
+                      flush=True)
+                dC = DeviceArray.from_host(C)
+                f(transb, r, N, K, -1.25, dA.ptr, lda, dB.ptr, ldb, beta, dC.ptr, big)
+                got = dC.to_host()
+                assert np.array_equal(got[:r], want[:r])
+                assert np.array_equal(got[r:], C[r:])
+
+
+def test_direct_in_place_panel():
+    """C == A with N <= 128 (the panel solve of a leaf): every row is read before it is written."""
+    rng = np.random.default_rng(9)
+    for M, N in [(1, 1), (40, 128), (333, 128), (9001, 77)]:
+        A = np.asfortranarray(rng.standard_normal((M, N)))
+        B = np.asfortranarray(rng.standard_normal((N, N)))
+        dA, dB, dC = DeviceArray.from_host(A), DeviceArray.from_host(B), DeviceArray((M, N))
+        for transb in (0, 1):
+            dgemm_dev(transb, M, N, N, 1.0, dA.ptr, M, dB.ptr, N, 0.0, dC.ptr, M)
+            want = dC.to_host()
+            dX = DeviceArray.from_host(A)
+            dgemm_dev(transb, M, N, N, 1.0, dX.ptr, M, dB.ptr, N, 0.0, dX.ptr, M)
+            assert np.array_equal(dX.to_host(), want), (M, N, transb)
