@@ -8,19 +8,25 @@
 // stored, the rest of the block keeps its input.  The inverse L^{-1} (lower, zero above the diagonal) goes to a
 // separate kLeaf x kLeaf buffer and turns every panel triangular solve into an MFMA GEMM.
 //
-// One workgroup (4 waves) per leaf; the block is zero-padded to kLeaf x kLeaf in LDS and
+// One workgroup (8 waves) per leaf; the block is zero-padded to kLeaf x kLeaf in LDS and
 // processed by 16-column blocks:
-//   load:   batched global loads (16 in flight per lane) before the LDS stores;
-//   factor: [wave 0] 16x16 diagonal block in registers (readlane broadcasts, 1/sqrt of each
-//           pivot by a refined hardware estimate), then D = inv(L_bb) by right-looking
-//           substitution, kept in the unused block above the diagonal; [all] rows below as
-//           A * D^T on f64 MFMA; the rank-16 update of the trailing lower triangle (f64 MFMA)
-//           runs one block late, beside the next diagonal factor: wave 0 updates that
-//           diagonal block first, waves 1-3 the rest;
-//   invert: block columns from last to first: [all] T = inv(L)[below, below] * L[below, j]
-//           and column j of inv(L) = -T * D, both on f64 MFMA, 16-row tiles per wave;
-//   store:  L and inv(L) with 16 LDS reads per lane in flight before the global stores.
+//   load:   every element of the lower triangle in flight before the LDS stores;
+//   factor: [wave 0] 16x16 diagonal block and its inverse together, in registers: unnormalised
+//           elimination of [A | I] (pivots' reciprocals only; one 1/sqrt per lane at the end
+//           scales L and D), columns passed between the lanes of a 16-lane row by DPP broadcasts;
+//           [all] rows below as A * D^T on f64 MFMA; the rank-16 update of the trailing lower
+//           triangle (f64 MFMA) runs one block late, beside the next diagonal factor: wave 0
+//           updates that diagonal block first, the other waves the rest;
+//   invert: by doubling: from the inverses of the 16x16 diagonal blocks to 32, 64 and 128:
+//           inv(L)21 = -inv(L)22 (L21 inv(L)11), both products on f64 MFMA over all waves, the
+//           inner one parked in the unused block above the diagonal;
+//   store:  L before the inversion overwrites it, inv(L) at the end.
+// The time is the serial chain of one workgroup, 128 pivots long.  What it was spent on before
+// (70 us): readlane broadcasts under a branch per column, 97 of 166 thousand cycles; an inversion
+// by block columns, 45 thousand.
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "common.hpp"
 #include "leaf.hpp"
@@ -29,29 +35,80 @@
 namespace moao {
 namespace {
 
-constexpr int NTL = 256;       // lanes per leaf workgroup
+constexpr int NTL = 512;       // lanes per leaf workgroup
+constexpr int NWL = NTL / 64;
 constexpr int LD = kLeaf + 1;  // odd stride: a row across columns hits distinct banks
 constexpr int kB = 16;         // inner block
+constexpr int kNB = kLeaf / kB;
 
 #define S_(r, c) S[(c) * LD + (r)]
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
-// Value of v in lane l (l wave-uniform).
-__device__ __forceinline__ double lane_value(double v, int l) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane((int)b, l);
-    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+// f(0), f(1), ..., f(N - 1) with the index as a compile-time constant
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+    if constexpr (N > 0) {
+        static_for<N - 1>(f);
+        f(std::integral_constant<int, N - 1>{});
+    }
 }
 
-// 1/sqrt(d) for d > 0: hardware estimate refined by two Newton steps (no division, no
-// correctly-rounded sqrt sequence on the pivot's critical path).
+// Value of v in lane L of the caller's 16-lane row.
+template <int L>
+__device__ __forceinline__ double row_value(double v) {
+    const long long b = __double_as_longlong(v);
+    return __longlong_as_double(__builtin_amdgcn_update_dpp(b, b, 0x150 + L, 0xf, 0xf, true));
+}
+
+// 1/sqrt(d) for d > 0: hardware estimate refined by two Newton steps.
 __device__ __forceinline__ double rsqrt_nr(double d) {
     double r = __builtin_amdgcn_rsq(d);
     r = r * (1.5 - 0.5 * d * r * r);
     r = r * (1.5 - 0.5 * d * r * r);
     return r;
+}
+
+// 1/d: hardware estimate refined by two Newton steps (no division on the pivots' chain).
+__device__ __forceinline__ double rcp_nr(double d) {
+    double r = __builtin_amdgcn_rcp(d);
+    r = fma(fma(-d, r, 1.0), r, r);
+    return fma(fma(-d, r, 1.0), r, r);
+}
+
+// A 16 x 16 block A = L L^T and D = inv(L) in one wave: lane i of every 16-lane row holds row i
+// (the four rows work alike).  Elimination of [A | I] with multipliers m_j = a_j / d_j: a[j] keeps
+// m_j d_j, x becomes the inverse of the unit factor; then L_ij = a[j] / sqrt(d_j) and
+// D_ij = x[j] / sqrt(d_i).  Returns the number of positive pivots before the first that is not.
+__device__ __forceinline__ int diag_factor(double (&a)[kB], double (&x)[kB], int li) {
+    double dv = 1.0;  // this lane's own pivot
+    int good = 0;
+    bool all = true;
+    static_for<kB>([&](auto J) {
+        constexpr int j = decltype(J)::value;
+        const double d = row_value<j>(a[j]);
+        all = all && d > 0.0;
+        good += all ? 1 : 0;
+        const double m = li > j ? a[j] * rcp_nr(d) : 0.0;
+        dv = li == j ? a[j] : dv;
+        // the next pivot's column first
+        static_for<kB - 1 - j>([&](auto Q) {
+            constexpr int k = j + 1 + decltype(Q)::value;
+            a[k] = fma(-m, row_value<k>(a[j]), a[k]);
+        });
+        static_for<j>([&](auto C) {
+            constexpr int c = decltype(C)::value;
+            x[c] = fma(-m, row_value<j>(x[c]), x[c]);
+        });
+        x[j] = li == j ? 1.0 : -m;
+    });
+    const double rs = rsqrt_nr(dv);
+    static_for<kB>([&](auto J) {
+        constexpr int j = decltype(J)::value;
+        a[j] *= row_value<j>(rs);
+        x[j] = li >= j ? x[j] * rs : 0.0;
+    });
+    return good;
 }
 
 // 16 x 16 block product on MFMA: acc += X[r0:r0+16, k0:k0+16*nc] * Y[k0:k0+16*nc, c0:c0+16]
@@ -95,52 +152,49 @@ template <typename TS>
 __global__ void __launch_bounds__(NTL) leaf_potrf_inv(TS* A, long lda, int nb, TS* inv,
                                                       int* info, int j0) {
     __shared__ double S[kLeaf * LD];
-    __shared__ double T[(kLeaf - kB) * kB];  // inverse: product of the trailing part
-    __shared__ double D[kB * kB];            // inverse of one diagonal block
-    __shared__ double rdiag[kLeaf];          // 1 / L_jj
+    __shared__ double D[kNB][kB * kB];  // inverses of the diagonal blocks, element (r, c) at r*kB+c
     __shared__ int fail;
-    if (*(volatile int*)info != 0) return;  // an earlier leaf failed: R is not computed
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: scalar branches
-    if (tid == 0) fail = 0;
-    // Load the lower triangle, zero-padded to kLeaf x kLeaf.  A wave owns columns
-    // wave, wave+4, ...; each batch issues 16 independent loads per lane before any LDS store
-    // (addresses clamped into the block, values outside the lower triangle replaced by 0).
+    const int li = lane & 15, lq = lane >> 4;
+    // Load the lower triangle, zero-padded to kLeaf x kLeaf: wave w takes columns w, w + 8, ...,
+    // every load issued before any LDS store (rows and columns clamped into the block, the
+    // rows above a column's 64-row half not read, values outside the triangle replaced by 0).
     {
-        constexpr int CB = 8;
+        constexpr int CW = kLeaf / NWL;
         const int rA = min(lane, nb - 1), rB = min(lane + 64, nb - 1);
-        for (int cb = wave; cb < kLeaf; cb += 4 * CB) {
-            double v0[CB], v1[CB];
+        double v0[CW / 2], v1[CW];
 #pragma unroll
-            for (int q = 0; q < CB; ++q) {
-                const long cc = min(cb + 4 * q, nb - 1);
-                v0[q] = (double)A[rA + cc * lda];
-                v1[q] = (double)A[rB + cc * lda];
-            }
+        for (int q = 0; q < CW; ++q) {
+            const long cc = min(wave + NWL * q, nb - 1);
+            if (q < CW / 2) v0[q] = (double)A[rA + cc * lda];
+            v1[q] = (double)A[rB + cc * lda];
+        }
+        if (*(volatile int*)info != 0) return;  // an earlier leaf failed: R is not computed
 #pragma unroll
-            for (int q = 0; q < CB; ++q) {
-                const int c = cb + 4 * q;
-                S_(lane, c) = (c < nb && lane < nb && lane >= c) ? v0[q] : 0.0;
-                S_(lane + 64, c) = (c < nb && lane + 64 < nb && lane + 64 >= c) ? v1[q] : 0.0;
-            }
+        for (int q = 0; q < CW; ++q) {
+            const int c = wave + NWL * q;
+            if (q < CW / 2) S_(lane, c) = (c < nb && lane < nb && lane >= c) ? v0[q] : 0.0;
+            S_(lane + 64, c) = (c < nb && lane + 64 < nb && lane + 64 >= c) ? v1[q] : 0.0;
         }
     }
+    if (tid == 0) fail = 0;
     __syncthreads();
 
     // Columns [0, ncol) of L back to global (lower part only), 16 LDS reads per lane in flight
     // before the stores.
     auto store_L = [&](int ncol) {
-        for (int cb = wave; cb < ncol; cb += 4 * 8) {
+        for (int cb = wave; cb < ncol; cb += 8 * NWL) {
             double v0[8], v1[8];
 #pragma unroll
             for (int q = 0; q < 8; ++q) {
-                const int c = min(cb + 4 * q, kLeaf - 1);
+                const int c = min(cb + NWL * q, kLeaf - 1);
                 v0[q] = S_(lane, c);
                 v1[q] = S_(lane + 64, c);
             }
 #pragma unroll
             for (int q = 0; q < 8; ++q) {
-                const int c = cb + 4 * q;
+                const int c = cb + NWL * q;
                 if (c >= ncol) break;
                 if (lane >= c && lane < nb) A[lane + (long)c * lda] = (TS)v0[q];
                 if (lane + 64 >= c && lane + 64 < nb) A[lane + 64 + (long)c * lda] = (TS)v1[q];
@@ -162,77 +216,43 @@ __global__ void __launch_bounds__(NTL) leaf_potrf_inv(TS* A, long lda, int nb, T
                             1, acc, lane);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const int r = base + 16 * ti + (lane >> 4) + 4 * e;
-            const int c = base + 16 * tj + (lane & 15);
+            const int r = base + 16 * ti + lq + 4 * e;
+            const int c = base + 16 * tj + li;
             if (r < nb && c < nb && r >= c) S_(r, c) -= acc[e];
         }
     };
     for (int kb = 0; kb < nb; kb += kB) {
         const int bs = min(kB, nb - kb);
+        double* Db = D[kb / kB];
         // Look-ahead: the previous block's trailing update runs here, beside this block's
         // diagonal factor.  Wave 0 takes tile 0 (this block's diagonal block) and then factors
-        // it; waves 1-3 take the other tiles, which this factor neither reads nor writes.
+        // it; the other waves take the other tiles, which this factor neither reads nor writes.
         if (kb > 0) {
             const int ht = (nb - kb + 15) / 16, ntile = ht * (ht + 1) / 2;
             if (wave == 0) trail_tile(kb - kB, 0);
             else
-                for (int t = wave; t < ntile; t += NTL / 64 - 1) trail_tile(kb - kB, t);
+                for (int t = wave; t < ntile; t += NWL - 1) trail_tile(kb - kB, t);
         }
         if (wave == 0) {
-            // Diagonal block: lane i holds row i in registers; column j is broadcast with
-            // readlane (uniform lane index), so the block needs no LDS round trips.
-            const int i = lane;
-            double a[kB];
+            // rows and columns past nb enter as the identity
+            double a[kB], x[kB];
 #pragma unroll
-            for (int k = 0; k < kB; ++k) a[k] = (i < bs && k <= i) ? S_(kb + i, kb + k) : 0.0;
-            bool bad = false;
-#pragma unroll
-            for (int j = 0; j < kB; ++j) {
-                if (j < bs && !bad) {
-                    const double d = lane_value(a[j], j);
-                    if (!(d > 0.0)) {  // same value in every lane
-                        bad = true;
-                        if (lane == 0) {
-                            fail = 1;
-                            atomicCAS(info, 0, j0 + kb + j + 1);
-                        }
-                    } else {
-                        const double rsd = rsqrt_nr(d), sd = d * rsd;
-                        a[j] = (i == j) ? sd : a[j] * rsd;
-                        if (lane == 0) rdiag[kb + j] = rsd;
-#pragma unroll
-                        for (int k = j + 1; k < kB; ++k) {
-                            const double lkj = lane_value(a[j], k);
-                            if (i >= k) a[k] -= a[j] * lkj;
-                        }
-                    }
-                }
+            for (int k = 0; k < kB; ++k) {
+                const double v = S_(kb + li, kb + k);
+                a[k] = li < bs && k < bs ? v : (li == k ? 1.0 : 0.0);
+                x[k] = 0.0;
             }
-            if (i < bs)
-#pragma unroll
-                for (int k = 0; k < kB; ++k)
-                    if (k <= i) S_(kb + i, kb + k) = a[k];
-            // D = inv(L_bb) (same wave, so the LDS writes above are visible): lane c builds
-            // column c right-looking from e_c; rows at or past bs are zero padding.  D is kept
-            // in the unused block above the diagonal, S_(kb + r, kb + kB + c), or in D[] for
-            // the last block; the rows below and the inverse phase both use it.
-            if (lane < kB) {
-                const int c = lane;
-                double x[kB];
-#pragma unroll
-                for (int r = 0; r < kB; ++r) x[r] = (r == c) ? 1.0 : 0.0;
-#pragma unroll
-                for (int r = 0; r < kB; ++r) {
-                    x[r] = r < bs ? x[r] * rdiag[kb + r] : 0.0;
-#pragma unroll
-                    for (int r2 = r + 1; r2 < kB; ++r2) x[r2] -= S_(kb + r2, kb + r) * x[r];
+            const int good = diag_factor(a, x, li);
+            if (good < kB) {
+                if (lane == 0) {
+                    fail = 1;
+                    atomicCAS(info, 0, j0 + kb + good + 1);
                 }
-                if (kb + kB < kLeaf) {
+            } else if (lq == 0) {
 #pragma unroll
-                    for (int r = 0; r < kB; ++r) S_(kb + r, kb + kB + c) = x[r];
-                } else {
-#pragma unroll
-                    for (int r = 0; r < kB; ++r) D[r * kB + c] = x[r];
+                for (int k = 0; k < kB; ++k) {
+                    if (li < bs && k <= li) S_(kb + li, kb + k) = a[k];
+                    Db[li * kB + k] = li < bs ? x[k] : 0.0;
                 }
             }
         }
@@ -244,81 +264,79 @@ __global__ void __launch_bounds__(NTL) leaf_potrf_inv(TS* A, long lda, int nb, T
             return;
         }
         // rows below the diagonal block: L[r, kb:kb+16] = A[r, kb:kb+16] * D^T on MFMA, a
-        // 16-row tile per wave turn, in place (bs is 16 whenever rows remain below the block)
-        const int rest = nb - kb - bs;
-        if (rest > 0) {
-            const bool up = kb + kB < kLeaf;
-            const double* Dp = up ? &S_(kb, kb + kB) : D;  // D element (r, c) at Dp[r*dr + c*dc]
-            const int dr = up ? 1 : kB, dc = up ? LD : 1;
-            const int ht = (rest + 15) / 16;
-            for (int i = wave; i < ht; i += NTL / 64) {
-                const int r0 = kb + kB + 16 * i;
-                f64x4 acc = {0, 0, 0, 0};
-                // Y element (k, c) = D^T(k, c) = D(c, k)
-                acc = mfma_block<1>(&S_(0, kb), LD, r0, Dp, dc, dr, 0, 0, 1, acc, lane);
+        // 16-row tile per wave, in place (bs is 16 whenever rows remain below the block)
+        const int ht = (nb - kb - bs + 15) / 16;
+        for (int i = wave; i < ht; i += NWL) {
+            const int r0 = kb + kB + 16 * i;
+            f64x4 acc = {0, 0, 0, 0};
+            // Y element (k, c) = D^T(k, c) = D(c, k)
+            acc = mfma_block<1>(&S_(0, kb), LD, r0, Db, 1, kB, 0, 0, 1, acc, lane);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int r = r0 + (lane >> 4) + 4 * e;
-                    if (r < nb) S_(r, kb + (lane & 15)) = acc[e];
-                }
+            for (int e = 0; e < 4; ++e) {
+                const int r = r0 + lq + 4 * e;
+                if (r < nb) S_(r, kb + li) = acc[e];
             }
         }
         __syncthreads();
     }
     store_L(nb);
+    __syncthreads();
 
     // ------------------------------------------------------------------ inverse
-    const int nblocks = (nb + kB - 1) / kB;
-    for (int jb = nblocks - 1; jb >= 0; --jb) {
-        const int c0 = jb * kB, bs = min(kB, nb - c0);
-        const int below = nb - c0 - bs;
-        const int kbeg = c0 + bs;
-        // D = inv(L_jj), computed during the factorization: copy it out of its storage above
-        // the diagonal (the last block left it in D[] already); used after the next barrier
-        if (c0 + kB < kLeaf)
-            for (int t = tid; t < kB * kB; t += NTL) D[t] = S_(c0 + t / kB, c0 + kB + t % kB);
-        // T = inv(L)[below, below] * L[below, c0:c0+16] on MFMA, a 16-row tile per wave turn;
-        // inv(L) of the trailing part is lower triangular (zero above, zero padding below nb),
-        // so row tile i needs k < 16 (i + 1) only.  Tiles go to the waves in snake order
-        // (0 1 2 3, then 7 6 5 4), which evens out the longer products of the later tiles.
-        const int nti = (below + 15) / 16;
-        for (int r = 0; 4 * r < nti; ++r) {
-            const int i = (r & 1) ? 4 * r + 3 - wave : 4 * r + wave;
-            if (i >= nti) continue;
-            f64x4 acc = {0, 0, 0, 0};
-            acc = mfma_block<kLeaf / kB - 1>(&S_(0, kbeg), LD, 16 * i + kbeg, &S_(kbeg, c0), 1,
-                                             LD, 0, 0, i + 1, acc, lane);
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                T[(lane & 15) * (kLeaf - kB) + 16 * i + (lane >> 4) + 4 * e] = acc[e];
-        }
-        __syncthreads();
-        // column block jb of inv(L): rows below = -T * D; diagonal block = D
-        for (int i = wave; i < nti; i += NTL / 64) {
-            f64x4 acc = {0, 0, 0, 0};
-            acc = mfma_block<1>(T, kLeaf - kB, 16 * i, D, kB, 1, 0, 0, 1, acc, lane);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int rr = 16 * i + (lane >> 4) + 4 * e;
-                if (rr < below) S_(kbeg + rr, c0 + (lane & 15)) = -acc[e];
-            }
-        }
-        {
-            const int tc = tid & (kB - 1), tr = tid / kB;
-            if (tc < bs && tr < bs) S_(c0 + tr, c0 + tc) = tr >= tc ? D[tr * kB + tc] : 0.0;
-        }
-        __syncthreads();
+    // The diagonal blocks' inverses in their place (zero past nb: rows and columns of zeros, as
+    // the padding of S), then doubling.  Level h joins pairs of h x h inverses: T = L21 inv11
+    // into the block above the diagonal, then inv21 = -inv22 T.  inv11 and inv22 are lower
+    // triangular: 16-wide chunks outside them are skipped.
+    for (int t = tid; t < kNB * kB * kB; t += NTL) {
+        const int b = t / (kB * kB), r = t / kB % kB, c = t % kB;
+        if (b * kB < nb) S_(b * kB + r, b * kB + c) = D[b][r * kB + c];
     }
-    for (int cb = wave; cb < kLeaf; cb += 4 * 8) {
+    __syncthreads();
+    auto level = [&](auto H) {
+        constexpr int h = decltype(H)::value, nt = h / 16, tiles = kLeaf / 2 / h * nt * nt;
+        // tile (i, j) of pair q; the column index of one half of the waves' tiles runs backwards,
+        // which evens out the triangles' shorter and longer products
+        auto tile = [&](int t, int& q, int& i, int& j) {
+            q = t / (nt * nt);
+            i = t / nt % nt;
+            j = (t / NWL) & 1 ? nt - 1 - t % nt : t % nt;
+        };
+        for (int t = wave; t < tiles; t += NWL) {
+            int q, i, j;
+            tile(t, q, i, j);
+            const int o = 2 * h * q;
+            f64x4 acc = {0, 0, 0, 0};
+            acc = mfma_block<nt>(&S_(0, o), LD, o + h + 16 * i, &S_(o, o), 1, LD, 16 * j, 16 * j,
+                                 nt - j, acc, lane);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) S_(o + 16 * i + lq + 4 * e, o + h + 16 * j + li) = acc[e];
+        }
+        __syncthreads();
+        for (int t = wave; t < tiles; t += NWL) {
+            int q, j, i;
+            tile(t, q, j, i);
+            const int o = 2 * h * q;
+            f64x4 acc = {0, 0, 0, 0};
+            acc = mfma_block<nt>(&S_(0, o + h), LD, o + h + 16 * i, &S_(o, o + h), 1, LD, 16 * j,
+                                 0, i + 1, acc, lane);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) S_(o + h + 16 * i + lq + 4 * e, o + 16 * j + li) = -acc[e];
+        }
+        __syncthreads();
+    };
+    if (nb > 16) level(std::integral_constant<int, 16>{});
+    if (nb > 32) level(std::integral_constant<int, 32>{});
+    if (nb > 64) level(std::integral_constant<int, 64>{});
+    for (int cb = wave; cb < kLeaf; cb += 8 * NWL) {
         double v0[8], v1[8];
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
-            v0[q] = S_(lane, cb + 4 * q);
-            v1[q] = S_(lane + 64, cb + 4 * q);
+            v0[q] = S_(lane, cb + NWL * q);
+            v1[q] = S_(lane + 64, cb + NWL * q);
         }
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
-            const int c = cb + 4 * q;
+            const int c = cb + NWL * q;
             inv[lane + (long)c * kLeaf] = (TS)((lane < nb && c < nb && lane >= c) ? v0[q] : 0.0);
             inv[lane + 64 + (long)c * kLeaf] =
                 (TS)((lane + 64 < nb && c < nb && lane + 64 >= c) ? v1[q] : 0.0);
