@@ -293,3 +293,34 @@ def test_solve_graph_replays_match_eager():
             assert reconstructor_dev(n, m, e1.ptr, n, e2.ptr, m, 1) == 0
     finally:
         lib().moao_hip_solve_graph_destroy(g)
+
+
+@pytest.mark.parametrize("n", [2, 4, 5, 15, 16, 17, 31, 33, 48, 63, 64, 65, 80, 97, 113, 126])
+def test_leaf_edges(n):
+    """One leaf at the edges of its 16-column blocks, of their four-column groups and of the
+    doubling levels of its inverse: factor and R, the upper part kept, and the order of a
+    non-positive or NaN pivot wherever it falls."""
+    from moao_amd.reconstructor import sreconstructor
+    print(f"[recon] leaf n={n}", flush=True)
+    rng = np.random.default_rng(100 + n)
+    G = rng.standard_normal((n, n))
+    S = G @ G.T / n + np.eye(n)
+    C = np.asfortranarray(np.tril(S) + np.triu(np.full((n, n), 3.5), 1))
+    B = np.asfortranarray(rng.standard_normal((37, n)))
+    Cg, Bg = C.copy(order="F"), B.copy(order="F")
+    assert reconstructor(n, 37, Cg, n, Bg, 37, 1) == 0
+    assert rel_fro(np.tril(Cg), np.linalg.cholesky(S)) <= 1e-13
+    assert np.linalg.norm(B - Bg @ S) / np.linalg.norm(B) <= 5e-13
+    assert np.array_equal(Cg[np.triu_indices(n, 1)], C[np.triu_indices(n, 1)])
+    C32, B32 = C.astype(np.float32, order="F"), B.astype(np.float32, order="F")
+    assert sreconstructor(n, 37, C32, n, B32, 37, 1) == 0
+    assert np.linalg.norm(B - B32.astype(np.float64) @ S) / np.linalg.norm(B) <= 1e-5
+    for p in sorted({0, 1, 3, 4, n // 2, n - 2, n - 1}):
+        if p >= n:
+            continue
+        for bad in (-1.0, np.nan):
+            Cb = C.copy(order="F")
+            Cb[p, p] = bad
+            Bb = B.copy(order="F")
+            assert reconstructor(n, 37, Cb, n, Bb, 37, 1) == p + 1, (n, p, bad)
+            assert np.array_equal(Bb, B)
