@@ -50,21 +50,32 @@ constexpr double kA2 = -0.08641975308641974829;
 constexpr double kA3 = 0.08001828989483310284;
 
 // Series coefficients of the reference (common/moao_defs.h:18-27): Gamma-function values.
-__constant__ double cGa[11] = {0, 12.067619015983075, 5.17183672113560444,
-                               0.795667187867016068, 0.0628158306210802181,
-                               0.00301515986981185091, 9.72632216068338833e-05,
-                               2.25320204494595251e-06, 3.93000356676612095e-08,
-                               5.34694362825451923e-10, 5.83302941264329804e-12};
-__constant__ double cGma[11] = {-3.74878707653729304, -2.04479295083852408,
-                                -0.360845814853857083, -0.0313778969438136685,
-                                -0.001622994669507603, -5.56455315259749673e-05,
-                                -1.35720808599938951e-06, -2.47515152461894642e-08,
-                                -3.50257291219662472e-10, -3.95770950530691961e-12,
-                                -3.65327031259100284e-14};
+#define MOAO_VK_GA                                                                          \
+    {0, 12.067619015983075, 5.17183672113560444, 0.795667187867016068, 0.0628158306210802181,  \
+     0.00301515986981185091, 9.72632216068338833e-05, 2.25320204494595251e-06,               \
+     3.93000356676612095e-08, 5.34694362825451923e-10, 5.83302941264329804e-12}
+#define MOAO_VK_GMA                                                                         \
+    {-3.74878707653729304, -2.04479295083852408, -0.360845814853857083, -0.0313778969438136685, \
+     -0.001622994669507603, -5.56455315259749673e-05, -1.35720808599938951e-06,              \
+     -2.47515152461894642e-08, -3.50257291219662472e-10, -3.95770950530691961e-12,           \
+     -3.65327031259100284e-14}
+__constant__ double cGa[11] = MOAO_VK_GA;
+__constant__ double cGma[11] = MOAO_VK_GMA;
+
+// Table of the normalised structure function f(t), t = q^2, q = 2 pi r / L0 (the function the two
+// branches below define): kSub intervals per octave of t from 2^kLo up to 2^kHi, a polynomial of
+// degree 7 each, then one constant (f is kK2 to the last bit past q = 45).  The interval that holds
+// the branches' border q = 3 pi / 2 is there twice, with the series and with the asymptote.
+constexpr int kSub = 32, kSubBits = 5, kLo = -16, kHi = 11;
+constexpr int kCoef = 8;
+constexpr int kTabN = (kHi - kLo) * kSub + 2;
+constexpr double kTBorder = kXlim * kXlim;
+// Arguments below the table and those within rounding of the border take the direct formulas.
+constexpr double kTMin = 1.0 / (1 << -kLo), kTBand = 1e-9;
 
 constexpr int kRows = 64;       // rows per workgroup (one wave tall)
 constexpr int kColsPerWave = 4; // columns per wave
-constexpr int kWaves = 4;       // waves per workgroup
+constexpr int kWaves = 8;       // waves per workgroup
 constexpr int kCols = kColsPerWave * kWaves;
 
 struct MatcovArgs {
@@ -80,6 +91,7 @@ struct MatcovArgs {
     const double* sspL;     // [Nw*Nlayer]
     const double* lk;       // [Nlayer] 2*pi/L0
     const double* amp;      // [Nlayer] k1*L0^(5/3)
+    const double* ftab;     // [kTabN * kCoef] table of f
     const double* cn2;      // [Nlayer]
     const double* sspsz;    // [Nw] diam/Nssp
     const double* nNGS;     // [Nw-nlgs]
@@ -130,32 +142,65 @@ __device__ __forceinline__ double vk_dphi(double x, double y, double lk, double 
     return res;
 }
 
-__device__ __forceinline__ double slope_cov(int kind, double du, double dv, double s1, double s2,
-                                            double lk, double amp) {
+// The same function from the table (in LDS): t's exponent and top mantissa bits give the interval,
+// its other bits the place in it (exact).  About 20 VALU instructions and four 16-byte LDS reads
+// where sqrt, cube root, both branches and exp take about 230.
+__device__ __forceinline__ double vk_table(const double* tab, double x, double y, double lk,
+                                           double amp) {
+    const double r2 = fma(x, x, y * y);
+    const double t = r2 * (lk * lk);
+    if (__builtin_expect(!(t >= kTMin) || fabs(t - kTBorder) < kTBand, 0))
+        return vk_dphi(x, y, lk, amp);
+    const unsigned hi = (unsigned)__double2hiint(t);
+    int k = (int)(hi >> (20 - kSubBits)) - ((1023 + kLo) << kSubBits);
+    k = min(k + (t > kTBorder ? 1 : 0), kTabN - 1);
+    const double w = __hiloint2double((int)((hi & ((1u << (20 - kSubBits)) - 1)) | 0x3ff00000u),
+                                      __double2loint(t));
+    const double z = w - (1.0 + 0.5 / kSub);
+    // coefficients 2n, 2n + 1 of interval k at double2 n * kTabN + k: lanes in different intervals
+    // read neighbouring 16-byte pieces, not one bank group 64 bytes apart
+    const double2* c = (const double2*)tab + k;
+    double f = 0.0;
+#pragma unroll
+    for (int n = kCoef / 2 - 1; n >= 0; --n) {
+        const double2 p = c[n * kTabN];
+        f = n == kCoef / 2 - 1 ? p.y : fma(f, z, p.y);
+        f = fma(f, z, p.x);
+    }
+    return f * amp;
+}
+
+__device__ __forceinline__ void load_table(const double* src, double* tab) {
+    for (int e = threadIdx.x; e < kTabN * kCoef / 2; e += kWaves * 64)
+        ((double2*)tab)[e] = ((const double2*)src)[e];
+    __syncthreads();
+}
+
+__device__ __forceinline__ double slope_cov(const double* tab, int kind, double du, double dv,
+                                            double s1, double s2, double lk, double amp) {
+    auto D = [&](double x, double y) { return vk_table(tab, x, y, lk, amp); };
     const double ac = s1 - s2, ad = s1 + s2, bc = -ad, bd = -ac;
     // Equal sizes (s1 == s2, most WFS pairs): ac = +0 and bd = -0, so the first and last
     // terms share one argument exactly; evaluating it once keeps every operation and its order.
     switch (kind) {
         case 0:
             if (ac == 0.0) {
-                const double d0 = vk_dphi(du, dv, lk, amp);
-                return -d0 + vk_dphi(du + ad, dv, lk, amp) + vk_dphi(du + bc, dv, lk, amp) - d0;
+                const double d0 = D(du, dv);
+                return -d0 + D(du + ad, dv) + D(du + bc, dv) - d0;
             }
-            return -vk_dphi(du + ac, dv, lk, amp) + vk_dphi(du + ad, dv, lk, amp) +
-                   vk_dphi(du + bc, dv, lk, amp) - vk_dphi(du + bd, dv, lk, amp);
+            return -D(du + ac, dv) + D(du + ad, dv) + D(du + bc, dv) - D(du + bd, dv);
         case 3:
             if (ac == 0.0) {
-                const double d0 = vk_dphi(du, dv, lk, amp);
-                return -d0 + vk_dphi(du, dv + ad, lk, amp) + vk_dphi(du, dv + bc, lk, amp) - d0;
+                const double d0 = D(du, dv);
+                return -d0 + D(du, dv + ad) + D(du, dv + bc) - d0;
             }
-            return -vk_dphi(du, dv + ac, lk, amp) + vk_dphi(du, dv + ad, lk, amp) +
-                   vk_dphi(du, dv + bc, lk, amp) - vk_dphi(du, dv + bd, lk, amp);
+            return -D(du, dv + ac) + D(du, dv + ad) + D(du, dv + bc) - D(du, dv + bd);
         case 1:
-            return -vk_dphi(du + s1, dv - s2, lk, amp) + vk_dphi(du + s1, dv + s2, lk, amp) +
-                   vk_dphi(du - s1, dv - s2, lk, amp) - vk_dphi(du - s1, dv + s2, lk, amp);
+            return -D(du + s1, dv - s2) + D(du + s1, dv + s2) + D(du - s1, dv - s2) -
+                   D(du - s1, dv + s2);
         default:
-            return -vk_dphi(du - s2, dv + s1, lk, amp) + vk_dphi(du + s2, dv + s1, lk, amp) +
-                   vk_dphi(du - s2, dv - s1, lk, amp) - vk_dphi(du + s2, dv - s1, lk, amp);
+            return -D(du - s2, dv + s1) + D(du + s2, dv + s1) + D(du - s2, dv - s1) -
+                   D(du + s2, dv - s1);
     }
 }
 
@@ -169,6 +214,8 @@ __global__ void __launch_bounds__(kWaves * 64) meas_kernel(MatcovArgs a) {
         const int last_row = a.xoffset + min(a.nrows - 1, (int)blockIdx.x * kRows + kRows - 1);
         if (last_row < a.yoffset + (int)blockIdx.y * kCols) return;
     }
+    __shared__ __attribute__((aligned(16))) double tab[kTabN * kCoef];
+    load_table(a.ftab, tab);
     if (lx >= a.nrows) return;
     const int ri = a.rowtab[lx];
     const int m = (ri >> 1) & 0xff, xi = ri & 1, p1 = ri >> 9;
@@ -189,7 +236,7 @@ __global__ void __launch_bounds__(kWaves * 64) meas_kernel(MatcovArgs a) {
                 const long o = (long)l * a.Nx;
                 const double du = a.u[o + p1] - a.u[o + p2];
                 const double dv = a.v[o + p1] - a.v[o + p2];
-                covar += 0.5 * slope_cov(kind, du, dv, sml * 0.5, snl * 0.5, a.lk[l], a.amp[l]) *
+                covar += 0.5 * slope_cov(tab, kind, du, dv, sml * 0.5, snl * 0.5, a.lk[l], a.amp[l]) *
                          kk * a.cn2[l];
             }
         }
@@ -222,6 +269,13 @@ __global__ void __launch_bounds__(kWaves * 64) pair_kernel(MatcovArgs a) {
     const int wave = threadIdx.x >> 6;
     const int rs = blockIdx.x * kRows + lane;
     const int cs0 = blockIdx.y * kCols + wave * kColsPerWave;
+    if (a.type_mat == 1) {
+        // no pair of this workgroup has a row (its y slope's, the largest) at or below a column
+        const int2 last = a.rsub[min((int)blockIdx.x * kRows + kRows, a.nrsub) - 1];
+        if (last.y + a.nsub[(last.x >> 1) & 0xff] < a.csub[blockIdx.y * kCols].y) return;
+    }
+    __shared__ __attribute__((aligned(16))) double tab[kTabN * kCoef];
+    load_table(a.ftab, tab);
     if (rs >= a.nrsub) return;
     const int2 re = a.rsub[rs];
     const int m = (re.x >> 1) & 0xff, p1 = re.x >> 9;
@@ -251,38 +305,39 @@ __global__ void __launch_bounds__(kWaves * 64) pair_kernel(MatcovArgs a) {
                 const double s1 = sml * 0.5, s2 = snl * 0.5;
                 const double lk = a.lk[l], amp = a.amp[l];
                 const double ac = s1 - s2, ad = s1 + s2, bc = -ad, bd = -ac;
+                auto D = [&](double x, double y) { return vk_table(tab, x, y, lk, amp); };
                 double sxx, syy, sxy, syx;
                 sxx = syy = sxy = 0.0;
                 if (ac == 0.0) {
                     if (nxx || nyy) {
-                        const double d0 = vk_dphi(du, dv, lk, amp);
+                        const double d0 = D(du, dv);
                         if (nxx)
-                            sxx = -d0 + vk_dphi(du + ad, dv, lk, amp) +
-                                  vk_dphi(du + bc, dv, lk, amp) - d0;
+                            sxx = -d0 + D(du + ad, dv) +
+                                  D(du + bc, dv) - d0;
                         if (nyy)
-                            syy = -d0 + vk_dphi(du, dv + ad, lk, amp) +
-                                  vk_dphi(du, dv + bc, lk, amp) - d0;
+                            syy = -d0 + D(du, dv + ad) +
+                                  D(du, dv + bc) - d0;
                     }
                     // s1 == s2: the corners of xy and yx are the same four arguments
-                    const double q1 = vk_dphi(du + s1, dv - s2, lk, amp);
-                    const double q2 = vk_dphi(du + s1, dv + s2, lk, amp);
-                    const double q3 = vk_dphi(du - s1, dv - s2, lk, amp);
-                    const double q4 = vk_dphi(du - s1, dv + s2, lk, amp);
+                    const double q1 = D(du + s1, dv - s2);
+                    const double q2 = D(du + s1, dv + s2);
+                    const double q3 = D(du - s1, dv - s2);
+                    const double q4 = D(du - s1, dv + s2);
                     if (nxy) sxy = -q1 + q2 + q3 - q4;
                     syx = -q4 + q2 + q3 - q1;
                 } else {
                     if (nxx)
-                        sxx = -vk_dphi(du + ac, dv, lk, amp) + vk_dphi(du + ad, dv, lk, amp) +
-                              vk_dphi(du + bc, dv, lk, amp) - vk_dphi(du + bd, dv, lk, amp);
+                        sxx = -D(du + ac, dv) + D(du + ad, dv) +
+                              D(du + bc, dv) - D(du + bd, dv);
                     if (nyy)
-                        syy = -vk_dphi(du, dv + ac, lk, amp) + vk_dphi(du, dv + ad, lk, amp) +
-                              vk_dphi(du, dv + bc, lk, amp) - vk_dphi(du, dv + bd, lk, amp);
+                        syy = -D(du, dv + ac) + D(du, dv + ad) +
+                              D(du, dv + bc) - D(du, dv + bd);
                     if (nxy)
-                        sxy = -vk_dphi(du + s1, dv - s2, lk, amp) +
-                              vk_dphi(du + s1, dv + s2, lk, amp) +
-                              vk_dphi(du - s1, dv - s2, lk, amp) - vk_dphi(du - s1, dv + s2, lk, amp);
-                    syx = -vk_dphi(du - s2, dv + s1, lk, amp) + vk_dphi(du + s2, dv + s1, lk, amp) +
-                          vk_dphi(du - s2, dv - s1, lk, amp) - vk_dphi(du + s2, dv - s1, lk, amp);
+                        sxy = -D(du + s1, dv - s2) +
+                              D(du + s1, dv + s2) +
+                              D(du - s1, dv - s2) - D(du - s1, dv + s2);
+                    syx = -D(du - s2, dv + s1) + D(du + s2, dv + s1) +
+                          D(du - s2, dv - s1) - D(du + s2, dv - s1);
                 }
                 cxx += 0.5 * sxx * kk * a.cn2[l];
                 cxy += 0.5 * sxy * kk * a.cn2[l];
@@ -319,6 +374,8 @@ __global__ void __launch_bounds__(kWaves * 64) truth_kernel(MatcovArgs a) {
     const int wave = threadIdx.x >> 6;
     const int lx = blockIdx.x * kRows + lane;
     const int ly0 = blockIdx.y * kCols + wave * kColsPerWave;
+    __shared__ __attribute__((aligned(16))) double tab[kTabN * kCoef];
+    load_table(a.ftab, tab);
     if (lx >= a.nrows) return;
     const int gx = lx + a.xoffset;
     const int ns = a.truth_nsub;
@@ -338,7 +395,7 @@ __global__ void __launch_bounds__(kWaves * 64) truth_kernel(MatcovArgs a) {
         const double dv = a.Y[a.truth_base + i] - a.Y[a.truth_base + j];
         double covar = 0.0;
         for (int l = 0; l < a.Nlayer; ++l) {
-            if (ss > 0) covar += 0.5 * slope_cov(kind, du, dv, s, s, a.lk[l], a.amp[l]) * kk * a.cn2[l];
+            if (ss > 0) covar += 0.5 * slope_cov(tab, kind, du, dv, s, s, a.lk[l], a.amp[l]) * kk * a.cn2[l];
         }
         a.out[(long)ly * a.lda + lx] = covar;
     }
@@ -362,6 +419,69 @@ inline int pack_truth(long g, const moao_tomo_view* t, const std::vector<long>& 
     int xy = 0;
     if (i >= t->Nsubap[w]) { i -= t->Nsubap[w]; xy = 1; }
     return (int)(((off[w] + i) << 9) | (w << 1) | xy);
+}
+
+// Coefficients of the table of f: interpolation at the eight Chebyshev points of an interval, in
+// extended precision, as a polynomial in z = mantissa - (1 + 1/(2 kSub)) of the interval's start.
+std::vector<double> structure_table() {
+    auto series = [](long double t) {
+        const long double q53 = std::pow(t, 5.0L / 6.0L), x22 = t / 4;
+        const double ga[11] = MOAO_VK_GA, gma[11] = MOAO_VK_GMA;
+        long double xn = 0.5L, s = 0;
+        for (int n = 0; n <= 10; ++n, xn *= x22) s += (gma[n] * q53 + ga[n]) * xn;
+        return -s;
+    };
+    auto asymptote = [](long double t) {
+        const long double x = std::sqrt(t), ix = 1 / x;
+        return kK2 - kK3 * std::exp(-x) * std::cbrt(x) *
+                         (1 + ix * (kA1 + ix * (kA2 + ix * (long double)kA3)));
+    };
+    std::vector<double> tab((size_t)kTabN * kCoef, 0.0);
+    for (int k = 0; k + 1 < kTabN; ++k) {
+        // intervals past the border's are one entry later (its second copy)
+        const int border = (int)((std::floor(std::log2(kTBorder)) - kLo) * kSub +
+                                 (kTBorder / std::exp2(std::floor(std::log2(kTBorder))) - 1) * kSub);
+        const int iv = k <= border ? k : k - 1;
+        const int e = kLo + iv / kSub;
+        const long double mid = 1 + (iv % kSub) / (long double)kSub + 0.5L / kSub;
+        long double z[kCoef], c[kCoef];
+        for (int n = 0; n < kCoef; ++n) {
+            z[n] = std::cos((2 * n + 1) * (long double)kPi / (2 * kCoef)) / (2 * kSub);
+            const long double t = std::ldexp(mid + z[n], e);
+            c[n] = k <= border ? series(t) : asymptote(t);
+        }
+        for (int o = 1; o < kCoef; ++o)  // Newton's divided differences
+            for (int n = kCoef - 1; n >= o; --n) c[n] = (c[n] - c[n - 1]) / (z[n] - z[n - o]);
+        long double p[kCoef] = {};       // ... multiplied out
+        for (int n = kCoef - 1; n >= 0; --n) {
+            for (int d = kCoef - 1; d >= 1; --d) p[d] = p[d - 1] - z[n] * p[d];
+            p[0] = c[n] - z[n] * p[0];
+        }
+        for (int d = 0; d < kCoef; ++d) tab[2 * ((size_t)(d / 2) * kTabN + k) + d % 2] = (double)p[d];
+    }
+    tab[2 * (size_t)(kTabN - 1)] = kK2;
+    return tab;
+}
+
+// The table on the device, made on the first use and kept for the life of the process (55 KiB).
+int structure_table_dev(const double** out) {
+    static std::mutex mu;
+    static double* dev = nullptr;
+    std::lock_guard<std::mutex> g(mu);
+    if (!dev) {
+        const std::vector<double> tab = structure_table();
+        double* d = nullptr;
+        MOAO_HIP_TRY(hipMalloc(reinterpret_cast<void**>(&d), sizeof(double) * tab.size()));
+        if (hipMemcpy(d, tab.data(), sizeof(double) * tab.size(), hipMemcpyHostToDevice) !=
+            hipSuccess) {
+            (void)hipFree(d);
+            set_error("matcov: table upload failed");
+            return MOAO_ERR_HIP;
+        }
+        dev = d;
+    }
+    *out = dev;
+    return MOAO_OK;
 }
 
 size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
@@ -484,6 +604,7 @@ int matcov_tile_launch(double* d_data, int nrows, int ncols, int xoffset, int yo
     MOAO_HIP_TRY(hipMemcpyAsync(d, host.data(), total, hipMemcpyHostToDevice, stream));
 
     MatcovArgs a;
+    if (int rc = structure_table_dev(&a.ftab)) return rc;
     a.out = d_data;
     a.lda = lda;
     a.nrows = nrows;

@@ -149,3 +149,22 @@ def test_whole_matrix_pair_kernel_is_bit_identical_to_element_tiles(tmp_path):
             bb = np.empty((m, W), order="F")
             gm.matcov_tile(bb, m, W, 0, c0, m, t, gm.CTM)
             assert np.array_equal(bb, B[:, c0:c0 + W]), (n, "Ctm", c0)
+
+
+@pytest.mark.parametrize("L0", [0.3, 2.0, 10.66, 25.0, 400.0, 1e5])
+def test_structure_function_range(tmp_path, L0):
+    """Outer scales that take the structure function's arguments q = 2 pi r / L0 through the whole
+    range of its table and past both ends (q < 1/256, q > 45), and near the border of its two
+    branches (r = 3/4 L0: 8 m for L0 = 10.66): Cmm, Ctm and Ctt within 1e-12 of the largest entry
+    of the oracle's, as for the fixtures (second differences amplify the last-ulp differences)."""
+    from moao_amd import systems
+    spec = systems.SystemSpec(diam=8.0, nssp=9, nlgs=2, nngs=1, nlayer=3, L0=L0, seed=77)
+    s, a = systems.make_system(str(tmp_path), spec)
+    t, o = Tomo(s, a[0]), OTomo.from_files(s, a[0])
+    t.set_target(0)
+    o.set_target(0)
+    for g, r in ((np.tril(gm.cmm(t)), np.tril(om.cmm(o))), (gm.ctm(t), om.ctm(o)),
+                 (gm.ctt(t), om.ctt(o))):
+        err = np.max(np.abs(g - r)) / np.max(np.abs(r))
+        print(f"[matcov-range] L0={L0} {g.shape}: {err:.2e}", flush=True)
+        assert err <= 1e-12
