@@ -875,13 +875,17 @@ __global__ void symdiag_kernel(const T* __restrict__ B, long ldb, int K, T* __re
 // faster ones.  16-row workgroups while they fit the 256 CUs at once (then a wave's own chain of
 // MFMAs is the time, and a 16-row block's is half a 32-row block's), else 32-row workgroups up to
 // the count where the slice kernels' operand reuse through LDS wins: the direct kernel reads every
-// operand from L1/L2, and op(B) = B or FP32's twice as fast MFMA reach that limit sooner.
-// Measured, slice kernel -> direct kernel, us (M x N x K, op(B) = B^T): FP64 152 x 128 x 128
-// 19.5 -> 7.4, 1000 x 512 x 512 63 -> 19, 2400 x 1024 x 1024 147 -> 123, 5000 x 1024 x 1024
-// (1,256 workgroups) 216 -> 199, 10000 x 1024 x 1024 (2,504) 394 -> 389, 10000 x 2048 x 2048 1259
-// -> 1507; op(B) = B 152 x 128 x 128 18.6 -> 9.1, 5000 x 512 x 512 (628) 81 -> 77, 5000 x 1024 x
-// 1024 (1,256) 204 -> 231; FP32 2400 x 128 x 128 15.7 -> 6.3, 20000 x 256 x 256 (1,250) 51 -> 47,
-// 5000 x 512 x 512 (628) 57 -> 52, 10000 x 512 x 512 (1,252) 76 -> 88.
+// operand from L1/L2.  That point comes the sooner the longer K (operands that leave L2), with FP32's
+// twice as fast MFMAs, and for FP64 op(B) = B (lane exchanges).
+// Measured, slice kernel -> direct kernel, us (M x N x K; w = 32-row workgroups).  FP64 op(B) = B^T:
+// 152 x 128 x 128 19.5 -> 7.4, 300 x 1000 x 8192 816 -> 225, 1000 x 1000 x 8192 (w 256) 822 -> 375,
+// 5000 x 1024 x 1024 (1,256) 216 -> 199, 20000 x 256 x 256 (1,250) 70 -> 61, 1500 x 1500 x 16384 (564)
+// 2035 -> 2033, 2336 x 2336 x 2048 (1,387) 416 -> 452, 2336 x 2336 x 8192 1637 -> 1782, 10000 x 2048 x
+// 2048 (5,008) 1259 -> 1507.  FP64 op(B) = B: 152 x 128 x 128 18.6 -> 9.1, 1000 x 1000 x 2048 (256)
+// 200 -> 103, 5000 x 512 x 512 (628) 81 -> 77, 1500 x 1500 x 2048 (564) 254 -> 269.  FP32 op(B) = B^T:
+// 2400 x 128 x 128 15.7 -> 6.3, 20000 x 256 x 256 (1,250) 51 -> 47, 1000 x 1000 x 2048 (256) 142 -> 62,
+// 1500 x 1500 x 1024 (564) 87 -> 103.  FP32 op(B) = B: 3000 x 1000 x 2048 (752) 184 -> 153, 2336 x
+// 2336 x 2048 (1,387) 247 -> 296.
 template <typename T>
 int direct_rows(const GemmArgs<T>& g, int maxM) {
     double cells = 0;  // C elements of the launch, trapezoids without their upper part
@@ -895,7 +899,12 @@ int direct_rows(const GemmArgs<T>& g, int maxM) {
     }
     const double groups = cells / (16 * BN);
     if (groups <= 256) return 16;
-    const double limit = sizeof(T) == 8 ? (g.transb == 1 ? 1500 : 640) : (g.K <= 256 ? 1500 : 640);
+    double limit;
+    if (sizeof(T) == 8)
+        limit = g.transb == 1 ? (g.K <= 256 ? 1500 : g.K <= 4096 ? 1280 : 640)
+                              : (g.K <= 512 ? 640 : 500);
+    else
+        limit = g.K <= 256 ? 1500 : g.transb == 1 ? 400 : 1000;
     return groups / 2 <= limit ? 32 : 0;
 }
 
