@@ -93,7 +93,62 @@ __global__ void sumsq_partial(const double* __restrict__ a, long lda, int rows, 
     if (threadIdx.x == 0) part[blockIdx.x] = red[0];
 }
 
+// rid[k] = the range that holds index k (-1: none) and the columns k of U^T (p x n, leading
+// dimension ldt), U the indicator of the ranges [ends[2q], ends[2q + 1]).
+__global__ void lowrank_init(const int* __restrict__ ends, int p, int n, int* __restrict__ rid,
+                             float* __restrict__ Ut, long ldt) {
+    const int k = blockIdx.x * 256 + threadIdx.x;
+    if (k >= n) return;
+    int r = -1;
+    for (int q = 0; q < p; ++q) {
+        const bool in = k >= ends[2 * q] && k < ends[2 * q + 1];
+        if (in) r = q;
+        Ut[q + (long)k * ldt] = in ? 1.0f : 0.0f;
+    }
+    rid[k] = r;
+}
+
+// Z = X U for the indicator U: Z[r, q] = sum of X[r, k] over the columns k of range q.  The range's
+// columns are cut into gridDim.z parts summed apart (part [.][r, q] in P) and added by
+// range_sums_add in part order.  A workgroup sums 64 rows, its four waves every fourth column.
+// Bound by the one read of X: as a K x N product this was one 128-column tile with 2 nlgs of its
+// columns in use (n = 9,632, m = 1,376: 515 -> 30 us).
+__global__ void range_sums(const double* __restrict__ X, long ldx, int rows,
+                           const int* __restrict__ ends, double* __restrict__ P, int p) {
+    __shared__ double red[4][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, q = blockIdx.y;
+    const int r = blockIdx.x * 64 + lane;
+    const int k0 = ends[2 * q], len = ends[2 * q + 1] - k0;
+    const int b = k0 + (int)((long)len * blockIdx.z / gridDim.z);
+    const int e = k0 + (int)((long)len * (blockIdx.z + 1) / gridDim.z);
+    double acc = 0.0;
+    if (r < rows) {
+        double a[4] = {0, 0, 0, 0};
+        int k = b + wave;
+        for (; k + 12 < e; k += 16)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) a[u] += X[r + (long)(k + 4 * u) * ldx];
+        for (; k < e; k += 4) a[0] += X[r + (long)k * ldx];
+        acc = (a[0] + a[1]) + (a[2] + a[3]);
+    }
+    red[wave][lane] = acc;
+    __syncthreads();
+    if (wave == 0 && r < rows)
+        P[(long)blockIdx.z * rows * p + r + (long)q * rows] =
+            (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
+}
+
+__global__ void range_sums_add(const double* __restrict__ P, long cells, int parts,
+                               double* __restrict__ Z) {
+    const long i = (long)blockIdx.x * 256 + threadIdx.x;
+    if (i >= cells) return;
+    double acc = P[i];
+    for (int z = 1; z < parts; ++z) acc += P[z * cells + i];
+    Z[i] = acc;
+}
+
 constexpr int kNormBlocks = 1024;
+constexpr int kSumParts = 8;    // parts of a range in range_sums
 
 dim3 grid2(int rows, int cols) { return dim3((rows + 63) / 64, (cols + 3) / 4); }
 
@@ -164,8 +219,8 @@ struct MixedWs {
     float* invL;   // leaves
     double* E;     // m x n residual / correction
     double* Ctm0;  // m x n copy of the right-hand side for the residuals
-    double* U;     // n x p indicator
     double* W;     // p x n
+    double* P;     // kSumParts x (m or p) x p partial sums of range_sums
     double* Z;     // m x p
     double* Z2;    // m x p
     double* Sinv;  // p x p
@@ -173,6 +228,7 @@ struct MixedWs {
     double* part;  // norm partial sums
     int* rid;      // n range ids
     int* info;
+    int* ends;     // p ranges: first index, one past the last
 };
 
 }  // namespace
@@ -197,8 +253,8 @@ static size_t mixed_layout(long n, long m, int p, int mode, std::vector<size_t>*
     take(sizeof(float) * recon_invl_doubles(n));
     take(sizeof(double) * m * n);
     take(sizeof(double) * m * n);
-    take(sizeof(double) * n * q);
     take(sizeof(double) * q * n);
+    take(sizeof(double) * kSumParts * std::max(m, (long)q) * q);
     take(sizeof(double) * m * q);
     take(sizeof(double) * m * q);
     take(sizeof(double) * q * q);
@@ -206,6 +262,7 @@ static size_t mixed_layout(long n, long m, int p, int mode, std::vector<size_t>*
     take(sizeof(double) * kNormBlocks);
     take(sizeof(int) * n);
     take(sizeof(int) * 4);
+    take(sizeof(int) * 2 * q);
     take(sizeof(double) * gemm_symdiag_elems(n));  // Cmm's symmetric diagonal blocks
     if (mode == MOAO_MIXED_BF16) {
         const long ld = plane_ld(n);
@@ -246,15 +303,15 @@ int reconstructor_mixed_dev(long n, long m, const double* Cmm, long ldCmm, doubl
               (double*)(b + offs[3]), (double*)(b + offs[4]), (double*)(b + offs[5]),
               (double*)(b + offs[6]), (double*)(b + offs[7]), (double*)(b + offs[8]),
               (double*)(b + offs[9]), (double*)(b + offs[10]), (double*)(b + offs[11]),
-              (int*)(b + offs[12]), (int*)(b + offs[13])};
-    double* const symd = (double*)(b + offs[14]);
+              (int*)(b + offs[12]), (int*)(b + offs[13]), (int*)(b + offs[14])};
+    double* const symd = (double*)(b + offs[15]);
     const int N = (int)n, M = (int)m;
     SplitWs sw{};
     const SplitWs* swp = nullptr;
     if (split) {
         const long ld = plane_ld(n);
-        sw = SplitWs{(unsigned short*)(b + offs[15]), (unsigned short*)(b + offs[16]),
-                     (unsigned short*)(b + offs[17]), ld, n * ld, n * ld, xr * ld};
+        sw = SplitWs{(unsigned short*)(b + offs[16]), (unsigned short*)(b + offs[17]),
+                     (unsigned short*)(b + offs[18]), ld, n * ld, n * ld, xr * ld};
         swp = &sw;
     }
 
@@ -272,30 +329,20 @@ int reconstructor_mixed_dev(long n, long m, const double* Cmm, long ldCmm, doubl
         return MOAO_OK;
     };
 
-    // --- range ids, U, U^T
-    {
-        std::vector<int> rid(n, -1);
-        std::vector<double> U((size_t)n * std::max(p, 1), 0.0);
-        std::vector<float> Ut((size_t)std::max(p, 1) * n, 0.0f);
-        for (int q = 0; q < p; ++q)
-            for (long k = rg.start[q]; k < rg.start[q] + rg.len[q]; ++k) {
-                rid[k] = q;
-                U[k + (size_t)q * n] = 1.0;
-            }
-        MOAO_HIP_TRY(hipMemcpyAsync(w.rid, rid.data(), sizeof(int) * n, hipMemcpyHostToDevice, s));
-        if (p) {
-            MOAO_HIP_TRY(hipMemcpyAsync(w.U, U.data(), sizeof(double) * n * p,
-                                        hipMemcpyHostToDevice, s));
-            // U^T rows live below the m right-hand-side rows of X32 (leading dimension xr)
-            std::vector<float> Xu((size_t)p * n);
-            for (int q = 0; q < p; ++q)
-                for (long k = 0; k < n; ++k) Xu[q + (size_t)k * p] = (float)U[k + (size_t)q * n];
-            MOAO_HIP_TRY(hipMemcpy2DAsync(w.X32 + m, xr * sizeof(float), Xu.data(),
-                                          p * sizeof(float), p * sizeof(float), n,
-                                          hipMemcpyHostToDevice, s));
+    // --- range ids and U^T (rows m .. m+p-1 of X32), written on the device from the ranges
+    if (p) {
+        std::vector<int> ends(2 * (size_t)p);
+        for (int q = 0; q < p; ++q) {
+            ends[2 * q] = (int)rg.start[q];
+            ends[2 * q + 1] = (int)(rg.start[q] + rg.len[q]);
         }
-        MOAO_HIP_TRY(hipStreamSynchronize(s));  // host vectors go out of scope
+        MOAO_HIP_TRY(hipMemcpyAsync(w.ends, ends.data(), sizeof(int) * 2 * p,
+                                    hipMemcpyHostToDevice, s));
+        MOAO_HIP_TRY(hipStreamSynchronize(s));  // the host vector goes out of scope
     }
+    hipLaunchKernelGGL(lowrank_init, dim3((N + 255) / 256), dim3(256), 0, s, w.ends, p, N, w.rid,
+                       w.X32 + m, xr);
+    MOAO_HIP_TRY(hipGetLastError());
 
     // --- 1. C0 in FP32; right-hand sides Ctm in FP32
     {
@@ -327,13 +374,23 @@ int reconstructor_mixed_dev(long n, long m, const double* Cmm, long ldCmm, doubl
     if (int rc = trsm_right_lower_notrans<float>(n, w.C0, n, w.invL, all, s, nullptr, swp))
         return rc;
 
+    // Z = X U (rows x p, leading dimension rows)
+    auto times_u = [&](const double* X, long ldx, int rows, double* Z) -> int {
+        hipLaunchKernelGGL(range_sums, dim3((rows + 63) / 64, p, kSumParts), dim3(256), 0, s, X,
+                           ldx, rows, w.ends, w.P, p);
+        const long cells = (long)rows * p;
+        hipLaunchKernelGGL(range_sums_add, dim3((unsigned)((cells + 255) / 256)), dim3(256), 0, s,
+                           w.P, cells, kSumParts, Z);
+        MOAO_HIP_TRY(hipGetLastError());
+        return MOAO_OK;
+    };
+
     // --- 3. Woodbury terms
     std::vector<double> Sinv;
     if (p) {
         hipLaunchKernelGGL(cvt_f32_f64, grid2(p, N), dim3(256), 0, s, w.X32 + m, xr, w.W, p, p, N);
         MOAO_HIP_TRY(hipGetLastError());
-        auto g = gemm_args<double>(p, p, N, 1.0, w.W, p, w.U, n, 0, 0.0, w.WU, p);
-        if (int rc = gemm_f64(g, s)) return rc;
+        if (int rc = times_u(w.W, p, p, w.WU)) return rc;
         std::vector<double> S((size_t)p * p);
         MOAO_HIP_TRY(hipMemcpyAsync(S.data(), w.WU, sizeof(double) * p * p, hipMemcpyDeviceToHost,
                                     s));
@@ -354,9 +411,8 @@ int reconstructor_mixed_dev(long n, long m, const double* Cmm, long ldCmm, doubl
     // Y (FP64) -> X; X -= (X U) S^{-1} W
     auto woodbury = [&](double* X, long ldx) -> int {
         if (!p) return MOAO_OK;
-        auto g = gemm_args<double>(M, p, N, 1.0, X, ldx, w.U, n, 0, 0.0, w.Z, m);
-        if (int rc = gemm_f64(g, s)) return rc;
-        g = gemm_args<double>(M, p, p, 1.0, w.Z, m, w.Sinv, p, 0, 0.0, w.Z2, m);
+        if (int rc = times_u(X, ldx, M, w.Z)) return rc;
+        auto g = gemm_args<double>(M, p, p, 1.0, w.Z, m, w.Sinv, p, 0, 0.0, w.Z2, m);
         if (int rc = gemm_f64(g, s)) return rc;
         g = gemm_args<double>(M, N, p, -1.0, w.Z2, m, w.W, p, 0, 1.0, X, ldx);
         return gemm_f64(g, s);
@@ -364,11 +420,10 @@ int reconstructor_mixed_dev(long n, long m, const double* Cmm, long ldCmm, doubl
     hipLaunchKernelGGL(cvt_f32_f64, grid2(M, N), dim3(256), 0, s, w.X32, xr, Ctm, ldCtm, M, N);
     MOAO_HIP_TRY(hipGetLastError());
     if (debug) {
-        double a = 0, b2 = 0, c2 = 0;
+        double a = 0, b2 = 0;
         norm(Ctm, ldCtm, M, N, &a);
         if (p) norm(w.W, p, p, N, &b2);
-        if (p) norm(w.U, n, N, p, &c2);
-        std::fprintf(stderr, "[mixed] |Ctm|=%.6e |Y|=%.6e |W|=%.6e |U|=%.6e\n", ctm_norm, a, b2, c2);
+        std::fprintf(stderr, "[mixed] |Ctm|=%.6e |Y|=%.6e |W|=%.6e\n", ctm_norm, a, b2);
     }
     if (int rc = woodbury(Ctm, ldCtm)) return rc;  // Ctm now holds R_0
     if (debug && p) {
