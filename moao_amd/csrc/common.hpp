@@ -34,11 +34,22 @@ struct DevBuf {
     T* as() const { return static_cast<T*>(ptr); }
 };
 
+// What matcov uploads for a call (pinned host staging and its device copy) and, behind it on the
+// device, the covariance tables it computes there.  Grows on demand, used by one call at a time.
+struct MatcovTables {
+    DevBuf dev;
+    unsigned char* host = nullptr;
+    size_t host_bytes = 0;
+    size_t upload = 0;  // bytes of the upload part of dev
+    int ensure(size_t upload_bytes, size_t table_bytes);
+    void release();
+};
+
 // One per process (single GPU).  Owns the library stream and reusable scratch.
 struct Context {
     int device = -1;
     hipStream_t stream = nullptr;
-    DevBuf matcov_tables;   // per-call tomo upload for matcov
+    MatcovTables matcov_tables;  // per-call tomo upload for matcov
     DevBuf host_stage;      // device copy of a host matrix for the host-pointer entry points
     DevBuf host_stage2;
     DevBuf recon_ws;        // reconstructor workspace (inverse leaves + status word)

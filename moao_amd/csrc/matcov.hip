@@ -18,16 +18,19 @@
 //  * per-layer constants 2*pi/L0 and k1*L0^(5/3) are computed once on the host with the
 //    reference's own expressions (identical bits), not per call of the structure function;
 //  * type 1 skips workgroups whose tile lies wholly above the diagonal;
-//  * a whole Cmm or Ctm (the lapack path's call) runs pair_kernel instead: one lane per pair
-//    of subapertures computes the pair's xx, xy, yx and yy elements, sharing the structure
-//    functions those four have in common (9 evaluations per layer instead of 14 for sensors
-//    of equal subaperture size), bit-identical to the element kernel.
+//  * sensors on one regular grid (find_lattices) have as many covariances as the grid has
+//    differences: lattice_table evaluates those, lattice_fill (whole matrices) and meas_kernel
+//    (tiles) read them;
+//  * the other pairs of a whole Cmm or Ctm (the lapack path's call) run pair_kernel: one lane
+//    per pair of subapertures computes the pair's xx, xy, yx and yy elements, sharing the structure
+//    functions those four have in common, bit-identical to the element kernel.
 // Contraction into FMA is disabled here so each product/sum rounds as in the reference; the
 // only differences left are the last-ulp differences of the device pow/exp/sqrt.
 #pragma clang fp contract(off)
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -78,6 +81,8 @@ constexpr int kColsPerWave = 4; // columns per wave
 constexpr int kWaves = 8;       // waves per workgroup
 constexpr int kCols = kColsPerWave * kWaves;
 
+constexpr int kLattice = -1, kFree = -2;  // MatcovArgs::cls without a table
+
 struct MatcovArgs {
     double* out;
     long lda;
@@ -102,6 +107,16 @@ struct MatcovArgs {
     const double* Y;
     int truth_base;         // Nsubap_t*(Nw-1), index of the truth sensor's first subap
     int truth_nsub;         // Nsubap of the truth sensor
+    // lattices: packed integer place (iy << 16 | ix) of every subaperture on its sensor's grid and
+    // the grid's origin on every layer; cls[m*Nw + n]: slot of the pair's covariance table (rows of
+    // sensor m, columns of n), kLattice (same grid, no table) or kFree
+    const int* lat;         // [Nx]
+    const double* u0;       // [Nw*Nlayer]
+    const double* v0;
+    const int* cls;         // [Nw*Nw]
+    const int* slots;       // sensor pairs (m << 8 | n) of the tables
+    double* ptab;           // [slots][3][W*W]: xx, yy, xy by (dy + ext - 1)*W + dx + ext - 1
+    int Nw, ext;            // ext: cells across the widest lattice; W = 2*ext - 1
     // pair kernel (whole matrices of types 1 and 3): one entry per subaperture of the row and
     // column sensors, {(pos << 9) | (wfs << 1), matrix index of its x slope}; the y slope sits
     // nsub[wfs] further
@@ -204,6 +219,125 @@ __device__ __forceinline__ double slope_cov(const double* tab, int kind, double 
     }
 }
 
+// Separation of subapertures p1 (sensor m) and p2 (sensor n) on layer l.  On a common lattice it
+// is a function of the integer places' difference alone, so every pair of one difference has the
+// same bits, whichever kernel computes it; else the difference of the positions.
+__device__ __forceinline__ void lattice_separation(const MatcovArgs& a, int m, int n, int dx, int dy,
+                                                   int l, double step, double& du, double& dv) {
+    const int om = m * a.Nlayer + l, on = n * a.Nlayer + l;
+    du = (a.u0[om] - a.u0[on]) + dx * step;
+    dv = (a.v0[om] - a.v0[on]) + dy * step;
+}
+__device__ __forceinline__ int lat_dx(int a, int b) { return (a & 0xffff) - (b & 0xffff); }
+__device__ __forceinline__ int lat_dy(int a, int b) { return (a >> 16) - (b >> 16); }
+__device__ __forceinline__ void separation(const MatcovArgs& a, bool lattice, int m, int n, int p1,
+                                           int p2, int l, double step, double& du, double& dv) {
+    if (lattice) {
+        lattice_separation(a, m, n, lat_dx(a.lat[p1], a.lat[p2]), lat_dy(a.lat[p1], a.lat[p2]), l,
+                           step, du, dv);
+        return;
+    }
+    const long o = (long)l * a.Nx;
+    du = a.u[o + p1] - a.u[o + p2];
+    dv = a.v[o + p1] - a.v[o + p2];
+}
+
+// Covariance tables of the sensor pairs on a common lattice (both sensors' subapertures on one
+// grid with the same size on every layer: every LGS pair of one altitude, every NGS pair).  All
+// subaperture pairs of one lattice difference have the same xx, yy and xy (= yx) covariance, and
+// there are (2*ext - 1)^2 differences against Nsubap^2 pairs (79^2 against 1168^2 at 40 x 40): one
+// lane per difference evaluates it, lattice_fill and meas_kernel read it.
+__global__ void __launch_bounds__(kWaves * 64) lattice_table(MatcovArgs a) {
+    __shared__ __attribute__((aligned(16))) double tab[kTabN * kCoef];
+    load_table(a.ftab, tab);
+    const int W = 2 * a.ext - 1, e = blockIdx.x * (kWaves * 64) + threadIdx.x;
+    if (e >= W * W) return;
+    const int pr = a.slots[blockIdx.y], m = pr >> 8, n = pr & 0xff;
+    const int dx = e % W - (a.ext - 1), dy = e / W - (a.ext - 1);
+    const double kk = kLambda2 / (a.sspsz[m] * a.sspsz[n]);
+    double cxx = 0.0, cxy = 0.0, cyy = 0.0;
+    for (int l = 0; l < a.Nlayer; ++l) {
+        const double sz = a.sspL[m * a.Nlayer + l];
+        if (!(sz > 0)) continue;
+        double du, dv;
+        lattice_separation(a, m, n, dx, dy, l, sz, du, dv);
+        const double s1 = sz * 0.5, ad = s1 + s1, bc = -ad, lk = a.lk[l], amp = a.amp[l];
+        auto D = [&](double x, double y) { return vk_table(tab, x, y, lk, amp); };
+        const double d0 = D(du, dv);
+        const double sxx = -d0 + D(du + ad, dv) + D(du + bc, dv) - d0;
+        const double syy = -d0 + D(du, dv + ad) + D(du, dv + bc) - d0;
+        const double sxy = -D(du + s1, dv - s1) + D(du + s1, dv + s1) + D(du - s1, dv - s1) -
+                           D(du - s1, dv + s1);
+        cxx += 0.5 * sxx * kk * a.cn2[l];
+        cyy += 0.5 * syy * kk * a.cn2[l];
+        cxy += 0.5 * sxy * kk * a.cn2[l];
+    }
+    double* o = a.ptab + (long)blockIdx.y * 3 * W * W + e;
+    o[0] = cxx;
+    o[W * W] = cyy;
+    o[2 * W * W] = cxy;
+}
+
+// Whole Cmm or Ctm: the pairs that have a table.  Bound by its stores (8 B an element; the tables
+// are read from L2).  Rows and columns as in pair_kernel, which takes the other pairs.
+__global__ void __launch_bounds__(256) lattice_fill(MatcovArgs a, int cols_per_wave) {
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int rs = blockIdx.x * 64 + lane;
+    const int cs0 = (blockIdx.y * 4 + wave) * cols_per_wave;
+    if (rs >= a.nrsub) return;
+    const int2 re = a.rsub[rs];
+    const int m = (re.x >> 1) & 0xff, p1 = re.x >> 9, la = a.lat[p1];
+    const int xr = re.y, yr = re.y + a.nsub[m];
+    const int W = 2 * a.ext - 1, WW = W * W;
+    for (int c = 0; c < cols_per_wave; ++c) {
+        const int cs = cs0 + c;
+        if (cs >= a.ncsub) break;
+        const int2 ce = a.csub[cs];
+        const int n = (ce.x >> 1) & 0xff, p2 = ce.x >> 9;
+        const int xc = ce.y, yc = ce.y + a.nsub[n];
+        const bool lo = a.type_mat == 1;
+        const bool nxx = !lo || xr >= xc, nyy = !lo || yr >= yc;
+        const bool nxy = !lo || xr >= yc, nyx = !lo || yr >= xc;
+        const int slot = a.cls[m * a.Nw + n];
+        if (!nyx || slot < 0) continue;
+        const int lb = a.lat[p2];
+        const double* t = a.ptab + (long)slot * 3 * WW + (lat_dy(la, lb) + a.ext - 1) * W +
+                          lat_dx(la, lb) + a.ext - 1;
+        double cxx = t[0], cyy = t[WW], cxy = t[2 * WW], cyx = cxy;
+        if (m == n) {
+            if (m < a.nlgs) {
+                if (p1 == p2) {
+                    cxx += a.nxx[p1];
+                    cyy += a.nyy[p1];
+                    cxy += a.nxy[p1];
+                    cyx += a.nxy[p1];
+                }
+                cxx += a.lgs_cst;
+                cyy += a.lgs_cst;
+            } else if (p1 == p2) {
+                cxx += a.nNGS[m - a.nlgs];
+                cyy += a.nNGS[m - a.nlgs];
+            }
+        }
+        double* ox = a.out + (long)xc * a.lda;
+        double* oy = a.out + (long)yc * a.lda;
+        if (nxx) ox[xr] = cxx;
+        ox[yr] = cyx;
+        if (nxy) oy[xr] = cxy;
+        if (nyy) oy[yr] = cyy;
+    }
+}
+
+// Whether a sensor of rows [m0, m1] and one of columns [n0, n1] have to be evaluated (no table).
+__device__ __forceinline__ bool any_without_table(const MatcovArgs& a, int m0, int m1, int n0,
+                                                  int n1) {
+    bool any = false;
+    for (int m = m0; m <= m1; ++m)
+        for (int n = n0; n <= n1; ++n) any = any || a.cls[m * a.Nw + n] < 0;
+    return any;
+}
+
 __global__ void __launch_bounds__(kWaves * 64) meas_kernel(MatcovArgs a) {
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
@@ -215,7 +349,11 @@ __global__ void __launch_bounds__(kWaves * 64) meas_kernel(MatcovArgs a) {
         if (last_row < a.yoffset + (int)blockIdx.y * kCols) return;
     }
     __shared__ __attribute__((aligned(16))) double tab[kTabN * kCoef];
-    load_table(a.ftab, tab);
+    const int cl = min((int)blockIdx.y * kCols + kCols, a.ncols) - 1;
+    const int rl = min((int)blockIdx.x * kRows + kRows, a.nrows) - 1;
+    if (any_without_table(a, (a.rowtab[blockIdx.x * kRows] >> 1) & 0xff, (a.rowtab[rl] >> 1) & 0xff,
+                          (a.coltab[blockIdx.y * kCols] >> 1) & 0xff, (a.coltab[cl] >> 1) & 0xff))
+        load_table(a.ftab, tab);
     if (lx >= a.nrows) return;
     const int ri = a.rowtab[lx];
     const int m = (ri >> 1) & 0xff, xi = ri & 1, p1 = ri >> 9;
@@ -227,17 +365,25 @@ __global__ void __launch_bounds__(kWaves * 64) meas_kernel(MatcovArgs a) {
         const int ci = a.coltab[ly];
         const int n = (ci >> 1) & 0xff, xj = ci & 1, p2 = ci >> 9;
         const int kind = xi * 2 + xj;
+        const int cls = a.cls[m * a.Nw + n];
         const double kk = kLambda2 / (a.sspsz[m] * a.sspsz[n]);
         double covar = 0.0;
-        for (int l = 0; l < a.Nlayer; ++l) {
-            const double sml = a.sspL[m * a.Nlayer + l];
-            const double snl = a.sspL[n * a.Nlayer + l];
-            if ((sml > 0) && (snl > 0)) {
-                const long o = (long)l * a.Nx;
-                const double du = a.u[o + p1] - a.u[o + p2];
-                const double dv = a.v[o + p1] - a.v[o + p2];
-                covar += 0.5 * slope_cov(tab, kind, du, dv, sml * 0.5, snl * 0.5, a.lk[l], a.amp[l]) *
-                         kk * a.cn2[l];
+        if (cls >= 0) {
+            const int W = 2 * a.ext - 1, la = a.lat[p1], lb = a.lat[p2];
+            covar = a.ptab[((long)cls * 3 + (kind == 0 ? 0 : kind == 3 ? 1 : 2)) * W * W +
+                           (lat_dy(la, lb) + a.ext - 1) * W + lat_dx(la, lb) + a.ext - 1];
+        } else {
+            // on a common lattice yx is xy, as in the tables
+            const int k = cls == kLattice && kind == 2 ? 1 : kind;
+            for (int l = 0; l < a.Nlayer; ++l) {
+                const double sml = a.sspL[m * a.Nlayer + l];
+                const double snl = a.sspL[n * a.Nlayer + l];
+                if ((sml > 0) && (snl > 0)) {
+                    double du, dv;
+                    separation(a, cls == kLattice, m, n, p1, p2, l, sml, du, dv);
+                    covar += 0.5 * slope_cov(tab, k, du, dv, sml * 0.5, snl * 0.5, a.lk[l],
+                                             a.amp[l]) * kk * a.cn2[l];
+                }
             }
         }
         if (m == n) {
@@ -274,6 +420,15 @@ __global__ void __launch_bounds__(kWaves * 64) pair_kernel(MatcovArgs a) {
         const int2 last = a.rsub[min((int)blockIdx.x * kRows + kRows, a.nrsub) - 1];
         if (last.y + a.nsub[(last.x >> 1) & 0xff] < a.csub[blockIdx.y * kCols].y) return;
     }
+    {
+        const int2 r0 = a.rsub[blockIdx.x * kRows];
+        const int2 r1 = a.rsub[min((int)blockIdx.x * kRows + kRows, a.nrsub) - 1];
+        const int2 c0 = a.csub[blockIdx.y * kCols];
+        const int2 c1 = a.csub[min((int)blockIdx.y * kCols + kCols, a.ncsub) - 1];
+        if (!any_without_table(a, (r0.x >> 1) & 0xff, (r1.x >> 1) & 0xff, (c0.x >> 1) & 0xff,
+                               (c1.x >> 1) & 0xff))
+            return;  // lattice_fill's
+    }
     __shared__ __attribute__((aligned(16))) double tab[kTabN * kCoef];
     load_table(a.ftab, tab);
     if (rs >= a.nrsub) return;
@@ -292,16 +447,17 @@ __global__ void __launch_bounds__(kWaves * 64) pair_kernel(MatcovArgs a) {
         const bool lo = a.type_mat == 1;
         const bool nxx = !lo || xr >= xc, nyy = !lo || yr >= yc;
         const bool nxy = !lo || xr >= yc, nyx = !lo || yr >= xc;
-        if (!nyx) continue;  // yx has the largest row and the smallest column
+        const int cls = a.cls[m * a.Nw + n];
+        // yx has the largest row and the smallest column; pairs with a table are lattice_fill's
+        if (!nyx || cls >= 0) continue;
         const double kk = kLambda2 / (a.sspsz[m] * a.sspsz[n]);
         double cxx = 0.0, cxy = 0.0, cyx = 0.0, cyy = 0.0;
         for (int l = 0; l < a.Nlayer; ++l) {
             const double sml = a.sspL[m * a.Nlayer + l];
             const double snl = a.sspL[n * a.Nlayer + l];
             if ((sml > 0) && (snl > 0)) {
-                const long o = (long)l * a.Nx;
-                const double du = a.u[o + p1] - a.u[o + p2];
-                const double dv = a.v[o + p1] - a.v[o + p2];
+                double du, dv;
+                separation(a, cls == kLattice, m, n, p1, p2, l, sml, du, dv);
                 const double s1 = sml * 0.5, s2 = snl * 0.5;
                 const double lk = a.lk[l], amp = a.amp[l];
                 const double ac = s1 - s2, ad = s1 + s2, bc = -ad, bd = -ac;
@@ -323,8 +479,8 @@ __global__ void __launch_bounds__(kWaves * 64) pair_kernel(MatcovArgs a) {
                     const double q2 = D(du + s1, dv + s2);
                     const double q3 = D(du - s1, dv - s2);
                     const double q4 = D(du - s1, dv + s2);
-                    if (nxy) sxy = -q1 + q2 + q3 - q4;
-                    syx = -q4 + q2 + q3 - q1;
+                    sxy = -q1 + q2 + q3 - q4;
+                    syx = cls == kLattice ? sxy : -q4 + q2 + q3 - q1;
                 } else {
                     if (nxx)
                         sxx = -D(du + ac, dv) + D(du + ad, dv) +
@@ -484,12 +640,86 @@ int structure_table_dev(const double** out) {
     return MOAO_OK;
 }
 
+// Regular grids among the sensors' subapertures.
+struct Lattices {
+    std::vector<int> place;         // [Nx] iy << 16 | ix
+    std::vector<double> u0, v0;     // [Nw*Nlayer] grid origin on each layer
+    std::vector<char> ok;           // [Nw] the sensor is a grid on every layer it sees
+    int ext = 1;                    // cells across the widest grid
+    // Sensors m and n on one grid: the same subaperture size, on the ground and on every layer.
+    bool same(const moao_tomo_view* t, int m, int n) const {
+        if (!ok[m] || !ok[n] || t->Nssp[m] != t->Nssp[n]) return false;
+        const int L = t->Nlayer;
+        for (int l = 0; l < L; ++l)
+            if (t->sspSizeL[m * L + l] != t->sspSizeL[n * L + l]) return false;
+        return true;
+    }
+};
+
+// A sensor is a grid when its unprojected positions are integer multiples of its subaperture size
+// apart and its positions on every layer are origin + place * size on that layer to within 4 ulp of
+// their magnitude (projection scales and shifts them; a rotated sensor fails).  The origin is the
+// mean of what the subapertures give, so it is nearer the exact one than any single position.
+Lattices find_lattices(const moao_tomo_view* t, const std::vector<long>& off,
+                       const std::vector<char>& used, const std::vector<double>& pitch) {
+    const int Nw = t->Nw, L = t->Nlayer;
+    Lattices r;
+    r.place.assign(t->Nx, 0);
+    r.u0.assign((size_t)Nw * L, 0.0);
+    r.v0.assign((size_t)Nw * L, 0.0);
+    r.ok.assign(Nw, 0);
+    std::vector<double> fx, fy;
+    for (int w = 0; w < Nw; ++w) {
+        const long N = t->Nsubap[w], o = off[w];
+        if (!used[w] || N < 1 || !(pitch[w] > 0)) continue;
+        const double* X = t->X + o;
+        const double* Y = t->Y + o;
+        const double x0 = *std::min_element(X, X + N), y0 = *std::min_element(Y, Y + N);
+        fx.resize(N);
+        fy.resize(N);
+        double far = 0, most = 0;
+        for (long i = 0; i < N; ++i) {
+            const double x = (X[i] - x0) / pitch[w], y = (Y[i] - y0) / pitch[w];
+            fx[i] = std::floor(x + 0.5);
+            fy[i] = std::floor(y + 0.5);
+            far = std::max(far, std::max(std::fabs(x - fx[i]), std::fabs(y - fy[i])));
+            most = std::max(most, std::max(fx[i], fy[i]));
+        }
+        bool ok = far < 1e-6 && most < 1024;
+        for (int l = 0; l < L && ok; ++l) {
+            const double s = t->sspSizeL[w * L + l];
+            if (!(s > 0)) continue;
+            auto origin = [&](const double* u, const double* f, double& u0) {
+                const double first = u[0] - f[0] * s;
+                double sum = 0, lo = first, hi = first;  // sum: of the differences to the first
+                for (long i = 0; i < N; ++i) {
+                    const double d = u[i] - f[i] * s;
+                    sum += d - first;
+                    lo = std::min(lo, d);
+                    hi = std::max(hi, d);
+                }
+                u0 = first + sum / N;
+                const double tol = 4 * 0x1p-52 * (std::fabs(u0) + most * s);
+                return hi - u0 <= tol && u0 - lo <= tol;  // false for a NaN
+            };
+            const long lo = (long)l * t->Nx + o;
+            ok = origin(t->u + lo, fx.data(), r.u0[w * L + l]) &&
+                 origin(t->v + lo, fy.data(), r.v0[w * L + l]);
+        }
+        if (!ok) continue;
+        r.ok[w] = 1;
+        r.ext = std::max(r.ext, (int)most + 1);
+        for (long i = 0; i < N; ++i) r.place[o + i] = (int)fy[i] << 16 | (int)fx[i];
+    }
+    return r;
+}
+
 size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 
 }  // namespace
 
 int matcov_tile_launch(double* d_data, int nrows, int ncols, int xoffset, int yoffset, int lda,
-                       const moao_tomo_view* t, int type_mat, hipStream_t stream, DevBuf* tables) {
+                       const moao_tomo_view* t, int type_mat, hipStream_t stream, MatcovTables* tables) {
     if (type_mat < 1 || type_mat > 4) {
         set_error("matcov_tile: unrecognized type_mat " + std::to_string(type_mat));
         return MOAO_ERR_ARG;
@@ -521,8 +751,13 @@ int matcov_tile_launch(double* d_data, int nrows, int ncols, int xoffset, int yo
             }
     }
 
-    std::vector<int> rowtab(nrows), coltab(ncols);
-    if (type_mat != 4) {
+    // Whole Cmm / Ctm: lattice_fill and pair_kernel (one lane per subaperture pair).
+    const bool pairs = (type_mat == 1 || type_mat == 3) && xoffset == 0 && yoffset == 0 &&
+                       nrows == row_lim && ncols == col_lim;
+    std::vector<int> rowtab, coltab;
+    if (!pairs && type_mat != 4) {
+        rowtab.resize(nrows);
+        coltab.resize(ncols);
         for (int r = 0; r < nrows; ++r)
             rowtab[r] = (type_mat == 3) ? pack_truth(r + xoffset, t, off)
                                         : pack_meas(r + xoffset, t, off);
@@ -530,13 +765,11 @@ int matcov_tile_launch(double* d_data, int nrows, int ncols, int xoffset, int yo
             coltab[c] = (type_mat == 2) ? pack_truth(c + yoffset, t, off)
                                         : pack_meas(c + yoffset, t, off);
     }
-    // Whole Cmm / Ctm: the pair kernel (one lane per subaperture pair).
-    const bool pairs = (type_mat == 1 || type_mat == 3) && xoffset == 0 && yoffset == 0 &&
-                       nrows == row_lim && ncols == col_lim;
     std::vector<int2> rsub, csub;
     std::vector<int> nsub(Nw);
     for (int w = 0; w < Nw; ++w) nsub[w] = (int)t->Nsubap[w];
     if (pairs) {
+        csub.reserve(nmeas / 2);
         for (int w = 0; w < Nw - 1; ++w)
             for (long i = 0; i < t->Nsubap[w]; ++i)
                 csub.push_back(make_int2((int)(((off[w] + i) << 9) | (w << 1)),
@@ -559,7 +792,43 @@ int matcov_tile_launch(double* d_data, int nrows, int ncols, int xoffset, int yo
     if (type_mat == 4) sspsz[0] = t->diam / t->Nssp[Nw - 1];
     const int nngs = Nw - t->nlgs;
 
-    // One contiguous upload of every vector the kernel reads.
+    // Sensors of the rows and of the columns, their lattices and the pairs that share one.
+    std::vector<int> cls, slots;
+    Lattices lat;
+    bool positions = false;  // some pair reads u, v
+    if (type_mat != 4) {
+        const int rm0 = pairs ? (rsub.front().x >> 1) & 0xff : (rowtab.front() >> 1) & 0xff;
+        const int rm1 = pairs ? (rsub.back().x >> 1) & 0xff : (rowtab.back() >> 1) & 0xff;
+        const int cn0 = pairs ? (csub.front().x >> 1) & 0xff : (coltab.front() >> 1) & 0xff;
+        const int cn1 = pairs ? (csub.back().x >> 1) & 0xff : (coltab.back() >> 1) & 0xff;
+        std::vector<char> used(Nw, 0);
+        for (int w = rm0; w <= rm1; ++w) used[w] = 1;
+        for (int w = cn0; w <= cn1; ++w) used[w] = 1;
+        lat = find_lattices(t, off, used, sspsz);
+        cls.assign((size_t)Nw * Nw, kFree);
+        for (int m = rm0; m <= rm1; ++m)
+            for (int n = cn0; n <= cn1; ++n) {
+                if (type_mat == 1 && n > m) continue;  // above the diagonal
+                if (lat.same(t, m, n)) {
+                    cls[m * Nw + n] = kLattice;
+                    slots.push_back(m << 8 | n);
+                } else {
+                    positions = true;
+                }
+            }
+        // A table entry takes 9 structure functions a layer, an element on its own 3 or 4: tables
+        // where they are the smaller work (a tile of a few hundred elements is not), 256 MiB at most.
+        const double W = 2.0 * lat.ext - 1;
+        if (slots.size() * W * W * 9 < 3.5 * nrows * ncols &&
+            slots.size() * W * W * 24 <= (256 << 20)) {
+            for (size_t k = 0; k < slots.size(); ++k)
+                cls[(slots[k] >> 8) * Nw + (slots[k] & 0xff)] = (int)k;
+        } else {
+            slots.clear();
+        }
+    }
+
+    // One contiguous upload of every vector the kernels read.
     struct Piece { const void* src; size_t bytes; size_t off; };
     std::vector<Piece> pieces;
     size_t total = 0;
@@ -568,43 +837,59 @@ int matcov_tile_launch(double* d_data, int nrows, int ncols, int xoffset, int yo
         total += align256(bytes);
         return pieces.size() - 1;
     };
-    const size_t iRow = add(rowtab.data(), sizeof(int) * nrows);
-    const size_t iCol = add(coltab.data(), sizeof(int) * ncols);
-    const size_t iU = add(t->u, sizeof(double) * L * Nx);
-    const size_t iV = add(t->v, sizeof(double) * L * Nx);
+    const bool noise = type_mat == 1;  // only its sensors meet themselves
+    const size_t iRow = add(rowtab.data(), sizeof(int) * rowtab.size());
+    const size_t iCol = add(coltab.data(), sizeof(int) * coltab.size());
+    const size_t iU = add(t->u, positions ? sizeof(double) * L * Nx : 0);
+    const size_t iV = add(t->v, positions ? sizeof(double) * L * Nx : 0);
     const size_t iS = add(t->sspSizeL, sizeof(double) * Nw * L);
     const size_t iLk = add(lk.data(), sizeof(double) * L);
     const size_t iAmp = add(amp.data(), sizeof(double) * L);
     const size_t iCn2 = add(t->cn2, sizeof(double) * L);
     const size_t iSz = add(sspsz.data(), sizeof(double) * Nw);
-    const size_t iNg = add(t->noiseNGS, sizeof(double) * nngs);
-    const size_t iXX = add(t->noiseLGSxx, sizeof(double) * Nx);
-    const size_t iYY = add(t->noiseLGSyy, sizeof(double) * Nx);
-    const size_t iXY = add(t->noiseLGSxy, sizeof(double) * Nx);
-    const size_t iX = add(t->X, sizeof(double) * Nx);
-    const size_t iY = add(t->Y, sizeof(double) * Nx);
+    const size_t iNg = add(t->noiseNGS, noise ? sizeof(double) * nngs : 0);
+    const size_t iXX = add(t->noiseLGSxx, noise ? sizeof(double) * Nx : 0);
+    const size_t iYY = add(t->noiseLGSyy, noise ? sizeof(double) * Nx : 0);
+    const size_t iXY = add(t->noiseLGSxy, noise ? sizeof(double) * Nx : 0);
+    const size_t iX = add(t->X, type_mat == 4 ? sizeof(double) * Nx : 0);
+    const size_t iY = add(t->Y, type_mat == 4 ? sizeof(double) * Nx : 0);
     const size_t iRs = add(rsub.data(), sizeof(int2) * rsub.size());
     const size_t iCs = add(csub.data(), sizeof(int2) * csub.size());
     const size_t iNs = add(nsub.data(), sizeof(int) * Nw);
+    const size_t iLat = add(lat.place.data(), sizeof(int) * lat.place.size());
+    const size_t iU0 = add(lat.u0.data(), sizeof(double) * lat.u0.size());
+    const size_t iV0 = add(lat.v0.data(), sizeof(double) * lat.v0.size());
+    const size_t iCls = add(cls.data(), sizeof(int) * cls.size());
+    const size_t iSl = add(slots.data(), sizeof(int) * slots.size());
 
-    std::vector<unsigned char> host(total);
-    for (auto& p : pieces)
-        if (p.src && p.bytes) std::memcpy(host.data() + p.off, p.src, p.bytes);
-    // Tables of the library context are shared by every caller: hold the lock until the kernel
-    // that reads them has run.  A caller-owned buffer (one per serving slot) needs no lock.
+    const dim3 grid((nrows + kRows - 1) / kRows, (ncols + kCols - 1) / kCols);
+    if (grid.y > 65535) {
+        set_error("matcov_tile: too many columns for one launch");
+        return MOAO_ERR_ARG;
+    }
+    MatcovArgs a;
+    if (int rc = structure_table_dev(&a.ftab)) return rc;
+
+    // Tables of the library context are shared by every caller: hold the lock until the kernels
+    // that read them have run.  A caller-owned buffer (one per serving slot) needs no lock.
     std::unique_lock<std::mutex> g;
     if (!tables) {
         g = std::unique_lock<std::mutex>(ctx().mu);
         tables = &ctx().matcov_tables;
     }
-    if (int rc = tables->ensure(total)) return rc;
-    unsigned char* d = tables->as<unsigned char>();
-    // The upload buffer is reused by the next call: order it on the stream and make the host
-    // copy complete before returning (hipMemcpyAsync from pageable memory is staged).
-    MOAO_HIP_TRY(hipMemcpyAsync(d, host.data(), total, hipMemcpyHostToDevice, stream));
+    const size_t W = 2 * (size_t)lat.ext - 1;
+    if (int rc = tables->ensure(total, slots.size() * 3 * W * W * sizeof(double))) return rc;
+    unsigned char* d = tables->dev.as<unsigned char>();
+    // Staged in pinned memory (the copy is one DMA).  Every way out of here waits for the stream, so
+    // the next call may rewrite the tables.
+    struct Drain {
+        hipStream_t s;
+        ~Drain() { (void)hipStreamSynchronize(s); }
+    } drain{stream};
+    for (auto& p : pieces)
+        if (p.src && p.bytes) std::memcpy(tables->host + p.off, p.src, p.bytes);
+    MOAO_HIP_TRY(hipMemcpyAsync(d, tables->host, total, hipMemcpyHostToDevice, stream));
 
-    MatcovArgs a;
-    if (int rc = structure_table_dev(&a.ftab)) return rc;
     a.out = d_data;
     a.lda = lda;
     a.nrows = nrows;
@@ -639,31 +924,49 @@ int matcov_tile_launch(double* d_data, int nrows, int ncols, int xoffset, int yo
     a.nsub = (const int*)P(iNs);
     a.nrsub = (int)rsub.size();
     a.ncsub = (int)csub.size();
+    a.lat = (const int*)P(iLat);
+    a.u0 = (const double*)P(iU0);
+    a.v0 = (const double*)P(iV0);
+    a.cls = (const int*)P(iCls);
+    a.slots = (const int*)P(iSl);
+    a.ptab = (double*)(d + tables->upload);
+    a.Nw = Nw;
+    a.ext = lat.ext;
 
-    dim3 grid((nrows + kRows - 1) / kRows, (ncols + kCols - 1) / kCols);
-    if (grid.y > 65535) {
-        set_error("matcov_tile: too many columns for one launch");
-        return MOAO_ERR_ARG;
-    }
     {
         // work = elements written (bytes = 8 x elements)
         double elems = (double)nrows * ncols;
-        if (type_mat == 1) {
+        if (type_mat == 1 && profiling()) {
             elems = 0;
             for (int c = 0; c < ncols; ++c)
                 elems += std::max(0, std::min(nrows, xoffset + nrows - (yoffset + c)));
         }
         ProfScope ps(kProfMatcov, elems, stream);
+        if (!slots.empty()) {
+            const dim3 tg((unsigned)((W * W + kWaves * 64 - 1) / (kWaves * 64)),
+                          (unsigned)slots.size());
+            hipLaunchKernelGGL(lattice_table, tg, dim3(kWaves * 64), 0, stream, a);
+        }
         if (pairs) {
-            const dim3 pg((a.nrsub + kRows - 1) / kRows, (a.ncsub + kCols - 1) / kCols);
-            hipLaunchKernelGGL(pair_kernel, pg, dim3(kWaves * 64), 0, stream, a);
+            if (!slots.empty()) {
+                // columns per wave: few enough that the launch fills the chip
+                const long rb = (a.nrsub + 63) / 64;
+                int cw = 8;
+                while (cw > 1 && rb * ((a.ncsub + 4 * cw - 1) / (4 * cw)) < 1024) cw /= 2;
+                hipLaunchKernelGGL(lattice_fill,
+                                   dim3((unsigned)rb, (unsigned)((a.ncsub + 4 * cw - 1) / (4 * cw))),
+                                   dim3(256), 0, stream, a, cw);
+            }
+            if (positions || slots.empty()) {
+                const dim3 pg((a.nrsub + kRows - 1) / kRows, (a.ncsub + kCols - 1) / kCols);
+                hipLaunchKernelGGL(pair_kernel, pg, dim3(kWaves * 64), 0, stream, a);
+            }
         } else if (type_mat == 4)
             hipLaunchKernelGGL(truth_kernel, grid, dim3(kWaves * 64), 0, stream, a);
         else
             hipLaunchKernelGGL(meas_kernel, grid, dim3(kWaves * 64), 0, stream, a);
     }
     MOAO_HIP_TRY(hipGetLastError());
-    // The staging buffer must not be rewritten by another call before this kernel ran.
     MOAO_HIP_TRY(hipStreamSynchronize(stream));
     return MOAO_OK;
 }

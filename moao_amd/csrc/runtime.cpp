@@ -46,6 +46,30 @@ void DevBuf::release() {
     bytes = 0;
 }
 
+int MatcovTables::ensure(size_t upload_bytes, size_t table_bytes) {
+    upload = (upload_bytes + 255) & ~size_t(255);
+    if (upload > host_bytes) {
+        if (host) (void)hipHostFree(host);
+        host = nullptr;
+        host_bytes = 0;
+        hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&host), upload);
+        if (e != hipSuccess) {
+            host = nullptr;
+            set_error(std::string("matcov: pinned staging: ") + hipGetErrorString(e));
+            return MOAO_ERR_NOMEM;
+        }
+        host_bytes = upload;
+    }
+    return dev.ensure(upload + table_bytes);
+}
+
+void MatcovTables::release() {
+    if (host) (void)hipHostFree(host);
+    host = nullptr;
+    host_bytes = 0;
+    dev.release();
+}
+
 Context& ctx() { return g_ctx; }
 
 static int init_device(int device) {

@@ -91,7 +91,7 @@ constexpr long kGraphMaxN = 16384;  // FP64 solves up to this order run as captu
 struct Slot {
     hipStream_t stream = nullptr;
     hipStream_t capture = nullptr;       // idle stream the slot records its graphs on
-    DevBuf tables;                       // matcov upload tables (small, kept)
+    MatcovTables tables;                 // matcov upload and covariance tables (kept)
     std::unique_ptr<SolveGraph> graph;   // the graph of this slot's last captured solve
     struct {
         long n = 0, m = 0;

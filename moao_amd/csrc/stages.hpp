@@ -13,7 +13,7 @@ namespace moao {
 // caller's upload buffer for the per-call tables; nullptr = the library context's buffer, used
 // under the context lock.  Returns after the kernel has run (the tables may be reused).
 int matcov_tile_launch(double* d_data, int nrows, int ncols, int xoffset, int yoffset, int lda,
-                       const moao_tomo_view* t, int type_mat, hipStream_t stream, DevBuf* tables);
+                       const moao_tomo_view* t, int type_mat, hipStream_t stream, MatcovTables* tables);
 
 // Bytes of scratch the mixed-precision reconstructor needs for this problem.
 size_t mixed_workspace_bytes(long n, long m, const moao_tomo_view* lowrank, int mode);

@@ -168,3 +168,49 @@ def test_structure_function_range(tmp_path, L0):
         err = np.max(np.abs(g - r)) / np.max(np.abs(r))
         print(f"[matcov-range] L0={L0} {g.shape}: {err:.2e}", flush=True)
         assert err <= 1e-12
+
+
+def _edit(path, field, values):
+    """Replace the values line that follows the field's name in a parameter file."""
+    lines = open(path).read().split("\n")
+    k = lines.index(field)
+    lines[k + 1] = " ".join(repr(v) for v in values)
+    open(path, "w").write("\n".join(lines))
+
+
+@pytest.mark.parametrize("field,value", [(None, 0.0), ("thetaML", 7.0), ("XPup", 0.37),
+                                         ("thetaCam", 5.0)])
+def test_grids_and_free_sensors(tmp_path, field, value):
+    """Sensors on one regular grid read their covariances from tables of the grid's differences,
+    others (here one LGS rotated or shifted in the pupil; LGS against NGS on the layers the cone
+    shrinks) are evaluated pair by pair: Cmm, Ctm and Cmaa against the oracle, and tiles of every
+    size, small ones evaluated without a table, against the whole matrices bit for bit."""
+    from moao_amd import systems
+    spec = systems.SystemSpec(diam=8.0, nssp=12, nlgs=3, nngs=2, nlayer=4, seed=19)
+    s, a = systems.make_system(str(tmp_path), spec)
+    if field:
+        _edit(s, field, [0.0, value, 0.0, 0.0, 0.0, 0.0])
+    t, o = Tomo(s, a[0]), OTomo.from_files(s, a[0])
+    t.set_target(0)
+    o.set_target(0)
+    n, m = t.nmeas(), t.nmeasts()
+    print(f"[matcov-grids] {field} n={n} m={m}", flush=True)
+    C, B = gm.cmm(t), gm.ctm(t)
+    _close(np.tril(C), np.tril(om.cmm(o)))
+    assert np.max(np.abs(B - om.ctm(o))) <= 1e-12 * np.max(np.abs(om.ctt(o)))
+    for nr, nc, xo, yo in [(n, 7, 0, 0), (9, 11, n - 9, 3), (40, 40, n // 2, n // 3),
+                           (130, 70, n - 130, n // 2), (1, 1, n - 1, 0), (250, 333, 411, 290)]:
+        buf = np.full((nr, nc), -1.0, order="F")
+        gm.matcov_tile(buf, nr, nc, xo, yo, nr, t, gm.CMM)
+        low = np.arange(xo, xo + nr)[:, None] >= np.arange(yo, yo + nc)[None, :]
+        assert np.array_equal(buf[low], C[xo:xo + nr, yo:yo + nc][low]), (nr, nc, xo, yo)
+        assert np.all(buf[~low] == -1.0)
+        nr = min(nr, m)
+        xo = min(xo, m - nr)
+        buf = np.empty((nr, nc), order="F")
+        gm.matcov_tile(buf, nr, nc, xo, yo, nr, t, gm.CTM)
+        assert np.array_equal(buf, B[xo:xo + nr, yo:yo + nc]), ("Ctm", nr, nc, xo, yo)
+    g, r = np.empty((n, m), order="F"), np.empty((n, m), order="F")
+    gm.matcov_tile(g, n, m, 0, 0, n, t, gm.CMAA)
+    om.matcov_tile(r, n, m, 0, 0, n, o, 2)
+    assert np.max(np.abs(g - r)) <= 1e-12 * np.max(np.abs(om.ctt(o)))
