@@ -67,19 +67,19 @@ __constant__ double cGma[11] = MOAO_VK_GMA;
 
 // Table of the normalised structure function f(t), t = q^2, q = 2 pi r / L0 (the function the two
 // branches below define): kSub intervals per octave of t from 2^kLo up to 2^kHi, a polynomial of
-// degree 7 each, then one constant (f is kK2 to the last bit past q = 45).  The interval that holds
+// degree 5 each, then one constant (f is kK2 to the last bit past q = 45).  The interval that holds
 // the branches' border q = 3 pi / 2 is there twice, with the series and with the asymptote.
-constexpr int kSub = 32, kSubBits = 5, kLo = -16, kHi = 11;
-constexpr int kCoef = 8;
+// An evaluation costs its LDS reads (16 bytes a lane each): 6 coefficients at 1/64 octave, three
+// reads, against 8 at 1/32 octave, four reads; two workgroups' tables fit a CU's LDS.
+constexpr int kSub = 64, kSubBits = 6, kLo = -10, kHi = 11;
+constexpr int kCoef = 6;
 constexpr int kTabN = (kHi - kLo) * kSub + 2;
 constexpr double kTBorder = kXlim * kXlim;
 // Arguments below the table and those within rounding of the border take the direct formulas.
 constexpr double kTMin = 1.0 / (1 << -kLo), kTBand = 1e-9;
 
 constexpr int kRows = 64;       // rows per workgroup (one wave tall)
-constexpr int kColsPerWave = 4; // columns per wave
-constexpr int kWaves = 8;       // waves per workgroup
-constexpr int kCols = kColsPerWave * kWaves;
+constexpr int kWaves = 8;       // waves per workgroup; each takes MatcovArgs::cw columns
 
 constexpr int kLattice = -1, kFree = -2;  // MatcovArgs::cls without a table
 
@@ -88,6 +88,7 @@ struct MatcovArgs {
     long lda;
     int nrows, ncols, xoffset, yoffset;
     int Nlayer, nlgs, Nx, type_mat;
+    int cw;                 // columns per wave
     double lgs_cst;
     const int* rowtab;      // packed (pos << 9) | (wfs << 1) | xy
     const int* coltab;
@@ -158,7 +159,7 @@ __device__ __forceinline__ double vk_dphi(double x, double y, double lk, double 
 }
 
 // The same function from the table (in LDS): t's exponent and top mantissa bits give the interval,
-// its other bits the place in it (exact).  About 20 VALU instructions and four 16-byte LDS reads
+// its other bits the place in it (exact).  About 20 VALU instructions and three 16-byte LDS reads
 // where sqrt, cube root, both branches and exp take about 230.
 __device__ __forceinline__ double vk_table(const double* tab, double x, double y, double lk,
                                            double amp) {
@@ -246,36 +247,44 @@ __device__ __forceinline__ void separation(const MatcovArgs& a, bool lattice, in
 // grid with the same size on every layer: every LGS pair of one altitude, every NGS pair).  All
 // subaperture pairs of one lattice difference have the same xx, yy and xy (= yx) covariance, and
 // there are (2*ext - 1)^2 differences against Nsubap^2 pairs (79^2 against 1168^2 at 40 x 40): one
-// lane per difference evaluates it, lattice_fill and meas_kernel read it.
+// lane per difference and layer evaluates it, lattice_fill and meas_kernel read it.  A
+// workgroup takes 64 differences, its waves the layers in turn (the chain of layers one lane would
+// walk was most of the time); the terms meet in LDS and are added in layer order, as an element
+// on its own adds them.
 __global__ void __launch_bounds__(kWaves * 64) lattice_table(MatcovArgs a) {
     __shared__ __attribute__((aligned(16))) double tab[kTabN * kCoef];
+    __shared__ double term[kWaves][3][64];
     load_table(a.ftab, tab);
-    const int W = 2 * a.ext - 1, e = blockIdx.x * (kWaves * 64) + threadIdx.x;
-    if (e >= W * W) return;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int W = 2 * a.ext - 1, e = blockIdx.x * 64 + lane, WW = W * W;
     const int pr = a.slots[blockIdx.y], m = pr >> 8, n = pr & 0xff;
     const int dx = e % W - (a.ext - 1), dy = e / W - (a.ext - 1);
     const double kk = kLambda2 / (a.sspsz[m] * a.sspsz[n]);
-    double cxx = 0.0, cxy = 0.0, cyy = 0.0;
-    for (int l = 0; l < a.Nlayer; ++l) {
-        const double sz = a.sspL[m * a.Nlayer + l];
-        if (!(sz > 0)) continue;
-        double du, dv;
-        lattice_separation(a, m, n, dx, dy, l, sz, du, dv);
-        const double s1 = sz * 0.5, ad = s1 + s1, bc = -ad, lk = a.lk[l], amp = a.amp[l];
-        auto D = [&](double x, double y) { return vk_table(tab, x, y, lk, amp); };
-        const double d0 = D(du, dv);
-        const double sxx = -d0 + D(du + ad, dv) + D(du + bc, dv) - d0;
-        const double syy = -d0 + D(du, dv + ad) + D(du, dv + bc) - d0;
-        const double sxy = -D(du + s1, dv - s1) + D(du + s1, dv + s1) + D(du - s1, dv - s1) -
-                           D(du - s1, dv + s1);
-        cxx += 0.5 * sxx * kk * a.cn2[l];
-        cyy += 0.5 * syy * kk * a.cn2[l];
-        cxy += 0.5 * sxy * kk * a.cn2[l];
+    double sum = 0.0;  // waves 0, 1, 2: xx, yy, xy
+    for (int l0 = 0; l0 < a.Nlayer; l0 += kWaves) {
+        const int l = l0 + wave;
+        const double sz = l < a.Nlayer ? a.sspL[m * a.Nlayer + l] : 0.0;
+        if (sz > 0) {
+            double du, dv;
+            lattice_separation(a, m, n, dx, dy, l, sz, du, dv);
+            const double s1 = sz * 0.5, ad = s1 + s1, bc = -ad, lk = a.lk[l], amp = a.amp[l];
+            auto D = [&](double x, double y) { return vk_table(tab, x, y, lk, amp); };
+            const double d0 = D(du, dv);
+            const double sxx = -d0 + D(du + ad, dv) + D(du + bc, dv) - d0;
+            const double syy = -d0 + D(du, dv + ad) + D(du, dv + bc) - d0;
+            const double sxy = -D(du + s1, dv - s1) + D(du + s1, dv + s1) + D(du - s1, dv - s1) -
+                               D(du - s1, dv + s1);
+            term[wave][0][lane] = 0.5 * sxx * kk * a.cn2[l];
+            term[wave][1][lane] = 0.5 * syy * kk * a.cn2[l];
+            term[wave][2][lane] = 0.5 * sxy * kk * a.cn2[l];
+        }
+        __syncthreads();
+        if (wave < 3)
+            for (int k = 0; k < kWaves && l0 + k < a.Nlayer; ++k)
+                if (a.sspL[m * a.Nlayer + l0 + k] > 0) sum += term[k][wave][lane];
+        __syncthreads();
     }
-    double* o = a.ptab + (long)blockIdx.y * 3 * W * W + e;
-    o[0] = cxx;
-    o[W * W] = cyy;
-    o[2 * W * W] = cxy;
+    if (wave < 3 && e < WW) a.ptab[((long)blockIdx.y * 3 + wave) * WW + e] = sum;
 }
 
 // Whole Cmm or Ctm: the pairs that have a table.  Bound by its stores (8 B an element; the tables
@@ -342,7 +351,7 @@ __global__ void __launch_bounds__(kWaves * 64) meas_kernel(MatcovArgs a) {
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int lx = blockIdx.x * kRows + lane;
-    const int ly0 = blockIdx.y * kCols + wave * kColsPerWave;
+    const int kCols = kWaves * a.cw, ly0 = blockIdx.y * kCols + wave * a.cw;
     if (a.type_mat == 1) {
         // whole workgroup above the diagonal: nothing to write
         const int last_row = a.xoffset + min(a.nrows - 1, (int)blockIdx.x * kRows + kRows - 1);
@@ -358,7 +367,7 @@ __global__ void __launch_bounds__(kWaves * 64) meas_kernel(MatcovArgs a) {
     const int ri = a.rowtab[lx];
     const int m = (ri >> 1) & 0xff, xi = ri & 1, p1 = ri >> 9;
     const int gx = lx + a.xoffset;
-    for (int c = 0; c < kColsPerWave; ++c) {
+    for (int c = 0; c < a.cw; ++c) {
         const int ly = ly0 + c;
         if (ly >= a.ncols) break;
         if (a.type_mat == 1 && ly + a.yoffset > gx) continue;
@@ -414,7 +423,7 @@ __global__ void __launch_bounds__(kWaves * 64) pair_kernel(MatcovArgs a) {
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int rs = blockIdx.x * kRows + lane;
-    const int cs0 = blockIdx.y * kCols + wave * kColsPerWave;
+    const int kCols = kWaves * a.cw, cs0 = blockIdx.y * kCols + wave * a.cw;
     if (a.type_mat == 1) {
         // no pair of this workgroup has a row (its y slope's, the largest) at or below a column
         const int2 last = a.rsub[min((int)blockIdx.x * kRows + kRows, a.nrsub) - 1];
@@ -435,7 +444,7 @@ __global__ void __launch_bounds__(kWaves * 64) pair_kernel(MatcovArgs a) {
     const int2 re = a.rsub[rs];
     const int m = (re.x >> 1) & 0xff, p1 = re.x >> 9;
     const int xr = re.y, yr = re.y + a.nsub[m];
-    for (int c = 0; c < kColsPerWave; ++c) {
+    for (int c = 0; c < a.cw; ++c) {
         const int cs = cs0 + c;
         if (cs >= a.ncsub) break;
         const int2 ce = a.csub[cs];
@@ -529,7 +538,7 @@ __global__ void __launch_bounds__(kWaves * 64) truth_kernel(MatcovArgs a) {
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int lx = blockIdx.x * kRows + lane;
-    const int ly0 = blockIdx.y * kCols + wave * kColsPerWave;
+    const int kCols = kWaves * a.cw, ly0 = blockIdx.y * kCols + wave * a.cw;
     __shared__ __attribute__((aligned(16))) double tab[kTabN * kCoef];
     load_table(a.ftab, tab);
     if (lx >= a.nrows) return;
@@ -540,7 +549,7 @@ __global__ void __launch_bounds__(kWaves * 64) truth_kernel(MatcovArgs a) {
     const double ss = a.sspsz[0];  // diam / Nssp of the truth sensor (set by the host)
     const double kk = kLambda2 / (ss * ss);
     const double s = ss * 0.5;
-    for (int c = 0; c < kColsPerWave; ++c) {
+    for (int c = 0; c < a.cw; ++c) {
         const int ly = ly0 + c;
         if (ly >= a.ncols) break;
         const int gy = ly + a.yoffset;
@@ -577,7 +586,7 @@ inline int pack_truth(long g, const moao_tomo_view* t, const std::vector<long>& 
     return (int)(((off[w] + i) << 9) | (w << 1) | xy);
 }
 
-// Coefficients of the table of f: interpolation at the eight Chebyshev points of an interval, in
+// Coefficients of the table of f: interpolation at the kCoef Chebyshev points of an interval, in
 // extended precision, as a polynomial in z = mantissa - (1 + 1/(2 kSub)) of the interval's start.
 std::vector<double> structure_table() {
     auto series = [](long double t) {
@@ -619,7 +628,7 @@ std::vector<double> structure_table() {
     return tab;
 }
 
-// The table on the device, made on the first use and kept for the life of the process (55 KiB).
+// The table on the device, made on the first use and kept for the life of the process (63 KiB).
 int structure_table_dev(const double** out) {
     static std::mutex mu;
     static double* dev = nullptr;
@@ -862,12 +871,20 @@ int matcov_tile_launch(double* d_data, int nrows, int ncols, int xoffset, int yo
     const size_t iCls = add(cls.data(), sizeof(int) * cls.size());
     const size_t iSl = add(slots.data(), sizeof(int) * slots.size());
 
-    const dim3 grid((nrows + kRows - 1) / kRows, (ncols + kCols - 1) / kCols);
+    MatcovArgs a;
+    // Columns per wave of the evaluating kernels: as many as leave two workgroups per CU, at
+    // most 8 (a workgroup's first work is its copy of the structure function's table).
+    const long rblocks = pairs ? (rsub.size() + kRows - 1) / kRows : (nrows + kRows - 1) / kRows;
+    const long ccount = pairs ? (long)csub.size() : ncols;
+    auto cblocks = [&](int cw) { return (ccount + kWaves * cw - 1) / (kWaves * cw); };
+    int cw = 8;
+    while (cw > 1 && rblocks * cblocks(cw) < 512) cw /= 2;
+    a.cw = cw;
+    const dim3 grid((unsigned)rblocks, (unsigned)cblocks(cw));
     if (grid.y > 65535) {
         set_error("matcov_tile: too many columns for one launch");
         return MOAO_ERR_ARG;
     }
-    MatcovArgs a;
     if (int rc = structure_table_dev(&a.ftab)) return rc;
 
     // Tables of the library context are shared by every caller: hold the lock until the kernels
@@ -943,8 +960,7 @@ int matcov_tile_launch(double* d_data, int nrows, int ncols, int xoffset, int yo
         }
         ProfScope ps(kProfMatcov, elems, stream);
         if (!slots.empty()) {
-            const dim3 tg((unsigned)((W * W + kWaves * 64 - 1) / (kWaves * 64)),
-                          (unsigned)slots.size());
+            const dim3 tg((unsigned)((W * W + 63) / 64), (unsigned)slots.size());
             hipLaunchKernelGGL(lattice_table, tg, dim3(kWaves * 64), 0, stream, a);
         }
         if (pairs) {
@@ -958,8 +974,7 @@ int matcov_tile_launch(double* d_data, int nrows, int ncols, int xoffset, int yo
                                    dim3(256), 0, stream, a, cw);
             }
             if (positions || slots.empty()) {
-                const dim3 pg((a.nrsub + kRows - 1) / kRows, (a.ncsub + kCols - 1) / kCols);
-                hipLaunchKernelGGL(pair_kernel, pg, dim3(kWaves * 64), 0, stream, a);
+                hipLaunchKernelGGL(pair_kernel, grid, dim3(kWaves * 64), 0, stream, a);
             }
         } else if (type_mat == 4)
             hipLaunchKernelGGL(truth_kernel, grid, dim3(kWaves * 64), 0, stream, a);
