@@ -161,29 +161,51 @@ __device__ __forceinline__ double vk_dphi(double x, double y, double lk, double 
 // The same function from the table (in LDS): t's exponent and top mantissa bits give the interval,
 // its other bits the place in it (exact).  About 20 VALU instructions and three 16-byte LDS reads
 // where sqrt, cube root, both branches and exp take about 230.
-__device__ __forceinline__ double vk_table(const double* tab, double x, double y, double lk,
-                                           double amp) {
-    const double r2 = fma(x, x, y * y);
-    const double t = r2 * (lk * lk);
-    if (__builtin_expect(!(t >= kTMin) || fabs(t - kTBorder) < kTBand, 0))
-        return vk_dphi(x, y, lk, amp);
-    const unsigned hi = (unsigned)__double2hiint(t);
-    int k = (int)(hi >> (20 - kSubBits)) - ((1023 + kLo) << kSubBits);
-    k = min(k + (t > kTBorder ? 1 : 0), kTabN - 1);
-    const double w = __hiloint2double((int)((hi & ((1u << (20 - kSubBits)) - 1)) | 0x3ff00000u),
-                                      __double2loint(t));
-    const double z = w - (1.0 + 0.5 / kSub);
-    // coefficients 2n, 2n + 1 of interval k at double2 n * kTabN + k: lanes in different intervals
-    // read neighbouring 16-byte pieces, not one bank group 64 bytes apart
-    const double2* c = (const double2*)tab + k;
-    double f = 0.0;
+//
+// N of them at a time: without a branch between them their LDS reads and products overlap (one by
+// one, each waited for its own reads).  The direct formulas stay out of line, so the kernels'
+// code is short of the instruction cache.
+__device__ __noinline__ double vk_direct(double x, double y, double lk, double amp) {
+    return vk_dphi(x, y, lk, amp);
+}
+
+template <int N>
+__device__ __forceinline__ void vk_table(const double* tab, const double (&x)[N],
+                                         const double (&y)[N], double lk, double amp,
+                                         double (&f)[N]) {
+    bool direct[N], any = false;
+    double t[N];
 #pragma unroll
-    for (int n = kCoef / 2 - 1; n >= 0; --n) {
-        const double2 p = c[n * kTabN];
-        f = n == kCoef / 2 - 1 ? p.y : fma(f, z, p.y);
-        f = fma(f, z, p.x);
+    for (int n = 0; n < N; ++n) {
+        t[n] = fma(x[n], x[n], y[n] * y[n]) * (lk * lk);
+        direct[n] = !(t[n] >= kTMin) || fabs(t[n] - kTBorder) < kTBand;
+        any = any || direct[n];
     }
-    return f * amp;
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+        const unsigned hi = (unsigned)__double2hiint(t[n]);
+        int k = (int)(hi >> (20 - kSubBits)) - ((1023 + kLo) << kSubBits);
+        k = max(min(k + (t[n] > kTBorder ? 1 : 0), kTabN - 1), 0);
+        const double w = __hiloint2double((int)((hi & ((1u << (20 - kSubBits)) - 1)) | 0x3ff00000u),
+                                          __double2loint(t[n]));
+        const double z = w - (1.0 + 0.5 / kSub);
+        // coefficients 2c, 2c + 1 of interval k at double2 c * kTabN + k: lanes in different
+        // intervals read neighbouring 16-byte pieces, not one bank group apart
+        const double2* c = (const double2*)tab + k;
+        double v = 0.0;
+#pragma unroll
+        for (int q = kCoef / 2 - 1; q >= 0; --q) {
+            const double2 p = c[q * kTabN];
+            v = q == kCoef / 2 - 1 ? p.y : fma(v, z, p.y);
+            v = fma(v, z, p.x);
+        }
+        f[n] = v * amp;
+    }
+    if (__builtin_expect(any, 0)) {
+#pragma unroll
+        for (int n = 0; n < N; ++n)
+            if (direct[n]) f[n] = vk_direct(x[n], y[n], lk, amp);
+    }
 }
 
 __device__ __forceinline__ void load_table(const double* src, double* tab) {
@@ -192,32 +214,54 @@ __device__ __forceinline__ void load_table(const double* src, double* tab) {
     __syncthreads();
 }
 
+// -D(p0) + D(p1) + D(p2) - D(p3): the second difference that is a slope covariance.
+__device__ __forceinline__ double second_difference(const double (&f)[4]) {
+    return -f[0] + f[1] + f[2] - f[3];
+}
+
+// kind: 0 xx, 1 xy, 2 yx, 3 yy.  Equal sizes (s1 == s2): the first and last term of xx and yy are
+// D(du, dv) both, with the same bits.
 __device__ __forceinline__ double slope_cov(const double* tab, int kind, double du, double dv,
                                             double s1, double s2, double lk, double amp) {
-    auto D = [&](double x, double y) { return vk_table(tab, x, y, lk, amp); };
     const double ac = s1 - s2, ad = s1 + s2, bc = -ad, bd = -ac;
-    // Equal sizes (s1 == s2, most WFS pairs): ac = +0 and bd = -0, so the first and last
-    // terms share one argument exactly; evaluating it once keeps every operation and its order.
-    switch (kind) {
-        case 0:
-            if (ac == 0.0) {
-                const double d0 = D(du, dv);
-                return -d0 + D(du + ad, dv) + D(du + bc, dv) - d0;
-            }
-            return -D(du + ac, dv) + D(du + ad, dv) + D(du + bc, dv) - D(du + bd, dv);
-        case 3:
-            if (ac == 0.0) {
-                const double d0 = D(du, dv);
-                return -d0 + D(du, dv + ad) + D(du, dv + bc) - d0;
-            }
-            return -D(du, dv + ac) + D(du, dv + ad) + D(du, dv + bc) - D(du, dv + bd);
-        case 1:
-            return -D(du + s1, dv - s2) + D(du + s1, dv + s2) + D(du - s1, dv - s2) -
-                   D(du - s1, dv + s2);
-        default:
-            return -D(du - s2, dv + s1) + D(du + s2, dv + s1) + D(du - s2, dv - s1) -
-                   D(du + s2, dv - s1);
+    double x[4], y[4], f[4];
+    if (kind == 0 || kind == 3) {
+        const double o[4] = {ac, ad, bc, bd};
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+            x[n] = kind == 0 ? du + o[n] : du;
+            y[n] = kind == 0 ? dv : dv + o[n];
+        }
+    } else {
+        const double ox[4] = {s1, s1, -s1, -s1}, oy[4] = {-s2, s2, -s2, s2};
+        const double px[4] = {-s2, s2, -s2, s2}, py[4] = {s1, s1, -s1, -s1};
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+            x[n] = du + (kind == 1 ? ox[n] : px[n]);
+            y[n] = dv + (kind == 1 ? oy[n] : py[n]);
+        }
     }
+    vk_table<4>(tab, x, y, lk, amp, f);
+    return second_difference(f);
+}
+
+// xx and yy, and xy, of sensors of one subaperture size s1 + s1 = ad: nine structure functions.
+__device__ __forceinline__ void slope_cov_equal(const double* tab, double du, double dv, double s1,
+                                                double lk, double amp, bool diag, double& sxx,
+                                                double& syy, double& sxy) {
+    const double ad = s1 + s1, bc = -ad;
+    if (diag) {
+        const double x[5] = {du, du + ad, du + bc, du, du}, y[5] = {dv, dv, dv, dv + ad, dv + bc};
+        double f[5];
+        vk_table<5>(tab, x, y, lk, amp, f);
+        sxx = -f[0] + f[1] + f[2] - f[0];
+        syy = -f[0] + f[3] + f[4] - f[0];
+    }
+    const double x[4] = {du + s1, du + s1, du - s1, du - s1};
+    const double y[4] = {dv - s1, dv + s1, dv - s1, dv + s1};
+    double f[4];
+    vk_table<4>(tab, x, y, lk, amp, f);
+    sxy = second_difference(f);
 }
 
 // Separation of subapertures p1 (sensor m) and p2 (sensor n) on layer l.  On a common lattice it
@@ -267,13 +311,8 @@ __global__ void __launch_bounds__(kWaves * 64) lattice_table(MatcovArgs a) {
         if (sz > 0) {
             double du, dv;
             lattice_separation(a, m, n, dx, dy, l, sz, du, dv);
-            const double s1 = sz * 0.5, ad = s1 + s1, bc = -ad, lk = a.lk[l], amp = a.amp[l];
-            auto D = [&](double x, double y) { return vk_table(tab, x, y, lk, amp); };
-            const double d0 = D(du, dv);
-            const double sxx = -d0 + D(du + ad, dv) + D(du + bc, dv) - d0;
-            const double syy = -d0 + D(du, dv + ad) + D(du, dv + bc) - d0;
-            const double sxy = -D(du + s1, dv - s1) + D(du + s1, dv + s1) + D(du - s1, dv - s1) -
-                               D(du - s1, dv + s1);
+            double sxx = 0.0, syy = 0.0, sxy = 0.0;
+            slope_cov_equal(tab, du, dv, sz * 0.5, a.lk[l], a.amp[l], true, sxx, syy, sxy);
             term[wave][0][lane] = 0.5 * sxx * kk * a.cn2[l];
             term[wave][1][lane] = 0.5 * syy * kk * a.cn2[l];
             term[wave][2][lane] = 0.5 * sxy * kk * a.cn2[l];
@@ -469,40 +508,17 @@ __global__ void __launch_bounds__(kWaves * 64) pair_kernel(MatcovArgs a) {
                 separation(a, cls == kLattice, m, n, p1, p2, l, sml, du, dv);
                 const double s1 = sml * 0.5, s2 = snl * 0.5;
                 const double lk = a.lk[l], amp = a.amp[l];
-                const double ac = s1 - s2, ad = s1 + s2, bc = -ad, bd = -ac;
-                auto D = [&](double x, double y) { return vk_table(tab, x, y, lk, amp); };
-                double sxx, syy, sxy, syx;
-                sxx = syy = sxy = 0.0;
-                if (ac == 0.0) {
-                    if (nxx || nyy) {
-                        const double d0 = D(du, dv);
-                        if (nxx)
-                            sxx = -d0 + D(du + ad, dv) +
-                                  D(du + bc, dv) - d0;
-                        if (nyy)
-                            syy = -d0 + D(du, dv + ad) +
-                                  D(du, dv + bc) - d0;
-                    }
-                    // s1 == s2: the corners of xy and yx are the same four arguments
-                    const double q1 = D(du + s1, dv - s2);
-                    const double q2 = D(du + s1, dv + s2);
-                    const double q3 = D(du - s1, dv - s2);
-                    const double q4 = D(du - s1, dv + s2);
-                    sxy = -q1 + q2 + q3 - q4;
-                    syx = cls == kLattice ? sxy : -q4 + q2 + q3 - q1;
+                double sxx = 0.0, syy = 0.0, sxy = 0.0, syx;
+                if (s1 == s2) {
+                    slope_cov_equal(tab, du, dv, s1, lk, amp, nxx || nyy, sxx, syy, sxy);
+                    // the corners of yx are those of xy, added in another order (on a common
+                    // lattice yx is xy, as in the tables): its own element's expression
+                    syx = cls == kLattice ? sxy : slope_cov(tab, 2, du, dv, s1, s2, lk, amp);
                 } else {
-                    if (nxx)
-                        sxx = -D(du + ac, dv) + D(du + ad, dv) +
-                              D(du + bc, dv) - D(du + bd, dv);
-                    if (nyy)
-                        syy = -D(du, dv + ac) + D(du, dv + ad) +
-                              D(du, dv + bc) - D(du, dv + bd);
-                    if (nxy)
-                        sxy = -D(du + s1, dv - s2) +
-                              D(du + s1, dv + s2) +
-                              D(du - s1, dv - s2) - D(du - s1, dv + s2);
-                    syx = -D(du - s2, dv + s1) + D(du + s2, dv + s1) +
-                          D(du - s2, dv - s1) - D(du + s2, dv - s1);
+                    if (nxx) sxx = slope_cov(tab, 0, du, dv, s1, s2, lk, amp);
+                    if (nyy) syy = slope_cov(tab, 3, du, dv, s1, s2, lk, amp);
+                    if (nxy) sxy = slope_cov(tab, 1, du, dv, s1, s2, lk, amp);
+                    syx = slope_cov(tab, 2, du, dv, s1, s2, lk, amp);
                 }
                 cxx += 0.5 * sxx * kk * a.cn2[l];
                 cxy += 0.5 * sxy * kk * a.cn2[l];
