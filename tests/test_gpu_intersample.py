@@ -207,3 +207,66 @@ def test_elt_psf_2048_eight_directions():
         assert 0.1 < s_ref < 0.7
         assert err <= 2e-5
         assert abs(s_gpu - s_ref) <= 1e-5
+
+
+@pytest.mark.parametrize("prec,tol", [(1, 1e-11), (0, 2e-5)])
+@pytest.mark.parametrize("N,nssp,batch", [(32, 3, 1), (64, 5, 3), (128, 30, 2), (256, 12, 4),
+                                          (512, 21, 6), (1024, 40, 3), (2048, 9, 1), (4096, 17, 3)])
+def test_every_grid_size(prec, tol, N, nssp, batch):
+    """Every transform length (its own radices, values per lane and rows per workgroup), with
+    batches that leave directions or a half pair unused; weights that are not even and the map
+    at strides from 2 to 152.  Tolerances as above: only the order of the sums differs."""
+    print(f"[psf] prec={prec} N={N} nssp={nssp} batch={batch}", flush=True)
+    dm, idx, a2f, otf, _ = _inputs(nssp, N, 8.0, 1.0)
+    rng = np.random.default_rng(N)
+    a2f = np.ascontiguousarray(a2f * (1 + 0.3 * rng.random(N * N)))
+    otf = np.ascontiguousarray(otf * (1 + 0.3 * rng.random(N * N)))
+    np_ = dm.ndiam
+    dact = N // (3 * (np_ - 1)) + 1
+    unit = 2 * (2 * 3.14159 / 1.65e-6) ** 2 / (float(N) * N * dact * dact) * a2f.sum()
+    cvvs = []
+    for b in range(batch):  # not symmetric; phase variance of about 1 rad^2
+        G = rng.standard_normal((dm.nact, dm.nact))
+        cvvs.append(((G @ G.T / dm.nact + 0.05 * G) * (0.3 + 0.2 * b) / unit).flatten())
+    h = _create(idx, np_, N, a2f, otf, prec)
+    dC = DeviceArray.from_host(np.concatenate(cvvs))
+    dP = DeviceArray((batch * N * N,))
+    check(lib().moao_hip_intersample_process_dev(h, ctypes.c_void_p(dC.ptr), batch,
+                                                 ctypes.c_void_p(dP.ptr), None), "process_dev")
+    out = dP.to_host().reshape(batch, N, N)
+    lib().moao_hip_intersample_destroy(h)
+    for b, c in enumerate(cvvs):
+        ref = oi.process(c, idx, a2f, otf, N, np_)
+        err = np.max(np.abs(out[b] - ref)) / np.max(np.abs(ref))
+        print(f"    direction {b}: err={err:.2e}", flush=True)
+        assert err <= tol
+
+
+@pytest.mark.parametrize("order", ["reversed", "transposed", "both", "shuffled", "few"])
+def test_index_orders(order):
+    """The index may list the pairs in any order: the other actuator first (map bins descend
+    along Cvv), actuators by columns (bins a map row apart), at random, or a few pairs only (bins
+    without hits)."""
+    print(f"[psf] index order {order}", flush=True)
+    N, nssp = 512, 20
+    dm, idx, a2f, otf, cvv = _inputs(nssp, N, 8.0, 3e-4)
+    np_, ncov = dm.ndiam, 2 * dm.ndiam - 1
+    ti, tj = (idx - 1) // ncov, (idx - 1) % ncov
+    if order in ("reversed", "both"):
+        ti, tj = ncov - 1 - ti, ncov - 1 - tj
+    if order in ("transposed", "both"):
+        ti, tj = tj, ti
+    idx = np.ascontiguousarray(ti * ncov + tj + 1)
+    p = np.arange(idx.size)
+    if order in ("shuffled", "few"):
+        p = np.random.default_rng(4).permutation(p)
+    if order == "few":
+        p = p[:1000]
+    idx, cvv = np.ascontiguousarray(idx[p]), np.ascontiguousarray(cvv[p])
+    ref = oi.process(cvv, idx, a2f, otf, N, np_)
+    h = _create(idx, np_, N, a2f, otf, 1)
+    psf = np.zeros(N * N)
+    check(lib().moao_hip_intersample_process(h, cvv.ctypes.data_as(dp), psf.ctypes.data_as(dp)),
+          "intersample_process")
+    lib().moao_hip_intersample_destroy(h)
+    assert np.max(np.abs(psf.reshape(N, N) - ref)) <= 1e-11 * np.max(np.abs(ref))
