@@ -4,13 +4,13 @@
 //   1 dsyr2k(L,N, -1, Cpm, R, 1, Cpp)       X = Cpm R^T (one GEMM) and Cpp -= X, Cpp -= X^T on
 //                                           the lower triangle (one elementwise kernel); two
 //                                           lower-trapezoid GEMMs when X has no scratch
-//   2 dsymm(R,L, 1, Cmm, R, 0, Cpm)         GEMM with B = Cmm read from its lower triangle
+//   2 dsymm(R,L, 1, Cmm, R, 0, Cpm)         GEMM with B = Cmm written out in full
 //   3-5 dlaset(U) + dlacpy(L) + in-place geadd('T') + dscal(0.5) on the diagonal
 //                                           one kernel: Cee = lower(Cpp) mirrored (the net
 //                                           effect of those four calls)
-//   6 dgemm(N,T, 1, Cpm, R, 1, Cee)         GEMM
-//   7 dsymm(R,L, 1, Cee, Dx, 0, Tmp)        GEMM with B = Cee read from its lower triangle
-//   8 dgemm(N,T, 1, Tmp, Dx, 0, Cvv)        GEMM
+//   6 dgemm(N,T, 1, Cpm, R, 1, Cee)         GEMM; its lower half, mirrored, where that saves tiles
+//   7 dsymm(R,L, 1, Cee, Dx, 0, Tmp)        GEMM with the full B = Cee
+//   8 dgemm(N,T, 1, Tmp, Dx, 0, Cvv)        as step 6
 // so Cee = Ctt - Ctm R^T - R Ctm^T + R Cmm R^T and Cvv = Dx Cee Dx^T, with the reference's side
 // effects on Cpp (lower part = step 1 result) and Cpm (= R Cmm).  Unlike the reference, every
 // leading-dimension argument is honoured (the reference passes nmeasts/nmeas/nact regardless).
@@ -31,12 +31,20 @@
 namespace moao {
 namespace {
 
-// Cee[i, j] = Cpp[max(i,j), min(i,j)]  (laset + lacpy + geadd('T') + scal on the diagonal)
-__global__ void mirror_lower(const double* __restrict__ src, long lds, double* __restrict__ dst,
-                             long ldd, int m) {
+// Orders from which a symmetric product is computed below the diagonal only and mirrored: up to
+// 1,024 the whole product is one round of the chip's workgroups, whose time half of them take too.
+// m = 2,336, n = 18,688, 8 targets: step 6 32 -> 17 ms.
+constexpr int kHalfFrom = 1024;
+
+// dst[i, j] = src[max(i,j), min(i,j)], target blockIdx.z (laset + lacpy + geadd('T') + scal on the
+// diagonal); in place (src = dst) the lower part stands as it is.
+__global__ void mirror_lower(const double* src, long lds, long sstride, double* dst, long ldd,
+                             long dstride, int m) {
     const int i = blockIdx.x * 64 + (threadIdx.x & 63);
     const int j = blockIdx.y * 4 + (threadIdx.x >> 6);
-    if (i >= m || j >= m) return;
+    if (i >= m || j >= m || (src == dst && i >= j)) return;
+    src += blockIdx.z * sstride;
+    dst += blockIdx.z * dstride;
     dst[i + (long)j * ldd] = i >= j ? src[i + (long)j * lds] : src[j + (long)i * lds];
 }
 
@@ -74,19 +82,15 @@ int cee_cvv_batched_dev(long n, long m, long nact, long ngal, const double* Cmm,
     auto Cee_ = [&](long g) { return Cee + g * ldCee * m; };
     auto Cvv_ = [&](long g) { return Cvv + g * ldCvv * nact; };
     auto Tmp_ = [&](long g) { return Tmp + g * ldTmp * m; };
-    // Stream-ordered scratch for the symmetric operands' diagonal blocks (steps 2 and 7), so
-    // calls on different streams never share it; without it those steps use the
-    // register-staged kernel.
+    // Stream-ordered scratch, so calls on different streams never share it: Cmm in full (step 2;
+    // without it that step runs on the fallback kernel) and step 1's product.
+    SymWork sym;
+    sym_alloc(sym, m * std::min<long>(ngal, kMaxSeg), n, s);
     struct Scratch {
         double* p = nullptr;
         hipStream_t s;
         ~Scratch() { if (p) (void)hipFreeAsync(p, s); }
-    } sd{nullptr, s}, sx{nullptr, s};
-    if (hipMallocAsync(reinterpret_cast<void**>(&sd.p),
-                       sizeof(double) * gemm_symdiag_elems(std::max(n, m)), s) != hipSuccess) {
-        sd.p = nullptr;
-        (void)hipGetLastError();
-    }
+    } sx{nullptr, s};
     // step 1's product X = Cpm R^T for up to kMaxSeg targets (m x m each); without it step 1
     // runs as two lower-trapezoid products
     const long nx = std::min<long>(ngal, kMaxSeg);
@@ -147,52 +151,53 @@ int cee_cvv_batched_dev(long n, long m, long nact, long ngal, const double* Cmm,
             return rc;
     }
     // 2: Cpm = R sym(Cmm), every target against the one Cmm
-    if (sd.p)
-        if (int rc = gemm_symdiag(Cmm, ldCmm, N, sd.p, s)) return rc;
     for (long g0 = 0; g0 < ngal; g0 += kMaxSeg) {
         const int ns = (int)std::min<long>(kMaxSeg, ngal - g0);
         auto g = gemm_args<double>(M, N, N, 1.0, nullptr, ldR, Cmm, ldCmm, 2, 0.0, nullptr, ldCpm);
-        g.symdiag = sd.p;
-        if (int rc = batch(g, g0, ns, [&](long t) { return Seg{R_(t), Cpm_(t), ldR, ldCpm, M}; }))
-            return rc;
+        g.nseg = ns;
+        for (int i = 0; i < ns; ++i) g.seg[i] = Seg{R_(g0 + i), Cpm_(g0 + i), ldR, ldCpm, M};
+        if (int rc = gemm_sym(g, sym, s)) return rc;
     }
+    // The lower part of k x k matrices (ld, target stride) onto the upper one
+    auto mirror = [&](const double* src, long lds, long ss, double* dst, long ldd, long ds, int k,
+                      int ns) {
+        ProfScope ps(kProfOther, 16.0 * k * k * ns, s);
+        hipLaunchKernelGGL(mirror_lower, dim3((k + 63) / 64, (k + 3) / 4, ns), dim3(256), 0, s, src,
+                           lds, ss, dst, ldd, ds, k);
+        return hipGetLastError();
+    };
     for (long g0 = 0; g0 < ngal; g0 += kMaxSeg) {
         const int ns = (int)std::min<long>(kMaxSeg, ngal - g0);
         // 3-5: Cee = lower(Cpp) mirrored
-        {
-            ProfScope ps(kProfOther, 16.0 * m * m * ns, s);
-            dim3 grid((M + 63) / 64, (M + 3) / 4);
-            for (int i = 0; i < ns; ++i)
-                hipLaunchKernelGGL(mirror_lower, grid, dim3(256), 0, s, Cpp_(g0 + i), ldCpp,
-                                   Cee_(g0 + i), ldCee, M);
-            MOAO_HIP_TRY(hipGetLastError());
-        }
+        MOAO_HIP_TRY(mirror(Cpp_(g0), ldCpp, ldCpp * m, Cee_(g0), ldCee, ldCee * m, M, ns));
         // 6: Cee += Cpm R^T
         auto g = gemm_args<double>(M, M, N, 1.0, nullptr, ldCpm, R_(g0), ldR, 1, 1.0, nullptr,
                                    ldCee);
+        g.tri = g.tri_all = M > kHalfFrom;
         if (int rc = batch(g, g0, ns, [&](long t) {
                 Seg q{Cpm_(t), Cee_(t), ldCpm, ldCee, M};
                 q.B = R_(t);
                 return q;
             }))
             return rc;
-    }
-    if (A == 0) return MOAO_OK;
-    // 7: Tmp = Dx sym(lower(Cee)), one launch per target (each has its own symmetric operand)
-    for (long t = 0; t < ngal; ++t) {
-        auto g = gemm_args<double>(A, M, M, 1.0, Dx, ldDx, Cee_(t), ldCee, 2, 0.0, Tmp_(t), ldTmp);
-        if (sd.p) {
-            if (int rc = gemm_symdiag(Cee_(t), ldCee, M, sd.p, s)) return rc;
-            g.symdiag = sd.p;
-        }
-        if (int rc = gemm_f64(g, s)) return rc;
-    }
-    // 8: Cvv = Tmp Dx^T, every target against the one Dx
-    for (long g0 = 0; g0 < ngal; g0 += kMaxSeg) {
-        const int ns = (int)std::min<long>(kMaxSeg, ngal - g0);
-        auto g = gemm_args<double>(A, A, M, 1.0, nullptr, ldTmp, Dx, ldDx, 1, 0.0, nullptr, ldCvv);
+        // below kHalfFrom too, so that step 7 may take the whole of Cee for its lower triangle
+        MOAO_HIP_TRY(mirror(Cee_(g0), ldCee, ldCee * m, Cee_(g0), ldCee, ldCee * m, M, ns));
+        if (A == 0) continue;
+        // 7: Tmp = Dx Cee
+        g = gemm_args<double>(A, M, M, 1.0, nullptr, ldDx, Cee_(g0), ldCee, 1, 0.0, nullptr, ldTmp);
+        if (int rc = batch(g, g0, ns, [&](long t) {
+                Seg q{Dx, Tmp_(t), ldDx, ldTmp, A};
+                q.B = Cee_(t);
+                return q;
+            }))
+            return rc;
+        // 8: Cvv = Tmp Dx^T, every target against the one Dx
+        g = gemm_args<double>(A, A, M, 1.0, nullptr, ldTmp, Dx, ldDx, 1, 0.0, nullptr, ldCvv);
+        g.tri = g.tri_all = A > kHalfFrom;
         if (int rc = batch(g, g0, ns, [&](long t) { return Seg{Tmp_(t), Cvv_(t), ldTmp, ldCvv, A}; }))
             return rc;
+        if (g.tri)
+            MOAO_HIP_TRY(mirror(Cvv_(g0), ldCvv, ldCvv * nact, Cvv_(g0), ldCvv, ldCvv * nact, A, ns));
     }
     return MOAO_OK;
 }

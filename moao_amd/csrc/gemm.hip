@@ -7,16 +7,17 @@
 // and r = l/16 + 4t for f64.
 //
 // Three kernels; the first and last share that structure:
-//  * gemm_dl_kernel (every launch with op(B) = B or B^T, and symmetric B when the caller
-//    supplies full copies of its diagonal blocks): buffer loads write LDS directly
+//  * gemm_dl_kernel (op(B) = B or B^T; gemm_sym turns most products with a symmetric B into such,
+//    few rows read it in place with full copies of its diagonal blocks): buffer loads write LDS
+//    directly
 //    (buffer_load_dword ... lds), so slices need no register staging; kStages slices are in
 //    flight and each slice costs one vmcnt wait and one plain s_barrier.  The buffer
 //    descriptors' range checks zero-fill what lies past the matrix (the range includes the
 //    scalar offset on gfx950, so every column gets a descriptor of its own).  Measured
-//    16384^3 FP64: 74 TF/s (94% of the MFMA peak).
+//    16384^3 FP64: 75 TF/s (96% of the MFMA peak).
 //  * gemm_direct_kernel (launches too small to fill the chip, direct_rows below): operands from
 //    global memory straight into MFMA registers, no LDS and no barriers.
-//  * gemm_kernel (fallback: symmetric B without diagonal copies, K x N slabs whose byte
+//  * gemm_kernel (fallback: symmetric B without scratch, K x N slabs whose byte
 //    offsets would overflow 32 bits): register-staged, double-buffered LDS, the next slice's
 //    global loads issued before the current slice's MFMAs.
 // A slice launch with fewer than two 128-row tiles per CU uses 64-row tiles (each wave 32x64, up
@@ -417,36 +418,89 @@ __global__ void __launch_bounds__(NT, TM == 128 ? 2 : 4) gemm_dl_kernel(GemmArgs
     const int bn = wn * 64 + (lane & 15);
     const int boffC = bn, boffS = (bn / CPI) * GS + (bn % CPI) * BK;  // panel / slab layouts
     constexpr int BJS = (16 / CPI) * GS;                // slab layout: step per j
-    for (int kt = 0; kt < nk; ++kt) {
-        // this wave's loads of slice kt are done once at most the later slices' are pending
-        if (kt + S - 2 >= nk) wait_vm<0>();
-        else if (isA) wait_vm<(S - 2) * IPWA>();
-        else wait_vm<(S - 2) * IPWB>();
-        bar();
-        if (kt + S - 1 < nk) issue(kt + S - 1);
-        const int cur = kt % S;
-        const bool tail = kt * BK + BK > K;
-        const bool slab = TB == 0 || (TB == 2 && kt * BK >= n0 + BN);
-        const int boff = slab ? boffS : boffC, bj = slab ? BJS : 16, bks = slab ? 1 : LDB;
+    if constexpr (TB == 1 && sizeof(T) == 8) {
+        // FP64 op(B) = B^T: the slice that K ends in is apart, so that no branch stands between a
+        // slice's reads and its MFMAs and the compiler starts the second half's reads before the
+        // first half's MFMAs; and waves with rows or columns outside the matrix (or wholly above
+        // the diagonal) leave out their MFMAs, which gives the matrix core to the CU's other
+        // workgroup.  16384^3: 73.5 -> 75.0 TF/s; 9344 x 2336 x 18688: 60.6 -> 64.2.  The other forms
+        // lose by either (16384^3, FP64 op(B) = B 72.8 -> 71.9, FP32 145 -> 137) and keep one loop.
+        auto slice = [&](int kt, auto tailc, auto nic) __attribute__((always_inline)) {
+            constexpr bool tail = decltype(tailc)::value;
+            constexpr int NI = decltype(nic)::value;  // of the wave's WMB row blocks
+            if (kt + S - 2 >= nk) wait_vm<0>();
+            else if (isA) wait_vm<(S - 2) * IPWA>();
+            else wait_vm<(S - 2) * IPWB>();
+            bar();
+            if (kt + S - 1 < nk) issue(kt + S - 1);
+            if constexpr (NI > 0) {
+                const int cur = kt % S;
 #pragma unroll
-        for (int kk = 0; kk < BK / 4; ++kk) {
-            const int k = kk * 4 + kq;
-            T a[WMB], b[4];
+                for (int kk = 0; kk < BK / 4; ++kk) {
+                    const int k = kk * 4 + kq;
+                    T a[NI], b[4];
 #pragma unroll
-            for (int i = 0; i < WMB; ++i) a[i] = As[cur][k][ar + 16 * i];
+                    for (int i = 0; i < NI; ++i) a[i] = As[cur][k][ar + 16 * i];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) b[j] = Bs[cur][boff + bj * j + bks * k];
-            if (tail) {
-                const bool ok = kt * BK + k < K;
+                    for (int j = 0; j < 4; ++j) b[j] = Bs[cur][bn + 16 * j + LDB * k];
+                    if constexpr (tail) {
+                        const bool ok = kt * BK + k < K;
 #pragma unroll
-                for (int i = 0; i < WMB; ++i) a[i] = ok ? a[i] : T(0);
+                        for (int i = 0; i < NI; ++i) a[i] = ok ? a[i] : T(0);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) b[j] = ok ? b[j] : T(0);
+                        for (int j = 0; j < 4; ++j) b[j] = ok ? b[j] : T(0);
+                    }
+#pragma unroll
+                    for (int i = 0; i < NI; ++i)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) acc[i][j] = Mfma<T>::mac(a[i], b[j], acc[i][j]);
+                }
             }
+        };
+        auto slices = [&](auto nic) __attribute__((always_inline)) {
+            const int kf = K / BK;
+            for (int kt = 0; kt < kf; ++kt) slice(kt, std::false_type{}, nic);
+            if (kf < nk) slice(kf, std::true_type{}, nic);
+        };
+        const int r0 = m0 + wm * 16 * WMB, c0 = n0 + wn * 64;
+        if (r0 >= M || c0 >= N || (tri && r0 + 16 * WMB - 1 + g.tri_off < c0))
+            slices(std::integral_constant<int, 0>{});
+        else if (WMB == 4 && r0 + 32 >= M)
+            slices(std::integral_constant<int, WMB / 2>{});
+        else
+            slices(std::integral_constant<int, WMB>{});
+    } else {
+        for (int kt = 0; kt < nk; ++kt) {
+            // this wave's loads of slice kt are done once at most the later slices' are pending
+            if (kt + S - 2 >= nk) wait_vm<0>();
+            else if (isA) wait_vm<(S - 2) * IPWA>();
+            else wait_vm<(S - 2) * IPWB>();
+            bar();
+            if (kt + S - 1 < nk) issue(kt + S - 1);
+            const int cur = kt % S;
+            const bool tail = kt * BK + BK > K;
+            const bool slab = TB == 0 || (TB == 2 && kt * BK >= n0 + BN);
+            const int boff = slab ? boffS : boffC, bj = slab ? BJS : 16, bks = slab ? 1 : LDB;
 #pragma unroll
-            for (int i = 0; i < WMB; ++i)
+            for (int kk = 0; kk < BK / 4; ++kk) {
+                const int k = kk * 4 + kq;
+                T a[WMB], b[4];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = Mfma<T>::mac(a[i], b[j], acc[i][j]);
+                for (int i = 0; i < WMB; ++i) a[i] = As[cur][k][ar + 16 * i];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) b[j] = Bs[cur][boff + bj * j + bks * k];
+                if (tail) {
+                    const bool ok = kt * BK + k < K;
+#pragma unroll
+                    for (int i = 0; i < WMB; ++i) a[i] = ok ? a[i] : T(0);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) b[j] = ok ? b[j] : T(0);
+                }
+#pragma unroll
+                for (int i = 0; i < WMB; ++i)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) acc[i][j] = Mfma<T>::mac(a[i], b[j], acc[i][j]);
+            }
         }
     }
 
@@ -864,11 +918,48 @@ __global__ void split_planes_kernel(const float* __restrict__ A, long lda, int r
 // out[b][r + 128c] = sym(B)[128b + r][128b + c] from the lower triangle of B.
 template <typename T>
 __global__ void symdiag_kernel(const T* __restrict__ B, long ldb, int K, T* __restrict__ out) {
-    const int idx = blockIdx.x * 256 + threadIdx.x;  // element of the 128 x 128 block
-    const int r = idx % BN, c = idx / BN;
-    const long gr = (long)blockIdx.y * BN + r, gc = (long)blockIdx.y * BN + c;
-    if (gr >= K || gc >= K) return;
-    out[(long)blockIdx.y * BN * BN + idx] = r >= c ? B[gr + gc * ldb] : B[gc + gr * ldb];
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    const int r = i % BN, c = i / BN;
+    const int row = blockIdx.y * BN + r, col = blockIdx.y * BN + c;
+    if (row >= K || col >= K) return;
+    const int hi = max(row, col), lo = min(row, col);
+    out[(long)blockIdx.y * BN * BN + i] = B[hi + (long)lo * ldb];
+}
+
+// out(c, k) = sym(B)(c0 + c, k), c < P, k < K, at out[c + k P]: rows c0 .. c0 + P - 1 of a symmetric
+// matrix of which the lower triangle is stored (c0 and, unless it ends the matrix, P multiples of
+// 64).  One workgroup per 64 x 64 tile of the triangle (blockIdx.x <= blockIdx.y), read once and
+// written as it is and, through LDS, transposed.  Bound by memory, 12 bytes per element.
+__global__ __launch_bounds__(256) void expand_sym_kernel(const double* __restrict__ B, long ldb,
+                                                         int K, int c0, int P,
+                                                         double* __restrict__ out) {
+    __shared__ double t[64][65];
+    const int i0 = blockIdx.y * 64, j0 = blockIdx.x * 64;
+    const bool keep = i0 >= c0 && i0 < c0 + P, turn = j0 >= c0 && j0 < c0 + P;
+    if (j0 > i0 || !(keep || turn)) return;
+    const int x = threadIdx.x & 63, y = threadIdx.x >> 6;
+    double v[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int i = min(i0 + x, K - 1), j = min(j0 + 4 * r + y, K - 1);
+        v[r] = B[max(i, j) + (long)min(i, j) * ldb];
+    }
+    if (keep && i0 + x < K) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int j = j0 + 4 * r + y;
+            if (j < K) out[i0 + x - c0 + (long)j * P] = v[r];
+        }
+    }
+    if (!turn || i0 == j0) return;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) t[4 * r + y][x] = v[r];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int i = i0 + 4 * r + y;  // j0 + 64 <= i0 < K: the column tile is whole
+        if (i < K) out[j0 + x - c0 + (long)i * P] = t[x][4 * r + y];
+    }
 }
 
 // Rows per workgroup of the direct kernel for this product, 0 where the slice kernels are the
@@ -983,12 +1074,12 @@ int launch(const GemmArgs<T>& g, hipStream_t stream) {
             return MOAO_OK;
         }
     }
-    if (small) {
+    if (small || (g.transb == 2 && g.symdiag)) {
         grid.x = (maxM + 63) / 64;
-        if (g.transb == 0 && kn_offsets_fit)
-            hipLaunchKernelGGL((gemm_dl_kernel<T, 0, kStages, 64>), grid, dim3(NT), 0, stream, g);
-        else if (g.transb == 2 && g.symdiag && kn_offsets_fit)
+        if (g.transb == 2 && g.symdiag && kn_offsets_fit)
             hipLaunchKernelGGL((gemm_dl_kernel<T, 2, kStages, 64>), grid, dim3(NT), 0, stream, g);
+        else if (g.transb == 0 && kn_offsets_fit)
+            hipLaunchKernelGGL((gemm_dl_kernel<T, 0, kStages, 64>), grid, dim3(NT), 0, stream, g);
         else if (g.transb == 0)
             hipLaunchKernelGGL((gemm_kernel<T, 0, 2>), grid, dim3(NT), 0, stream, g);
         else if (g.transb == 1)
@@ -997,8 +1088,6 @@ int launch(const GemmArgs<T>& g, hipStream_t stream) {
             hipLaunchKernelGGL((gemm_kernel<T, 2, 2>), grid, dim3(NT), 0, stream, g);
     } else if (g.transb == 0 && kn_offsets_fit)
         hipLaunchKernelGGL((gemm_dl_kernel<T, 0, kStages, 128>), grid, dim3(NT), 0, stream, g);
-    else if (g.transb == 2 && g.symdiag && kn_offsets_fit)
-        hipLaunchKernelGGL((gemm_dl_kernel<T, 2, kStages, 128>), grid, dim3(NT), 0, stream, g);
     else if (g.transb == 0)
         hipLaunchKernelGGL((gemm_kernel<T, 0, 4>), grid, dim3(NT), 0, stream, g);
     else if (g.transb == 1)
@@ -1029,14 +1118,56 @@ int split_planes(const float* A, long lda, int rows, int cols, unsigned short* h
     return MOAO_OK;
 }
 
-size_t gemm_symdiag_elems(long K) { return (size_t)((K + BN - 1) / BN) * BN * BN; }
+void sym_alloc(SymWork& w, long rows, long K, hipStream_t s) {
+    // in full where that stays below 4 GB, else as many columns at a time as do; for few rows
+    // the diagonal blocks
+    const long cols = rows < kSymRows ? 0 : std::min<long>(K, (1L << 29) / K / BN * BN);
+    const long elems = cols ? K * cols : (K + BN - 1) / BN * BN * BN;
+    if (hipMallocAsync(reinterpret_cast<void**>(&w.p), sizeof(double) * elems, s) != hipSuccess) {
+        w.p = nullptr;
+        (void)hipGetLastError();
+        return;
+    }
+    w.s = s;
+    w.cols = (int)cols;
+}
 
-int gemm_symdiag(const double* B, long ldb, int K, double* out, hipStream_t stream) {
-    if (K <= 0) return MOAO_OK;
-    ProfScope ps(kProfOther, 0.0, stream);
-    hipLaunchKernelGGL(symdiag_kernel<double>, dim3(BN * BN / 256, (K + BN - 1) / BN), dim3(256),
-                       0, stream, B, ldb, K, out);
-    MOAO_HIP_TRY(hipGetLastError());
+SymWork::~SymWork() {
+    if (p) (void)hipFreeAsync(p, s);
+}
+
+int gemm_sym(const GemmArgs<double>& a, SymWork& w, hipStream_t stream) {
+    const int K = a.K;
+    if (!w.p || K < 1 || a.N != K) return gemm_f64(a, stream);
+    GemmArgs<double> g = a;
+    if (w.cols == 0) {
+        if (!w.held) {
+            ProfScope ps(kProfOther, 0.0, stream);
+            hipLaunchKernelGGL(symdiag_kernel<double>, dim3(BN * BN / 256, (K + BN - 1) / BN),
+                               dim3(256), 0, stream, a.B, a.ldb, K, w.p);
+            MOAO_HIP_TRY(hipGetLastError());
+            w.held = true;
+        }
+        g.symdiag = w.p;
+        return gemm_f64(g, stream);
+    }
+    g.transb = 1;
+    g.B = w.p;
+    for (int c0 = 0; c0 < K; c0 += w.cols) {
+        const int P = std::min(w.cols, K - c0);
+        if (!w.held) {
+            ProfScope ps(kProfOther, 12.0 * K * P, stream);
+            const int n = (K + 63) / 64;
+            hipLaunchKernelGGL(expand_sym_kernel, dim3(n, n), dim3(256), 0, stream, a.B, a.ldb, K,
+                               c0, P, w.p);
+            MOAO_HIP_TRY(hipGetLastError());
+            w.held = P == K;
+        }
+        g.N = P;
+        g.ldb = P;
+        for (int i = 0; i < g.nseg; ++i) g.seg[i].C = a.seg[i].C + (long)c0 * a.seg[i].ldc;
+        if (int rc = gemm_f64(g, stream)) return rc;
+    }
     return MOAO_OK;
 }
 
@@ -1058,21 +1189,9 @@ int moao_hip_dgemm_dev(int transb, int M, int N, int K, double alpha, const doub
     auto a = moao::gemm_args<double>(M, N, K, alpha, A, lda, B, ldb, transb, beta, C, ldc);
     hipStream_t s = moao::pick_stream(stream);
     if (transb != 2 || K == 0) return moao::gemm_f64(a, s);
-    // symmetric B: its diagonal blocks in stream-ordered scratch (register-staged kernel if
-    // that allocation fails)
-    double* sd = nullptr;
-    if (hipMallocAsync(reinterpret_cast<void**>(&sd), sizeof(double) * moao::gemm_symdiag_elems(K),
-                       s) != hipSuccess) {
-        (void)hipGetLastError();
-        return moao::gemm_f64(a, s);
-    }
-    int rc = moao::gemm_symdiag(B, ldb, K, sd, s);
-    if (rc == MOAO_OK) {
-        a.symdiag = sd;
-        rc = moao::gemm_f64(a, s);
-    }
-    (void)hipFreeAsync(sd, s);
-    return rc;
+    moao::SymWork sym;
+    moao::sym_alloc(sym, M, K, s);
+    return moao::gemm_sym(a, sym, s);
 }
 
 int moao_hip_sgemm_dev(int transb, int M, int N, int K, float alpha, const float* A, long lda,

@@ -54,8 +54,8 @@ struct GemmArgs {
     int tri_off;
     int tri_all;  // with tri: every segment restricted, not only segment 0
     T alpha, beta;
-    // transb = 2 only, optional: full symmetric copies of B's 128 x 128 diagonal blocks
-    // (gemm_symdiag); with it the launch runs on the direct-to-LDS kernel.
+    // transb = 2 only, optional: full symmetric copies of B's 128 x 128 diagonal blocks (gemm_sym);
+    // with it the launch runs on the direct-to-LDS kernel.
     const T* symdiag;
     // FP32 only: 2 = run the product on BF16 MFMA from split-BF16 planes of the operands
     // (hi = bf16(a), lo = bf16(a - hi); hi*hi + hi*lo + lo*hi accumulated in FP32; A from
@@ -68,12 +68,26 @@ struct GemmArgs {
     const int* skip_if;
 };
 
-// Elements of the gemm_symdiag copy of a K x K matrix.
-size_t gemm_symdiag_elems(long K);
-// out[b] (128 x 128, leading dimension 128) = the full symmetric diagonal block b of the K x K
-// matrix whose lower triangle B holds; what a transb = 2 launch reads where its K slices cross
-// the diagonal.
-int gemm_symdiag(const double* B, long ldb, int K, double* out, hipStream_t stream);
+// Scratch for products with a symmetric operand.  From kSymRows rows on it holds the matrix written
+// out in full, so that they run on the kernel for op(B) = B^T; with fewer, full copies of its 128 x
+// 128 diagonal blocks, with which a kernel reads the lower triangle in place, columns above the
+// diagonal and rows below it.  K = 18,688, in place -> in full: 256 rows 4.1 -> 5.3 ms, 512 rows 9.8 ->
+// 7.6, 8 x 2,336 rows 213 -> 187.  Stream-ordered, for one matrix and one caller's scope.
+constexpr long kSymRows = 448;
+struct SymWork {
+    double* p = nullptr;
+    hipStream_t s = nullptr;
+    int cols = 0;       // columns written out at a time; 0: diagonal blocks
+    bool held = false;  // the whole matrix, or its blocks, are there
+    SymWork() = default;
+    SymWork(const SymWork&) = delete;
+    SymWork& operator=(const SymWork&) = delete;
+    ~SymWork();
+};
+// Allocates for products of `rows` rows with a K x K matrix; leaves w empty where it cannot.
+void sym_alloc(SymWork& w, long rows, long K, hipStream_t s);
+// The transb = 2 product, through w where it has room, else on the fallback kernel.
+int gemm_sym(const GemmArgs<double>& a, SymWork& w, hipStream_t stream);
 
 // Planes of an FP32 column-major region (rows x cols at A, leading dimension lda):
 // transposed = 1 writes element (r, c) as plane row r, k = c (hi[r * ld + c]); transposed = 0 as

@@ -263,7 +263,6 @@ static size_t mixed_layout(long n, long m, int p, int mode, std::vector<size_t>*
     take(sizeof(int) * n);
     take(sizeof(int) * 4);
     take(sizeof(int) * 2 * q);
-    take(sizeof(double) * gemm_symdiag_elems(n));  // Cmm's symmetric diagonal blocks
     if (mode == MOAO_MIXED_BF16) {
         const long ld = plane_ld(n);
         take(sizeof(unsigned short) * 2 * n * ld);   // L, plane row = row
@@ -304,14 +303,13 @@ int reconstructor_mixed_dev(long n, long m, const double* Cmm, long ldCmm, doubl
               (double*)(b + offs[6]), (double*)(b + offs[7]), (double*)(b + offs[8]),
               (double*)(b + offs[9]), (double*)(b + offs[10]), (double*)(b + offs[11]),
               (int*)(b + offs[12]), (int*)(b + offs[13]), (int*)(b + offs[14])};
-    double* const symd = (double*)(b + offs[15]);
     const int N = (int)n, M = (int)m;
     SplitWs sw{};
     const SplitWs* swp = nullptr;
     if (split) {
         const long ld = plane_ld(n);
-        sw = SplitWs{(unsigned short*)(b + offs[16]), (unsigned short*)(b + offs[17]),
-                     (unsigned short*)(b + offs[18]), ld, n * ld, n * ld, xr * ld};
+        sw = SplitWs{(unsigned short*)(b + offs[15]), (unsigned short*)(b + offs[16]),
+                     (unsigned short*)(b + offs[17]), ld, n * ld, n * ld, xr * ld};
         swp = &sw;
     }
 
@@ -434,8 +432,9 @@ int reconstructor_mixed_dev(long n, long m, const double* Cmm, long ldCmm, doubl
         std::fprintf(stderr, "[mixed] |Z|=%.6e |Z2|=%.6e |R0|=%.6e\n", a, b2, c2);
     }
 
-    // --- 4. refinement (the residual's symmetric operand Cmm feeds the direct-to-LDS GEMM)
-    if (int rc = gemm_symdiag(Cmm, ldCmm, N, symd, s)) return rc;
+    // --- 4. refinement (the residual's symmetric operand Cmm written out in full where there is room)
+    SymWork sym;
+    sym_alloc(sym, m, n, s);
     double rel = 0;
     int it = 0;
     int status = MOAO_OK;
@@ -443,8 +442,7 @@ int reconstructor_mixed_dev(long n, long m, const double* Cmm, long ldCmm, doubl
         MOAO_HIP_TRY(hipMemcpyAsync(w.E, w.Ctm0, sizeof(double) * m * n, hipMemcpyDeviceToDevice,
                                     s));
         auto g = gemm_args<double>(M, N, N, -1.0, Ctm, ldCtm, Cmm, ldCmm, 2, 1.0, w.E, m);
-        g.symdiag = symd;
-        if (int rc = gemm_f64(g, s)) { status = rc; break; }
+        if (int rc = gemm_sym(g, sym, s)) { status = rc; break; }
         double en = 0;
         if (int rc = norm(w.E, m, M, N, &en)) { status = rc; break; }
         rel = ctm_norm > 0 ? en / ctm_norm : en;

@@ -176,3 +176,35 @@ def test_direct_in_place_panel():
             dX = DeviceArray.from_host(A)
             dgemm_dev(transb, M, N, N, 1.0, dX.ptr, M, dB.ptr, N, 0.0, dX.ptr, M)
             assert np.array_equal(dX.to_host(), want), (M, N, transb)
+
+
+@pytest.mark.parametrize("M,N,K", [(3073, 2945, 257), (3103, 3009, 260), (3105, 2943, 8),
+                                   (3136, 2977, 7), (3137, 3041, 264), (3199, 3039, 129)])
+def test_tiles_at_the_edge(M, N, K):
+    """op(B) = B^T launches of 128-row tiles whose last row and column tiles hold 1, 31, 33, 64, 65 or
+    127 rows and columns (waves that leave out their MFMAs) and whose K ends inside a slice.
+    Tolerance: K products of values below 1, each rounded once and added once."""
+    print(f"[gemm] edge tiles {M} x {N} x {K}", flush=True)
+    rng = np.random.default_rng(M)
+    A, B, C = (np.asfortranarray(rng.uniform(-1, 1, s)) for s in ((M, K), (N, K), (M, N)))
+    dA, dB, dC = (DeviceArray.from_host(x) for x in (A, B, C))
+    dgemm_dev(1, M, N, K, 0.5, dA.ptr, M, dB.ptr, N, 1.0, dC.ptr, M)
+    err = np.max(np.abs(dC.to_host() - (0.5 * (A @ B.T) + C)))
+    assert err <= 2 * K * 2.0 ** -52
+
+
+@pytest.mark.parametrize("M", [1, 130, 447, 448, 1000])
+@pytest.mark.parametrize("K", [1, 63, 65, 128, 700])
+def test_symmetric_operand_from_its_lower_triangle(M, K):
+    """The symmetric operand written out in full (448 rows and more) or read in place (fewer); its
+    upper triangle holds NaN, so nothing may be read from there.  Tolerance as above."""
+    print(f"[gemm] symmetric B {M} x {K}", flush=True)
+    rng = np.random.default_rng(M + K)
+    A = np.asfortranarray(rng.uniform(-1, 1, (M, K)))
+    S = rng.uniform(-1, 1, (K, K))
+    S = S + S.T
+    low = np.asfortranarray(np.where(np.tri(K, dtype=bool), S, np.nan))
+    dA, dB, dC = DeviceArray.from_host(A), DeviceArray.from_host(low), \
+        DeviceArray.from_host(np.zeros((M, K), order="F"))
+    dgemm_dev(2, M, K, K, 1.0, dA.ptr, M, dB.ptr, K, 0.0, dC.ptr, M)
+    assert np.max(np.abs(dC.to_host() - A @ S)) <= 2 * K * 2.0 ** -52 * 2
