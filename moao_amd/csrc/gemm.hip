@@ -20,8 +20,7 @@
 //  * gemm_kernel (fallback: symmetric B without scratch, K x N slabs whose byte
 //    offsets would overflow 32 bits): register-staged, double-buffered LDS, the next slice's
 //    global loads issued before the current slice's MFMAs.
-// A slice launch with fewer than two 128-row tiles per CU uses 64-row tiles (each wave 32x64, up
-// to 4 workgroups per CU), which doubles the workgroups that fill the device.
+// Slice launches use 128-row or 64-row tiles (each wave 32x64, up to 4 workgroups per CU): half_tiles.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -978,16 +977,7 @@ __global__ __launch_bounds__(256) void expand_sym_kernel(const double* __restric
 // 1500 x 1500 x 1024 (564) 87 -> 103.  FP32 op(B) = B: 3000 x 1000 x 2048 (752) 184 -> 153, 2336 x
 // 2336 x 2048 (1,387) 247 -> 296.
 template <typename T>
-int direct_rows(const GemmArgs<T>& g, int maxM) {
-    double cells = 0;  // C elements of the launch, trapezoids without their upper part
-    for (int i = 0; i < g.nseg; ++i) {
-        const double M = g.seg[i].M, N = g.N;
-        cells += M * N;
-        if (g.tri && (i == 0 || g.tri_all)) {
-            const double w = std::min(N, M + g.tri_off);
-            cells -= M * (N - w) + w * w / 2;
-        }
-    }
+int direct_rows(const GemmArgs<T>& g, double cells) {
     const double groups = cells / (16 * BN);
     if (groups <= 256) return 16;
     double limit;
@@ -997,6 +987,27 @@ int direct_rows(const GemmArgs<T>& g, int maxM) {
     else
         limit = g.K <= 256 ? 1500 : g.transb == 1 ? 400 : 1000;
     return groups / 2 <= limit ? 32 : 0;
+}
+
+// Whether the slice kernel runs 64-row tiles.  They read op(B) twice as often and reach less on a
+// large product, but a CU carries four and not two of them, which hides a short K's first and last
+// slices, and the launch's end leaves fewer CUs idle: with w 128-row tiles per CU the last of
+// ceil(w) rounds is part empty.  So: few rounds, or a short K; sooner so for op(B) = B, whose loads
+// of half cache lines gain from more waves, and later for FP32, whose 128-row tiles are five to a
+// CU already.  Measured, 128 -> 64 rows, TF/s.  FP64 op(B) = B^T: w 3.2, K 1024 51 -> 61; 4.1, 4096
+// 58 -> 61; 6.9, 4096 70.0 -> 68.3; 16, 256 45 -> 53; 16, 1024 67.7 -> 68.0; 64, 1024 70.1 -> 69.2.  FP64
+// op(B) = B: 3.2, 1024 52 -> 62; 64, 4096 70.4 -> 70.9; 9.4, 16384 67.6 -> 69.3; 16, 16384 72.2 -> 70.2.
+// FP32 op(B) = B^T: 5.1, 1024 105 -> 111; 8.6, 1024 123 -> 118; 4.1, 4096 114 -> 114; 16, 256 76 -> 79.
+// FP32 op(B) = B: 9.4, 1024 117 -> 123; 16, 1024 126 -> 123; 4.1, 4096 111 -> 116; 6.9, 4096 134 -> 128.
+template <typename T>
+bool half_tiles(const GemmArgs<T>& g, double cells) {
+    const double w = cells / (BM * BN * 256.0);
+    if (g.transb == 2 || w < 2) return true;
+    if (sizeof(T) == 8)
+        return g.transb == 0 ? g.K <= 8192 || w < 13
+                             : w < 5 || g.K <= 512 || (g.K <= 2048 && w < 20);
+    return g.transb == 0 ? w < 5 || (g.K <= 2048 && w < 14)
+                         : w < 4 || (g.K <= 2048 && w < 8) || (g.K <= 512 && w < 32);
 }
 
 template <typename T>
@@ -1033,7 +1044,16 @@ int launch(const GemmArgs<T>& g, hipStream_t stream) {
         }
     }
     ProfScope ps(sizeof(T) == 8 ? kProfGemmF64 : kProfGemmF32, work, stream);
-    // 128-row tiles when they fill the device (>= 2 per CU), else 64-row tiles
+    double cells = 0;  // C elements of the launch, trapezoids without their upper part
+    for (int i = 0; i < g.nseg; ++i) {
+        const double M = g.seg[i].M, N = g.N;
+        cells += M * N;
+        if (g.tri && (i == 0 || g.tri_all)) {
+            const double w = std::min(N, M + g.tri_off);
+            cells -= M * (N - w) + w * w / 2;
+        }
+    }
+    // planes and fallback kernels: 128-row tiles when they fill the device (>= 2 per CU)
     const bool small = (long)grid.x * grid.y * grid.z < 2L * 256;
     if constexpr (std::is_same<T, float>::value) {
         if (g.split == 2) {
@@ -1063,7 +1083,7 @@ int launch(const GemmArgs<T>& g, hipStream_t stream) {
     // the K x N slab loads address 128 columns with 32-bit byte offsets
     const bool kn_offsets_fit = (long)BN * g.ldb * (long)sizeof(T) < (1L << 31);
     if (g.transb < 2 && (g.transb == 1 || kn_offsets_fit)) {
-        if (const int rows = direct_rows(g, maxM)) {
+        if (const int rows = direct_rows(g, cells)) {
             grid.x = (maxM + rows - 1) / rows;
             auto k = g.transb == 1 ? (rows == 16 ? gemm_direct_kernel<T, 1, 1, 4>
                                                  : gemm_direct_kernel<T, 1, 2, 3>)
@@ -1074,26 +1094,21 @@ int launch(const GemmArgs<T>& g, hipStream_t stream) {
             return MOAO_OK;
         }
     }
-    if (small || (g.transb == 2 && g.symdiag)) {
-        grid.x = (maxM + 63) / 64;
-        if (g.transb == 2 && g.symdiag && kn_offsets_fit)
-            hipLaunchKernelGGL((gemm_dl_kernel<T, 2, kStages, 64>), grid, dim3(NT), 0, stream, g);
-        else if (g.transb == 0 && kn_offsets_fit)
-            hipLaunchKernelGGL((gemm_dl_kernel<T, 0, kStages, 64>), grid, dim3(NT), 0, stream, g);
-        else if (g.transb == 0)
-            hipLaunchKernelGGL((gemm_kernel<T, 0, 2>), grid, dim3(NT), 0, stream, g);
-        else if (g.transb == 1)
-            hipLaunchKernelGGL((gemm_dl_kernel<T, 1, kStages, 64>), grid, dim3(NT), 0, stream, g);
-        else
-            hipLaunchKernelGGL((gemm_kernel<T, 2, 2>), grid, dim3(NT), 0, stream, g);
-    } else if (g.transb == 0 && kn_offsets_fit)
-        hipLaunchKernelGGL((gemm_dl_kernel<T, 0, kStages, 128>), grid, dim3(NT), 0, stream, g);
-    else if (g.transb == 0)
-        hipLaunchKernelGGL((gemm_kernel<T, 0, 4>), grid, dim3(NT), 0, stream, g);
+    // the direct-to-LDS slice kernel, else the fallback
+    const bool dl = g.transb == 1 || (kn_offsets_fit && (g.transb == 0 || g.symdiag));
+    const bool half = dl ? half_tiles(g, cells) : small;
+    if (half) grid.x = (maxM + 63) / 64;
+    void (*k)(GemmArgs<T>);
+    if (!dl)
+        k = g.transb == 0 ? (half ? gemm_kernel<T, 0, 2> : gemm_kernel<T, 0, 4>)
+                          : (half ? gemm_kernel<T, 2, 2> : gemm_kernel<T, 2, 4>);
+    else if (g.transb == 2)
+        k = gemm_dl_kernel<T, 2, kStages, 64>;
     else if (g.transb == 1)
-        hipLaunchKernelGGL((gemm_dl_kernel<T, 1, kStages, 128>), grid, dim3(NT), 0, stream, g);
+        k = half ? gemm_dl_kernel<T, 1, kStages, 64> : gemm_dl_kernel<T, 1, kStages, 128>;
     else
-        hipLaunchKernelGGL((gemm_kernel<T, 2, 4>), grid, dim3(NT), 0, stream, g);
+        k = half ? gemm_dl_kernel<T, 0, kStages, 64> : gemm_dl_kernel<T, 0, kStages, 128>;
+    hipLaunchKernelGGL(k, grid, dim3(NT), 0, stream, g);
     MOAO_HIP_TRY(hipGetLastError());
     return MOAO_OK;
 }
