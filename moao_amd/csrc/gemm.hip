@@ -556,6 +556,31 @@ __device__ __forceinline__ void lane_rows_transpose(T& a, T& b, T& c, T& d) {
     __builtin_memcpy(&d, v[3], sizeof(T));
 }
 
+// hi and lo planes of four consecutive k of one row, those below N (see Planes).
+__device__ __forceinline__ void write_planes(const float (&v)[4], unsigned short* hi, long ps,
+                                             int k, int N) {
+    typedef unsigned short us4 __attribute__((ext_vector_type(4)));
+    us4 h, l;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        const __bf16 a = (__bf16)v[t];
+        h[t] = __builtin_bit_cast(unsigned short, a);
+        l[t] = __builtin_bit_cast(unsigned short, (__bf16)(v[t] - (float)a));
+    }
+    if (k + 4 <= N) {
+        *(us4*)(hi + k) = h;
+        *(us4*)(hi + ps + k) = l;
+        return;
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+        if (k + t < N) {
+            hi[k + t] = h[t];
+            hi[ps + k + t] = l[t];
+        }
+}
+__device__ __forceinline__ void write_planes(const double (&)[4], unsigned short*, long, int, int) {}
+
 // Direct kernel for launches too small to hide the slice pipeline above: a K = 128 product is
 // 16 slices there, each a barrier and a share of the load latency.  Here no LDS and no barrier
 // stand between the loads and the MFMAs: every wave loads its A and op(B) fragments from global
@@ -709,16 +734,20 @@ __global__ void __launch_bounds__(NT) gemm_direct_kernel(GemmArgs<T> g) {
     for (int i = 0; i < WM; ++i) {
         const int row = m0 + 16 * i + li;
 #pragma unroll
-        for (int j = 0; j < WN; ++j)
+        for (int j = 0; j < WN; ++j) {
+            T v[4];
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
                 const int col = nw + 16 * j + Mfma<T>::row(lane, t);
+                v[t] = alpha * acc[i][j][t];
+                if (beta != T(0)) v[t] += beta * old[i][j][t];
                 if (row >= M || col >= N || (tri && row + g.tri_off < col)) continue;
-                T* c = s.C + row + (long)col * s.ldc;
-                T v = alpha * acc[i][j][t];
-                if (beta != T(0)) v += beta * old[i][j][t];
-                *c = v;
+                s.C[row + (long)col * s.ldc] = v[t];
             }
+            if constexpr (sizeof(T) == 4)  // a lane's 4 columns are 4 consecutive k of a plane row
+                if (s.cp) write_planes(v, s.cp + (long)row * s.cpl.ld, s.cpl.ps,
+                                       nw + 16 * j + 4 * lq, row < M ? N : 0);
+        }
     }
 }
 
@@ -739,11 +768,11 @@ constexpr int KC = 32;  // k per chunk (one 16x16x32 step)
 // as the 16x16x32 MFMA takes its operands: lane l of a fragment read supplies row l % 16 and
 // k = 8 (l / 16) .. + 7, i.e. bytes [16 l, 16 l + 16) of the block, so every fragment is one
 // conflict-free 16-byte LDS read.  The blocks are filled by 16-byte buffer loads straight into
-// LDS (buffer_load_dwordx4 ... lds, one 1 KB block per instruction, no registers), kS2 stages
-// deep.  Products accumulate in FP32 in the MFMA; every kFlush stages the accumulators are
+// LDS (buffer_load_dwordx4 ... lds, one 1 KB block per instruction, no registers), S stages
+// deep: two for 128-row tiles, so that two workgroups share a CU (4864 x 9728 x 4864: 1,258 us with
+// three to five stages and one workgroup, 935 with two).  Products accumulate in FP32 in the MFMA; every kFlush stages the accumulators are
 // added into a second set of FP32 sums and restarted, so no accumulation chain runs longer
 // than 256 k.
-constexpr int kS2 = 3;      // stages of the planes kernel
 constexpr int kFlush = 8;   // stages between flushes of the MFMA accumulators
 
 __device__ __forceinline__ void dl_load16(__amdgpu_buffer_rsrc_t r, void* lds, int voff) {
@@ -752,13 +781,13 @@ __device__ __forceinline__ void dl_load16(__amdgpu_buffer_rsrc_t r, void* lds, i
     __builtin_amdgcn_raw_ptr_buffer_load_lds(r, l, 16, voff, 0, 0, 0);
 }
 
-template <int TM>
-__global__ void __launch_bounds__(NT, TM == 128 ? 1 : 2) gemm_split2_kernel(GemmArgs<float> g) {
+template <int TM, int S>
+__global__ void __launch_bounds__(NT, TM == 128 && S > 2 ? 1 : 2) gemm_split2_kernel(GemmArgs<float> g) {
     constexpr int WMB = TM / 32;          // 16-row MFMA blocks per wave along M
     constexpr int ABLK = TM / 16;         // 16-row blocks of the A tile
     constexpr int NBLK = ABLK + BN / 16;  // blocks per plane per stage
     constexpr int IPW = 2 * NBLK / 4;     // 16-byte DMA instructions per wave per stage
-    __shared__ __attribute__((aligned(16))) unsigned char lds[kS2][2][NBLK][1024];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[S][2][NBLK][1024];
 
     if (g.skip_if && *(volatile const int*)g.skip_if != 0) return;
     const GemmSeg<float> s = g.seg[blockIdx.z];
@@ -797,19 +826,19 @@ __global__ void __launch_bounds__(NT, TM == 128 ? 1 : 2) gemm_split2_kernel(Gemm
             const unsigned short* base = P.hi + (pl ? P.ps : 0) + (long)rb * P.ld + k0;
             const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
                 (void*)base, 0, (int)(16 * P.ld * 2), 0x00020000);
-            dl_load16(r, &lds[kt % kS2][pl][blk][0], (rl * (int)P.ld + 8 * lkg) * 2);
+            dl_load16(r, &lds[kt % S][pl][blk][0], (rl * (int)P.ld + 8 * lkg) * 2);
         }
     };
 
     const int nk = (K + KC - 1) / KC;
-    for (int p = 0; p < kS2 - 1; ++p)
+    for (int p = 0; p < S - 1; ++p)
         if (p < nk) issue(p);
     for (int kt = 0; kt < nk; ++kt) {
-        if (kt + kS2 - 2 >= nk) wait_vm<0>();
-        else wait_vm<(kS2 - 2) * IPW>();
+        if (kt + S - 2 >= nk) wait_vm<0>();
+        else wait_vm<(S - 2) * IPW>();
         bar();
-        if (kt + kS2 - 1 < nk) issue(kt + kS2 - 1);
-        const int cur = kt % kS2;
+        if (kt + S - 1 < nk) issue(kt + S - 1);
+        const int cur = kt % S;
         bf16x8 ah[WMB], al[WMB], bh[4], bl[4];
 #pragma unroll
         for (int i = 0; i < WMB; ++i) {
@@ -869,6 +898,139 @@ __global__ void __launch_bounds__(NT, TM == 128 ? 1 : 2) gemm_split2_kernel(Gemm
                 float v = alpha * tot[t];
                 if (beta != 0.0f) v += beta * *c;
                 *c = v;
+            }
+        }
+    }
+}
+
+// Split-BF16 products too small to fill the chip with the stages above: as gemm_direct_kernel, from
+// the planes in global memory (a fragment is 16 consecutive bytes of a plane row) straight into the
+// MFMA registers, D chunks of 32 k ahead, 16 WM rows x 128 columns per workgroup, its four waves
+// side by side, operands swapped.  Products, their order and the flushes are those of the kernel
+// above, so both give the same bits.  Bound by the load latency and, with more rows, by the L1,
+// which passes each A fragment four times.
+template <int WM, int D>
+__global__ void __launch_bounds__(NT) gemm_split2_direct_kernel(GemmArgs<float> g) {
+    constexpr int WN = 2, TM = 16 * WM;
+    const GemmSeg<float> s = g.seg[blockIdx.z];
+    const int m0 = blockIdx.x * TM;
+    const int n0 = blockIdx.y * BN;
+    if (m0 >= s.M) return;
+    const bool tri = g.tri && (blockIdx.z == 0 || g.tri_all);
+    if (tri && m0 + TM - 1 + g.tri_off < n0) return;
+    const int skip = *(volatile const int*)(g.skip_if ? g.skip_if : &never_skip);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int li = lane & 15, lq = lane >> 4;
+    const int K = g.K, N = g.N, M = s.M;
+    const int nw = n0 + 32 * wave;
+    if (nw >= N) return;
+
+    // fragment bases; rows and columns clamped into the operands
+    const unsigned short *pa[WM], *pb[WN];
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+        pa[i] = s.ap.hi + (long)min(m0 + 16 * i + li, M - 1) * s.ap.ld + 8 * lq;
+#pragma unroll
+    for (int j = 0; j < WN; ++j)
+        pb[j] = g.bp.hi + (long)min(nw + 16 * j + li, N - 1) * g.bp.ld + 8 * lq;
+    const float alpha = g.alpha, beta = g.beta;
+    float old[WM][WN][4];
+    if (beta != 0.0f) {
+#pragma unroll
+        for (int i = 0; i < WM; ++i)
+#pragma unroll
+            for (int j = 0; j < WN; ++j)
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    old[i][j][t] = s.C[min(m0 + 16 * i + li, M - 1) +
+                                       (long)min(nw + 16 * j + 4 * lq + t, N - 1) * s.ldc];
+    }
+    f32x4 acc[WM][WN], sum[WM][WN];
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int j = 0; j < WN; ++j) acc[i][j] = sum[i][j] = f32x4{0, 0, 0, 0};
+    struct Frag {
+        bf16x8 a[2][WM], b[2][WN];
+    } f[D];
+    const int nk = (K + KC - 1) / KC;
+    auto load = [&](Frag& x, int kt) __attribute__((always_inline)) {
+        const long k0 = (long)min(kt, nk - 1) * KC;  // unconditional: the wait counts stay exact
+#pragma unroll
+        for (int i = 0; i < WM; ++i) {
+            x.a[0][i] = *(const bf16x8*)(pa[i] + k0);
+            x.a[1][i] = *(const bf16x8*)(pa[i] + s.ap.ps + k0);
+        }
+#pragma unroll
+        for (int j = 0; j < WN; ++j) {
+            x.b[0][j] = *(const bf16x8*)(pb[j] + k0);
+            x.b[1][j] = *(const bf16x8*)(pb[j] + g.bp.ps + k0);
+        }
+    };
+    auto mma = [&](Frag& x, int kt) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < WM; ++i)
+#pragma unroll
+            for (int j = 0; j < WN; ++j) {
+                f32x4& c = acc[i][j];
+                c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x.b[0][j], x.a[1][i], c, 0, 0, 0);
+                c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x.b[1][j], x.a[0][i], c, 0, 0, 0);
+                c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x.b[0][j], x.a[0][i], c, 0, 0, 0);
+            }
+        if ((kt % kFlush) == kFlush - 1) {
+#pragma unroll
+            for (int i = 0; i < WM; ++i)
+#pragma unroll
+                for (int j = 0; j < WN; ++j) {
+                    sum[i][j] += acc[i][j];
+                    acc[i][j] = f32x4{0, 0, 0, 0};
+                }
+        }
+    };
+    const int kf = K / KC;  // whole chunks
+#pragma unroll
+    for (int d = 0; d < D - 1; ++d) load(f[d], d);
+    int kt = 0;
+    for (; kt + D <= kf; kt += D) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            load(f[(d + D - 1) % D], kt + d + D - 1);
+            mma(f[d], kt + d);
+        }
+    }
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+        if (kt + d >= nk) break;
+        if (d == D - 1) load(f[d], kt + d);
+        if (kt + d >= kf) {
+            // the last chunk reads what follows in the plane row past K; zero it on both sides
+            const int kv = K - (kt + d) * KC - 8 * lq;
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                if (e >= kv) {
+#pragma unroll
+                    for (int i = 0; i < WM; ++i) f[d].a[0][i][e] = f[d].a[1][i][e] = (__bf16)0.0f;
+#pragma unroll
+                    for (int j = 0; j < WN; ++j) f[d].b[0][j][e] = f[d].b[1][j][e] = (__bf16)0.0f;
+                }
+        }
+        mma(f[d], kt + d);
+    }
+    if (skip) return;
+#pragma unroll
+    for (int i = 0; i < WM; ++i) {
+        const int row = m0 + 16 * i + li;
+#pragma unroll
+        for (int j = 0; j < WN; ++j) {
+            const f32x4 tot = sum[i][j] + acc[i][j];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const int col = nw + 16 * j + 4 * lq + t;
+                if (row >= M || col >= N || (tri && row + g.tri_off < col)) continue;
+                float v = alpha * tot[t];
+                if (beta != 0.0f) v += beta * old[i][j][t];
+                s.C[row + (long)col * s.ldc] = v;
             }
         }
     }
@@ -976,6 +1138,10 @@ __global__ __launch_bounds__(256) void expand_sym_kernel(const double* __restric
 // 2400 x 128 x 128 15.7 -> 6.3, 20000 x 256 x 256 (1,250) 51 -> 47, 1000 x 1000 x 2048 (256) 142 -> 62,
 // 1500 x 1500 x 1024 (564) 87 -> 103.  FP32 op(B) = B: 3000 x 1000 x 2048 (752) 184 -> 153, 2336 x
 // 2336 x 2048 (1,387) 247 -> 296.
+// 16-row groups up to which a split-BF16 product runs on its direct kernel.  Measured, staged ->
+// direct, us: 1400 rows, N = K = 128 (88) 15.8 -> 8.9, N = 256 (176) 18.1 -> 12.3, N = 384 (264) 18.6 ->
+// 12.8, N = 640 (440) 26.4 -> 23.0, N = 1280 (880) 40.8 -> 73.2.
+constexpr double kSplitDirect = 600;
 template <typename T>
 int direct_rows(const GemmArgs<T>& g, double cells) {
     const double groups = cells / (16 * BN);
@@ -1066,11 +1232,17 @@ int launch(const GemmArgs<T>& g, hipStream_t stream) {
                     set_error("gemm: the planes product takes one B for all segments");
                     return MOAO_ERR_ARG;
                 }
-            if (small) {
+            const double groups = cells / (16 * BN);
+            if (g.K > 0 && groups <= kSplitDirect) {
+                const int rows = groups <= 256 ? 16 : 32;
+                grid.x = (maxM + rows - 1) / rows;
+                auto k = rows == 16 ? gemm_split2_direct_kernel<1, 4> : gemm_split2_direct_kernel<2, 3>;
+                hipLaunchKernelGGL(k, grid, dim3(NT), 0, stream, g);
+            } else if (small) {
                 grid.x = (maxM + 63) / 64;
-                hipLaunchKernelGGL((gemm_split2_kernel<64>), grid, dim3(NT), 0, stream, g);
+                hipLaunchKernelGGL((gemm_split2_kernel<64, 3>), grid, dim3(NT), 0, stream, g);
             } else {
-                hipLaunchKernelGGL((gemm_split2_kernel<128>), grid, dim3(NT), 0, stream, g);
+                hipLaunchKernelGGL((gemm_split2_kernel<128, 2>), grid, dim3(NT), 0, stream, g);
             }
             MOAO_HIP_TRY(hipGetLastError());
             return MOAO_OK;
@@ -1094,6 +1266,21 @@ int launch(const GemmArgs<T>& g, hipStream_t stream) {
             return MOAO_OK;
         }
     }
+    // the kernels below leave seg[].cp to a pass of its own
+    struct AfterPlanes {
+        const GemmArgs<T>& g;
+        hipStream_t s;
+        int run() {
+            if constexpr (std::is_same<T, float>::value)
+                for (int i = 0; i < g.nseg; ++i)
+                    if (g.seg[i].cp)
+                        if (int rc = split_planes(g.seg[i].C, g.seg[i].ldc, g.seg[i].M, g.N,
+                                                  g.seg[i].cp, g.seg[i].cpl.ld, g.seg[i].cpl.ps, 1,
+                                                  s))
+                            return rc;
+            return MOAO_OK;
+        }
+    } after{g, stream};
     // the direct-to-LDS slice kernel, else the fallback
     const bool dl = g.transb == 1 || (kn_offsets_fit && (g.transb == 0 || g.symdiag));
     const bool half = dl ? half_tiles(g, cells) : small;
@@ -1110,7 +1297,7 @@ int launch(const GemmArgs<T>& g, hipStream_t stream) {
         k = half ? gemm_dl_kernel<T, 0, kStages, 64> : gemm_dl_kernel<T, 0, kStages, 128>;
     hipLaunchKernelGGL(k, grid, dim3(NT), 0, stream, g);
     MOAO_HIP_TRY(hipGetLastError());
-    return MOAO_OK;
+    return after.run();
 }
 
 }  // namespace

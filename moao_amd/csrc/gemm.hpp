@@ -40,6 +40,10 @@ struct GemmSeg {
     int M;
     Planes ap;  // split = 2: A's planes (row = row of this segment)
     const T* B;  // optional: this segment's own B (same shape and ldb), else GemmArgs::B
+    // FP32, split = 0, optional: the planes of C, written with it (element (r, c) as plane row r,
+    // k = c, at cp[r * cpl.ld + c]; 4 * N bytes aligned to 8)
+    unsigned short* cp;
+    Planes cpl;  // ld and ps of cp
 };
 
 template <typename T>

@@ -81,26 +81,12 @@ int over_groups(const std::vector<RowGroup<T>>& groups, GemmArgs<T> proto, bool 
     return MOAO_OK;
 }
 
-// Planes of the columns [j0, j0 + nn) just finalised, for the split-BF16 updates: rows
-// [r0, n) of the SPD block (lead) and every row of the (single) row group.
+// The planes of a panel's result, for the split-BF16 updates.
 template <typename T>
-int split_cols_done(const Tall<T>& p, long r0, long j0, long nn, bool lead) {
-    if constexpr (std::is_same<T, float>::value) {
-        const SplitWs& w = *p.sw;
-        if (lead && p.n > r0)
-            if (int rc = split_planes(p.a(r0, j0), p.lda, (int)(p.n - r0), (int)nn,
-                                      w.lp + r0 * w.ld + j0, w.ld, w.lps, 1, p.s))
-                return rc;
-        for (const auto& g : *p.groups)
-            if (g.rows > 0)
-                if (int rc = split_planes(g.p + j0 * g.ld, g.ld, g.rows, (int)nn, w.xp + j0, w.ld,
-                                          w.xps, 1, p.s))
-                    return rc;
-        return MOAO_OK;
-    } else {
-        set_error("split-BF16 planes need FP32 storage");
-        return MOAO_ERR_ARG;
-    }
+GemmSeg<T> with_planes(GemmSeg<T> sg, const Planes& p) {
+    sg.cp = const_cast<unsigned short*>(p.hi);
+    sg.cpl = p;
+    return sg;
 }
 
 // Factor columns [j0, j0+nn) of the tall matrix (all earlier columns already applied).
@@ -125,16 +111,17 @@ int potrf_rec(const Tall<T>& p, long j0, long nn) {
         if (int rc = over_groups<T>(
                 G, proto, below > 0,
                 [&] {
-                    return GemmSeg<T>{p.a(j0 + nn, j0), p.a(j0 + nn, j0), p.lda, p.lda,
-                                      (int)below};
+                    GemmSeg<T> sg{p.a(j0 + nn, j0), p.a(j0 + nn, j0), p.lda, p.lda, (int)below};
+                    return p.sw ? with_planes(sg, p.sw->l_rows(j0 + nn, j0)) : sg;
                 },
                 [&](const RowGroup<T>& g) {
                     T* c = g.p + j0 * g.ld;
-                    return GemmSeg<T>{c, c, g.ld, g.ld, g.rows};
+                    GemmSeg<T> sg{c, c, g.ld, g.ld, g.rows};
+                    return p.sw ? with_planes(sg, p.sw->x_rows(j0)) : sg;
                 },
                 p.s))
             return rc;
-        return p.sw ? split_cols_done(p, j0, j0, nn, true) : MOAO_OK;
+        return MOAO_OK;
     }
     const long n1 = split(nn);
     if (int rc = potrf_rec(p, j0, n1)) return rc;
@@ -190,11 +177,12 @@ int trsmN_rec(const Tall<T>& p, long j0, long nn) {
         if (int rc = over_groups<T>(G, proto, false, none,
                                     [&](const RowGroup<T>& g) {
                                         T* c = g.p + j0 * g.ld;
-                                        return GemmSeg<T>{c, c, g.ld, g.ld, g.rows};
+                                        GemmSeg<T> sg{c, c, g.ld, g.ld, g.rows};
+                                        return p.sw ? with_planes(sg, p.sw->x_rows(j0)) : sg;
                                     },
                                     p.s))
             return rc;
-        return p.sw ? split_cols_done(p, 0, j0, nn, false) : MOAO_OK;
+        return MOAO_OK;
     }
     const long n1 = split(nn);
     if (int rc = trsmN_rec(p, j0 + n1, nn - n1)) return rc;
@@ -242,11 +230,12 @@ int trsmT_rec(const Tall<T>& p, long j0, long nn) {
         if (int rc = over_groups<T>(G, proto, false, none,
                                     [&](const RowGroup<T>& g) {
                                         T* c = g.p + j0 * g.ld;
-                                        return GemmSeg<T>{c, c, g.ld, g.ld, g.rows};
+                                        GemmSeg<T> sg{c, c, g.ld, g.ld, g.rows};
+                                        return p.sw ? with_planes(sg, p.sw->x_rows(j0)) : sg;
                                     },
                                     p.s))
             return rc;
-        return p.sw ? split_cols_done(p, 0, j0, nn, false) : MOAO_OK;
+        return MOAO_OK;
     }
     const long n1 = split(nn);
     if (int rc = trsmT_rec(p, j0, n1)) return rc;

@@ -38,7 +38,7 @@ struct RowGroup {
 // solved by L^T on the way (first right-side solve fused).  invL receives the inverse of every
 // kLeaf leaf (ceil(n/kLeaf)*kLeaf*kLeaf elements); *info the dpotrf status (device int).
 // sw (FP32 storage only): run the update products (not the leaves' panel products) on the
-// split-BF16 planes kernel, writing the planes of every finished leaf column into sw->lp and
+// split-BF16 kernels; the panel products write the planes of what they finish into sw->lp and
 // sw->xp (one row group at most).
 template <typename T>
 int potrf_tall(long n, T* A, long lda, const std::vector<RowGroup<T>>& groups, T* invL,

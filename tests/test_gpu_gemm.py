@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 from moao_amd.device import DeviceArray
-from moao_amd.reconstructor import dgemm_dev, sgemm_dev
+from moao_amd.reconstructor import dgemm_dev, sgemm_bf16x3_dev, sgemm_dev
 
 pytestmark = pytest.mark.gpu
 
@@ -208,3 +208,29 @@ def test_symmetric_operand_from_its_lower_triangle(M, K):
         DeviceArray.from_host(np.zeros((M, K), order="F"))
     dgemm_dev(2, M, K, K, 1.0, dA.ptr, M, dB.ptr, K, 0.0, dC.ptr, M)
     assert np.max(np.abs(dC.to_host() - A @ S)) <= 2 * K * 2.0 ** -52 * 2
+
+
+@pytest.mark.parametrize("transb", [0, 1])
+def test_few_rows_of_the_split_bf16_product(transb):
+    """The split-BF16 product of few rows (16- or 32-row workgroups without LDS) has the bits of those
+    rows in a product large enough for the staged kernel: K below, at and past whole chunks of 32
+    and flushes of 256, ragged columns, beta = 0 and 1."""
+    rng = np.random.default_rng(30 + transb)
+    big = 16000
+    for N, K in [(128, 128), (131, 300), (97, 31), (128, 600)]:
+        ldb = N if transb == 1 else K
+        A = np.asfortranarray(rng.standard_normal((big, K)).astype(np.float32))
+        B = np.asfortranarray(rng.standard_normal((ldb, N if transb == 0 else K)).astype(np.float32))
+        C = np.asfortranarray(rng.standard_normal((big, N)).astype(np.float32))
+        dA, dB = DeviceArray.from_host(A), DeviceArray.from_host(B)
+        for beta in (0.0, 1.0):
+            dC = DeviceArray.from_host(C)
+            sgemm_bf16x3_dev(transb, big, N, K, -1.25, dA.ptr, big, dB.ptr, ldb, beta, dC.ptr, big)
+            want = dC.to_host()
+            for r in (1, 16, 17, 300, 2049, 4097, 5000):
+                print(f"[split-direct] transb={transb} N={N} K={K} rows={r}", flush=True)
+                dC = DeviceArray.from_host(C)
+                sgemm_bf16x3_dev(transb, r, N, K, -1.25, dA.ptr, big, dB.ptr, ldb, beta, dC.ptr, big)
+                got = dC.to_host()
+                assert np.array_equal(got[:r], want[:r])
+                assert np.array_equal(got[r:], C[r:])
