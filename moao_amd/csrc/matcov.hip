@@ -776,6 +776,13 @@ int matcov_tile_launch(double* d_data, int nrows, int ncols, int xoffset, int yo
             }
     }
 
+    if (type_mat == 1 && xoffset + nrows - 1 < yoffset) {
+        // wholly above the diagonal: nothing to write, no tables to build (53 -> 10 us); as below,
+        // the call returns when the stream is idle
+        MOAO_HIP_TRY(hipStreamSynchronize(stream));
+        return MOAO_OK;
+    }
+
     // Whole Cmm / Ctm: lattice_fill and pair_kernel (one lane per subaperture pair).
     const bool pairs = (type_mat == 1 || type_mat == 3) && xoffset == 0 && yoffset == 0 &&
                        nrows == row_lim && ncols == col_lim;

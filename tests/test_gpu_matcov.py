@@ -214,3 +214,20 @@ def test_grids_and_free_sensors(tmp_path, field, value):
     gm.matcov_tile(g, n, m, 0, 0, n, t, gm.CMAA)
     om.matcov_tile(r, n, m, 0, 0, n, o, 2)
     assert np.max(np.abs(g - r)) <= 1e-12 * np.max(np.abs(om.ctt(o)))
+
+
+@pytest.mark.parametrize("xo,yo", [(0, 90), (10, 90), (49, 89), (50, 89), (51, 89)])
+def test_cmm_tiles_at_and_above_the_diagonal(tmp_path, xo, yo):
+    """A 40 x 30 tile of Cmm wholly above the diagonal writes nothing; one that touches it with its
+    last row writes what lies on or below it."""
+    from moao_amd import systems
+    s, a = systems.make_system(str(tmp_path), systems.SystemSpec(diam=8.0, nssp=8, nlgs=2, nngs=1,
+                                                                 nlayer=2, seed=5))
+    t = Tomo(s, a[0])
+    t.set_target(0)
+    C = gm.cmm(t)
+    buf = np.full((40, 30), -1.0, order="F")
+    gm.matcov_tile(buf, 40, 30, xo, yo, 40, t, gm.CMM)
+    low = np.arange(xo, xo + 40)[:, None] >= np.arange(yo, yo + 30)[None, :]
+    assert np.array_equal(buf[low], C[xo:xo + 40, yo:yo + 30][low])
+    assert np.all(buf[~low] == -1.0)
