@@ -20,7 +20,8 @@
 //  * gemm_kernel (fallback: symmetric B without scratch, K x N slabs whose byte
 //    offsets would overflow 32 bits): register-staged, double-buffered LDS, the next slice's
 //    global loads issued before the current slice's MFMAs.
-// Slice launches use 128-row or 64-row tiles (each wave 32x64, up to 4 workgroups per CU): half_tiles.
+// Slice launches use 128-row or 64-row tiles (each wave 32x64, up to 4 workgroups per CU):
+// half_tiles.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -422,8 +423,9 @@ __global__ void __launch_bounds__(NT, TM == 128 ? 2 : 4) gemm_dl_kernel(GemmArgs
         // slice's reads and its MFMAs and the compiler starts the second half's reads before the
         // first half's MFMAs; and waves with rows or columns outside the matrix (or wholly above
         // the diagonal) leave out their MFMAs, which gives the matrix core to the CU's other
-        // workgroup.  16384^3: 73.5 -> 75.0 TF/s; 9344 x 2336 x 18688: 60.6 -> 64.2.  The other forms
-        // lose by either (16384^3, FP64 op(B) = B 72.8 -> 71.9, FP32 145 -> 137) and keep one loop.
+        // workgroup.  16384^3: 73.5 -> 75.0 TF/s; 9344 x 2336 x 18688: 60.6 -> 64.2.  The other
+        // forms lose by either (16384^3, FP64 op(B) = B 72.8 -> 71.9, FP32 145 -> 137) and keep one
+        // loop.
         auto slice = [&](int kt, auto tailc, auto nic) __attribute__((always_inline)) {
             constexpr bool tail = decltype(tailc)::value;
             constexpr int NI = decltype(nic)::value;  // of the wave's WMB row blocks
@@ -770,9 +772,9 @@ constexpr int KC = 32;  // k per chunk (one 16x16x32 step)
 // conflict-free 16-byte LDS read.  The blocks are filled by 16-byte buffer loads straight into
 // LDS (buffer_load_dwordx4 ... lds, one 1 KB block per instruction, no registers), S stages
 // deep: two for 128-row tiles, so that two workgroups share a CU (4864 x 9728 x 4864: 1,258 us with
-// three to five stages and one workgroup, 935 with two).  Products accumulate in FP32 in the MFMA; every kFlush stages the accumulators are
-// added into a second set of FP32 sums and restarted, so no accumulation chain runs longer
-// than 256 k.
+// three to five stages and one workgroup, 935 with two).  Products accumulate in FP32 in the MFMA;
+// every kFlush stages the accumulators are added into a second set of FP32 sums and restarted, so
+// no accumulation chain runs longer than 256 k.
 constexpr int kFlush = 8;   // stages between flushes of the MFMA accumulators
 
 __device__ __forceinline__ void dl_load16(__amdgpu_buffer_rsrc_t r, void* lds, int voff) {
@@ -1087,10 +1089,11 @@ __global__ void symdiag_kernel(const T* __restrict__ B, long ldb, int K, T* __re
     out[(long)blockIdx.y * BN * BN + i] = B[hi + (long)lo * ldb];
 }
 
-// out(c, k) = sym(B)(c0 + c, k), c < P, k < K, at out[c + k P]: rows c0 .. c0 + P - 1 of a symmetric
-// matrix of which the lower triangle is stored (c0 and, unless it ends the matrix, P multiples of
-// 64).  One workgroup per 64 x 64 tile of the triangle (blockIdx.x <= blockIdx.y), read once and
-// written as it is and, through LDS, transposed.  Bound by memory, 12 bytes per element.
+// out(c, k) = sym(B)(c0 + c, k), c < P, k < K, at out[c + k P]: rows c0 .. c0 + P - 1 of a
+// symmetric matrix of which the lower triangle is stored (c0 and, unless it ends the matrix, P
+// multiples of 64).  One workgroup per 64 x 64 tile of the triangle (blockIdx.x <= blockIdx.y),
+// read once and written as it is and, through LDS, transposed.  Bound by memory, 12 bytes per
+// element.
 __global__ __launch_bounds__(256) void expand_sym_kernel(const double* __restrict__ B, long ldb,
                                                          int K, int c0, int P,
                                                          double* __restrict__ out) {
@@ -1123,25 +1126,26 @@ __global__ __launch_bounds__(256) void expand_sym_kernel(const double* __restric
     }
 }
 
+// 16-row groups up to which a split-BF16 product runs on its direct kernel.  Measured, staged ->
+// direct, us: 1400 rows, N = K = 128 (88) 15.8 -> 8.9, N = 256 (176) 18.1 -> 12.3, N = 384 (264)
+// 18.6 -> 12.8, N = 640 (440) 26.4 -> 23.0, N = 1280 (880) 40.8 -> 73.2.
+constexpr double kSplitDirect = 600;
+
 // Rows per workgroup of the direct kernel for this product, 0 where the slice kernels are the
 // faster ones.  16-row workgroups while they fit the 256 CUs at once (then a wave's own chain of
 // MFMAs is the time, and a 16-row block's is half a 32-row block's), else 32-row workgroups up to
 // the count where the slice kernels' operand reuse through LDS wins: the direct kernel reads every
-// operand from L1/L2.  That point comes the sooner the longer K (operands that leave L2), with FP32's
-// twice as fast MFMAs, and for FP64 op(B) = B (lane exchanges).
-// Measured, slice kernel -> direct kernel, us (M x N x K; w = 32-row workgroups).  FP64 op(B) = B^T:
-// 152 x 128 x 128 19.5 -> 7.4, 300 x 1000 x 8192 816 -> 225, 1000 x 1000 x 8192 (w 256) 822 -> 375,
-// 5000 x 1024 x 1024 (1,256) 216 -> 199, 20000 x 256 x 256 (1,250) 70 -> 61, 1500 x 1500 x 16384 (564)
-// 2035 -> 2033, 2336 x 2336 x 2048 (1,387) 416 -> 452, 2336 x 2336 x 8192 1637 -> 1782, 10000 x 2048 x
-// 2048 (5,008) 1259 -> 1507.  FP64 op(B) = B: 152 x 128 x 128 18.6 -> 9.1, 1000 x 1000 x 2048 (256)
-// 200 -> 103, 5000 x 512 x 512 (628) 81 -> 77, 1500 x 1500 x 2048 (564) 254 -> 269.  FP32 op(B) = B^T:
-// 2400 x 128 x 128 15.7 -> 6.3, 20000 x 256 x 256 (1,250) 51 -> 47, 1000 x 1000 x 2048 (256) 142 -> 62,
-// 1500 x 1500 x 1024 (564) 87 -> 103.  FP32 op(B) = B: 3000 x 1000 x 2048 (752) 184 -> 153, 2336 x
-// 2336 x 2048 (1,387) 247 -> 296.
-// 16-row groups up to which a split-BF16 product runs on its direct kernel.  Measured, staged ->
-// direct, us: 1400 rows, N = K = 128 (88) 15.8 -> 8.9, N = 256 (176) 18.1 -> 12.3, N = 384 (264) 18.6 ->
-// 12.8, N = 640 (440) 26.4 -> 23.0, N = 1280 (880) 40.8 -> 73.2.
-constexpr double kSplitDirect = 600;
+// operand from L1/L2.  That point comes the sooner the longer K (operands that leave L2), with
+// FP32's twice as fast MFMAs, and for FP64 op(B) = B (lane exchanges). Measured, slice kernel ->
+// direct kernel, us (M x N x K; w = 32-row workgroups).  FP64 op(B) = B^T: 152 x 128 x 128 19.5 ->
+// 7.4, 300 x 1000 x 8192 816 -> 225, 1000 x 1000 x 8192 (w 256) 822 -> 375, 5000 x 1024 x 1024
+// (1,256) 216 -> 199, 20000 x 256 x 256 (1,250) 70 -> 61, 1500 x 1500 x 16384 (564) 2035 -> 2033,
+// 2336 x 2336 x 2048 (1,387) 416 -> 452, 2336 x 2336 x 8192 1637 -> 1782, 10000 x 2048 x 2048
+// (5,008) 1259 -> 1507.  FP64 op(B) = B: 152 x 128 x 128 18.6 -> 9.1, 1000 x 1000 x 2048 (256) 200
+// -> 103, 5000 x 512 x 512 (628) 81 -> 77, 1500 x 1500 x 2048 (564) 254 -> 269.  FP32 op(B) = B^T:
+// 2400 x 128 x 128 15.7 -> 6.3, 20000 x 256 x 256 (1,250) 51 -> 47, 1000 x 1000 x 2048 (256) 142 ->
+// 62, 1500 x 1500 x 1024 (564) 87 -> 103.  FP32 op(B) = B: 3000 x 1000 x 2048 (752) 184 -> 153,
+// 2336 x 2336 x 2048 (1,387) 247 -> 296.
 template <typename T>
 int direct_rows(const GemmArgs<T>& g, double cells) {
     const double groups = cells / (16 * BN);
@@ -1161,10 +1165,11 @@ int direct_rows(const GemmArgs<T>& g, double cells) {
 // ceil(w) rounds is part empty.  So: few rounds, or a short K; sooner so for op(B) = B, whose loads
 // of half cache lines gain from more waves, and later for FP32, whose 128-row tiles are five to a
 // CU already.  Measured, 128 -> 64 rows, TF/s.  FP64 op(B) = B^T: w 3.2, K 1024 51 -> 61; 4.1, 4096
-// 58 -> 61; 6.9, 4096 70.0 -> 68.3; 16, 256 45 -> 53; 16, 1024 67.7 -> 68.0; 64, 1024 70.1 -> 69.2.  FP64
-// op(B) = B: 3.2, 1024 52 -> 62; 64, 4096 70.4 -> 70.9; 9.4, 16384 67.6 -> 69.3; 16, 16384 72.2 -> 70.2.
-// FP32 op(B) = B^T: 5.1, 1024 105 -> 111; 8.6, 1024 123 -> 118; 4.1, 4096 114 -> 114; 16, 256 76 -> 79.
-// FP32 op(B) = B: 9.4, 1024 117 -> 123; 16, 1024 126 -> 123; 4.1, 4096 111 -> 116; 6.9, 4096 134 -> 128.
+// 58 -> 61; 6.9, 4096 70.0 -> 68.3; 16, 256 45 -> 53; 16, 1024 67.7 -> 68.0; 64, 1024 70.1 -> 69.2.
+// FP64 op(B) = B: 3.2, 1024 52 -> 62; 64, 4096 70.4 -> 70.9; 9.4, 16384 67.6 -> 69.3; 16, 16384
+// 72.2 -> 70.2. FP32 op(B) = B^T: 5.1, 1024 105 -> 111; 8.6, 1024 123 -> 118; 4.1, 4096 114 -> 114;
+// 16, 256 76 -> 79. FP32 op(B) = B: 9.4, 1024 117 -> 123; 16, 1024 126 -> 123; 4.1, 4096 111 ->
+// 116; 6.9, 4096 134 -> 128.
 template <typename T>
 bool half_tiles(const GemmArgs<T>& g, double cells) {
     const double w = cells / (BM * BN * 256.0);

@@ -75,8 +75,8 @@ struct GemmArgs {
 // Scratch for products with a symmetric operand.  From kSymRows rows on it holds the matrix written
 // out in full, so that they run on the kernel for op(B) = B^T; with fewer, full copies of its 128 x
 // 128 diagonal blocks, with which a kernel reads the lower triangle in place, columns above the
-// diagonal and rows below it.  K = 18,688, in place -> in full: 256 rows 4.1 -> 5.3 ms, 512 rows 9.8 ->
-// 7.6, 8 x 2,336 rows 213 -> 187.  Stream-ordered, for one matrix and one caller's scope.
+// diagonal and rows below it.  K = 18,688, in place -> in full: 256 rows 4.1 -> 5.3 ms, 512 rows
+// 9.8 -> 7.6, 8 x 2,336 rows 213 -> 187.  Stream-ordered, for one matrix and one caller's scope.
 constexpr long kSymRows = 448;
 struct SymWork {
     double* p = nullptr;

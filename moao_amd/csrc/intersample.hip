@@ -24,8 +24,8 @@
 //   psf_rows     per row: along the last axis -> PSF, and its mirror row
 // Between passes H(x, j) and H(-x, j) are stored for x = N/2 .. N and j = 0 .. N/2, in tiles of
 // kRows x kRows that the writing workgroup fills and the reading workgroup takes whole.
-// N = 2048, 8 directions, FP32, nact = 4,724: 6 launches, 0.54 ms (gather 0.37, then 0.01, 0.01, 0.04,
-// 0.06, 0.06); as full transforms (radix-4 rows, transpose, rows) with pointwise passes and a
+// N = 2048, 8 directions, FP32, nact = 4,724: 6 launches, 0.54 ms (gather 0.37, then 0.01, 0.01,
+// 0.04, 0.06, 0.06); as full transforms (radix-4 rows, transpose, rows) with pointwise passes and a
 // gather by entries between them 15 launches, 2.2 ms, of which the gather 1.17.  N = 512, one
 // direction, FP64: 49 -> 18 us.
 #include <hip/hip_runtime.h>
@@ -92,9 +92,11 @@ constexpr int kMaxSlabs = 32;
 // bins read neighbouring entries and 3.3 ms in random order.
 constexpr long kRunFrom = 4;
 constexpr long kSlabMax = 1L << 26;  // doubles: byte offsets in a slab stay below 2^31
-// Bins per group: wide groups read a DM row, and mostly the next one too, with the same wave, so
-// the cache lines in which rows meet are fetched once; narrow ones spread a small map's work.
-constexpr int kWide = 8, kWideFrom = 128 * 64;
+// Bins per group, in blocks of 64: wide groups read a DM row with one wave, so its cache lines are
+// fetched once; narrower ones spread the work of a small map or a single direction.  nact = 4,724,
+// whole call at N = 512, us by 2, 3, 5, 8 blocks: 8 directions 406, 398, 398, 403; one 62, 72, 99,
+// 159.
+constexpr int kWide = 3, kWideFrom = 128 * 64;
 
 enum { kOrderRowUp = 0, kOrderRowDown, kOrderColUp, kOrderColDown };
 __host__ __device__ inline int bin_place(int order, int ti, int tj, int ncov) {
@@ -102,13 +104,13 @@ __host__ __device__ inline int bin_place(int order, int ti, int tj, int ncov) {
     return order & 1 ? ncov * ncov - 1 - c : c;
 }
 
-// Partial sums of one item for ND directions; the waves take 8 runs each in turn.  Bound by HBM: 1.43
-// GB of Cvv (nact = 4,724, 8 directions) in 370 us; with groups of 64 bins, where rows are cut at
-// every group, 400 us and 1.4 times the cache lines.  Lanes outside a run and directions outside the batch read past the buffer
-// resource's end, which the hardware answers with zero and no traffic, so the loads stand without
-// branches.  A run lies in blocks k and k + 1 of the group's W blocks of 64 bins, k uniform.
-// XCD c takes the c-th eighth of the items.
-// part[((item W + k) batch + direction) 64 + lane].
+// Partial sums of one item for ND directions; the waves take 8 runs each in turn.  Bound by HBM:
+// 1.43 GB of Cvv (nact = 4,724, 8 directions) in 370 us; with groups of 64 bins, where rows are cut
+// at every group, 400 us and 1.4 times the cache lines.  Lanes outside a run and directions outside
+// the batch read past the buffer resource's end, which the hardware answers with zero and no
+// traffic, so the loads stand without branches.  A run lies in blocks k and k + 1 of the group's W
+// blocks of 64 bins, k uniform. XCD c takes the c-th eighth of the items. part[((item W + k) batch
+// + direction) 64 + lane].
 template <int W, int ND>
 __global__ __launch_bounds__(kGatherWaves * 64) void gather_runs(
     const double* __restrict__ cvv, long nidx, long slab, const Item* __restrict__ items,
@@ -176,8 +178,8 @@ __global__ __launch_bounds__(kGatherWaves * 64) void gather_runs(
     }
 }
 
-// The same sums where consecutive entries seldom fall in consecutive bins: one wave per bin over the
-// list of its entries.  Sums as map_sums leaves them.
+// The same sums where consecutive entries seldom fall in consecutive bins: one wave per bin over
+// the list of its entries.  Sums as map_sums leaves them.
 __global__ __launch_bounds__(256) void gather_entries(const double* __restrict__ cvv, long nidx,
                                                       const int* __restrict__ off,
                                                       const int* __restrict__ ent, int nmap,
@@ -351,7 +353,8 @@ __global__ __launch_bounds__((RowFft<R, LOG>::kThreads), (RowFft<R, LOG>::kWaves
     }
 }
 
-// Bound by its writes (67 MB at N = 2048 and 4 pairs, 40 us): columns j <= N/2, transform along x, product with abs2fi, transform back.  mid[j] = H(N/2, j).
+// Bound by its writes (67 MB at N = 2048 and 4 pairs, 40 us): columns j <= N/2, transform along x,
+// product with abs2fi, transform back.  mid[j] = H(N/2, j).
 template <typename R, int LOG>
 __global__ __launch_bounds__((RowFft<R, LOG>::kThreads), (RowFft<R, LOG>::kWaves)) void map_cols(
     Grid<R> g, const typename Cplx<R>::type* __restrict__ A, const R* __restrict__ w,
@@ -411,9 +414,9 @@ __device__ __forceinline__ double phase_exp(double x) {
 }
 
 // Bound half by memory (67 MB in, 67 MB out), half by arithmetic; 57 us at N = 2048, 4 pairs.
-// Rows N/2 + r, r <= N/2: D along y, dphi = exp(-0.5 (norm - D) scale), scale = fact / fact2, shifted by half a
-// row (its row r, column y + N/2), times the OTF's row r, transform along the row.
-// norm = D(N/2, N/2) = the alternating sum of H(N/2, j) over all j, taken in FP64.
+// Rows N/2 + r, r <= N/2: D along y, dphi = exp(-0.5 (norm - D) scale), scale = fact / fact2,
+// shifted by half a row (its row r, column y + N/2), times the OTF's row r, transform along the
+// row. norm = D(N/2, N/2) = the alternating sum of H(N/2, j) over all j, taken in FP64.
 template <typename R, int LOG>
 __global__ __launch_bounds__((RowFft<R, LOG>::kThreads), (RowFft<R, LOG>::kWaves)) void dphi_rows(
     Grid<R> g, const typename Cplx<R>::type* __restrict__ H,

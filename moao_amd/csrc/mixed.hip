@@ -432,7 +432,8 @@ int reconstructor_mixed_dev(long n, long m, const double* Cmm, long ldCmm, doubl
         std::fprintf(stderr, "[mixed] |Z|=%.6e |Z2|=%.6e |R0|=%.6e\n", a, b2, c2);
     }
 
-    // --- 4. refinement (the residual's symmetric operand Cmm written out in full where there is room)
+    // --- 4. refinement (the residual's symmetric operand Cmm written out in full where there is
+    // room)
     SymWork sym;
     sym_alloc(sym, m, n, s);
     double rel = 0;

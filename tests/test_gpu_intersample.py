@@ -242,13 +242,14 @@ def test_every_grid_size(prec, tol, N, nssp, batch):
         assert err <= tol
 
 
+@pytest.mark.parametrize("nssp", [20, 46])  # groups of 64 bins and of 192
 @pytest.mark.parametrize("order", ["reversed", "transposed", "both", "shuffled", "few"])
-def test_index_orders(order):
+def test_index_orders(order, nssp):
     """The index may list the pairs in any order: the other actuator first (map bins descend
     along Cvv), actuators by columns (bins a map row apart), at random, or a few pairs only (bins
     without hits)."""
-    print(f"[psf] index order {order}", flush=True)
-    N, nssp = 512, 20
+    print(f"[psf] index order {order} nssp={nssp}", flush=True)
+    N = 512
     dm, idx, a2f, otf, cvv = _inputs(nssp, N, 8.0, 3e-4)
     np_, ncov = dm.ndiam, 2 * dm.ndiam - 1
     ti, tj = (idx - 1) // ncov, (idx - 1) % ncov
