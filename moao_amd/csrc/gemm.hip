@@ -29,6 +29,7 @@
 
 #include "common.hpp"
 #include "gemm.hpp"
+#include "mfma.hpp"
 #include "profile.hpp"
 
 namespace moao {
@@ -41,29 +42,6 @@ constexpr int NT = 256;
 #define MOAO_GEMM_STAGES 3
 #endif
 constexpr int kStages = MOAO_GEMM_STAGES;  // direct-to-LDS pipeline depth (slices in flight + 1)
-
-template <typename T>
-struct Mfma;
-
-template <>
-struct Mfma<double> {
-    typedef double acc_t __attribute__((ext_vector_type(4)));
-    static __device__ __forceinline__ acc_t mac(double a, double b, acc_t c) {
-        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-    }
-    // accumulator item t of lane l holds row (l/16) + 4t of the 16x16 block
-    static __device__ __forceinline__ int row(int lane, int t) { return (lane >> 4) + 4 * t; }
-};
-
-template <>
-struct Mfma<float> {
-    typedef float acc_t __attribute__((ext_vector_type(4)));
-    static __device__ __forceinline__ acc_t mac(float a, float b, acc_t c) {
-        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-    }
-    // accumulator item t of lane l holds row 4*(l/16) + t of the 16x16 block
-    static __device__ __forceinline__ int row(int lane, int t) { return 4 * (lane >> 4) + t; }
-};
 
 // TB: 0 = B is K x N, 1 = B is N x K (op = transpose), 2 = B symmetric K x K, lower stored.
 // Loads are branch-free: addresses are clamped into the matrix and out-of-range values zeroed
@@ -524,38 +502,6 @@ __global__ void __launch_bounds__(NT, TM == 128 ? 2 : 4) gemm_dl_kernel(GemmArgs
             }
         }
     }
-}
-
-// 4x4 transpose between four registers and the four 16-lane rows of a wave: lane row q's
-// register t becomes lane row t's register q (gfx950 row swaps; no LDS).
-__device__ __forceinline__ void swap_rows(unsigned (&x)[4]) {
-    auto p = __builtin_amdgcn_permlane32_swap(x[0], x[2], false, false);
-    auto q = __builtin_amdgcn_permlane32_swap(x[1], x[3], false, false);
-    auto r = __builtin_amdgcn_permlane16_swap(p[0], q[0], false, false);
-    auto s = __builtin_amdgcn_permlane16_swap(p[1], q[1], false, false);
-    x[0] = r[0];
-    x[1] = r[1];
-    x[2] = s[0];
-    x[3] = s[1];
-}
-template <typename T>
-__device__ __forceinline__ void lane_rows_transpose(T& a, T& b, T& c, T& d) {
-    constexpr int W = sizeof(T) / 4;
-    unsigned v[4][W], x[4];
-    __builtin_memcpy(v[0], &a, sizeof(T));
-    __builtin_memcpy(v[1], &b, sizeof(T));
-    __builtin_memcpy(v[2], &c, sizeof(T));
-    __builtin_memcpy(v[3], &d, sizeof(T));
-#pragma unroll
-    for (int w = 0; w < W; ++w) {
-        for (int t = 0; t < 4; ++t) x[t] = v[t][w];
-        swap_rows(x);
-        for (int t = 0; t < 4; ++t) v[t][w] = x[t];
-    }
-    __builtin_memcpy(&a, v[0], sizeof(T));
-    __builtin_memcpy(&b, v[1], sizeof(T));
-    __builtin_memcpy(&c, v[2], sizeof(T));
-    __builtin_memcpy(&d, v[3], sizeof(T));
 }
 
 // hi and lo planes of four consecutive k of one row, those below N (see Planes).

@@ -324,3 +324,42 @@ def test_leaf_edges(n):
             Bb = B.copy(order="F")
             assert reconstructor(n, 37, Cb, n, Bb, 37, 1) == p + 1, (n, p, bad)
             assert np.array_equal(Bb, B)
+
+
+@pytest.mark.parametrize("n,m,ngal", [(129, 1, 1), (200, 15, 1), (256, 16, 2), (257, 17, 1), (300, 33, 9),
+                                      (384, 16, 1), (385, 20, 1), (450, 31, 3), (511, 16, 1), (512, 48, 1),
+                                      (513, 16, 1), (640, 7, 1), (1100, 40, 2), (1409, 16, 1)])
+def test_backward_solve_segments(n, m, ngal):
+    """The backward solve's segments of two, three and four leaves, the last one whole or down to a
+    single column, rows at the edges of the 16-row workgroups and more targets than one launch
+    takes: backward error of R in both precisions (bars as above), and every target as alone."""
+    from moao_amd.reconstructor import sreconstructor
+    print(f"[recon] segments n={n} m={m} ngal={ngal}", flush=True)
+    rng = np.random.default_rng(n + m)
+    G = rng.standard_normal((n, n))
+    S = G @ G.T / n + np.eye(n)
+    B = [np.asfortranarray(rng.standard_normal((m, n))) for _ in range(ngal)]
+    for f, dt, bar in ((reconstructor, np.float64, 5e-13), (sreconstructor, np.float32, 1e-5)):
+        R = np.concatenate([b.astype(dt).flatten(order="F") for b in B])
+        C = np.asfortranarray(np.tril(S).astype(dt))
+        assert f(n, m, C, n, R, m, ngal) == 0
+        for g in range(ngal):
+            r = R[g * n * m:(g + 1) * n * m].reshape((m, n), order="F")
+            assert np.linalg.norm(B[g] - r.astype(np.float64) @ S) / np.linalg.norm(B[g]) <= bar
+        one = np.asfortranarray(B[-1].astype(dt))
+        assert f(n, m, np.asfortranarray(np.tril(S).astype(dt)), n, one, m, 1) == 0
+        assert np.array_equal(one, r)
+
+
+def test_backward_solve_of_many_rows_equals_that_of_few():
+    """Beyond 8,192 rows the segments run as single products again, in the same order: the first rows
+    of a large solve have the bits of a small one."""
+    n, big, few = 640, 8300, 40
+    rng = np.random.default_rng(77)
+    G = rng.standard_normal((n, n))
+    C = np.asfortranarray(np.tril(G @ G.T / n + np.eye(n)))
+    B = np.asfortranarray(rng.standard_normal((big, n)))
+    R, r = B.copy(order="F"), np.asfortranarray(B[:few].copy())
+    assert reconstructor(n, big, C.copy(order="F"), n, R, big, 1) == 0
+    assert reconstructor(n, few, C.copy(order="F"), n, r, few, 1) == 0
+    assert np.array_equal(R[:few], r)
