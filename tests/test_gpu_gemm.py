@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 from moao_amd.device import DeviceArray
-from moao_amd.reconstructor import dgemm_dev, sgemm_bf16x3_dev, sgemm_dev
+from moao_amd.reconstructor import dgemm_dev, sgemm_dev
 
 pytestmark = pytest.mark.gpu
 
@@ -215,6 +215,7 @@ def test_few_rows_of_the_split_bf16_product(transb):
     """The split-BF16 product of few rows (16- or 32-row workgroups without LDS) has the bits of those
     rows in a product large enough for the staged kernel: K below, at and past whole chunks of 32
     and flushes of 256, ragged columns, beta = 0 and 1."""
+    from moao_amd.reconstructor import sgemm_bf16x3_dev
     rng = np.random.default_rng(30 + transb)
     big = 16000
     for N, K in [(128, 128), (131, 300), (97, 31), (128, 600)]:
