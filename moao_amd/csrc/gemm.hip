@@ -504,31 +504,6 @@ __global__ void __launch_bounds__(NT, TM == 128 ? 2 : 4) gemm_dl_kernel(GemmArgs
     }
 }
 
-// hi and lo planes of four consecutive k of one row, those below N (see Planes).
-__device__ __forceinline__ void write_planes(const float (&v)[4], unsigned short* hi, long ps,
-                                             int k, int N) {
-    typedef unsigned short us4 __attribute__((ext_vector_type(4)));
-    us4 h, l;
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-        const __bf16 a = (__bf16)v[t];
-        h[t] = __builtin_bit_cast(unsigned short, a);
-        l[t] = __builtin_bit_cast(unsigned short, (__bf16)(v[t] - (float)a));
-    }
-    if (k + 4 <= N) {
-        *(us4*)(hi + k) = h;
-        *(us4*)(hi + ps + k) = l;
-        return;
-    }
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-        if (k + t < N) {
-            hi[k + t] = h[t];
-            hi[ps + k + t] = l[t];
-        }
-}
-__device__ __forceinline__ void write_planes(const double (&)[4], unsigned short*, long, int, int) {}
-
 // Direct kernel for launches too small to hide the slice pipeline above: a K = 128 product is
 // 16 slices there, each a barrier and a share of the load latency.  Here no LDS and no barrier
 // stand between the loads and the MFMAs: every wave loads its A and op(B) fragments from global

@@ -1,4 +1,5 @@
-// 16x16x4 MFMA steps and the lane exchange that feeds them from memory order (gfx950).
+// 16x16x4 MFMA steps, the lane exchange that feeds them from memory order, and the split-BF16 planes
+// of what they leave (gfx950).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -60,6 +61,31 @@ __device__ __forceinline__ void lane_rows_transpose(T& a, T& b, T& c, T& d) {
     __builtin_memcpy(&c, v[2], sizeof(T));
     __builtin_memcpy(&d, v[3], sizeof(T));
 }
+
+// hi and lo planes of four consecutive k of one row, those below N (see Planes).
+__device__ __forceinline__ void write_planes(const float (&v)[4], unsigned short* hi, long ps,
+                                             int k, int N) {
+    typedef unsigned short us4 __attribute__((ext_vector_type(4)));
+    us4 h, l;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        const __bf16 a = (__bf16)v[t];
+        h[t] = __builtin_bit_cast(unsigned short, a);
+        l[t] = __builtin_bit_cast(unsigned short, (__bf16)(v[t] - (float)a));
+    }
+    if (k + 4 <= N) {
+        *(us4*)(hi + k) = h;
+        *(us4*)(hi + ps + k) = l;
+        return;
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+        if (k + t < N) {
+            hi[k + t] = h[t];
+            hi[ps + k + t] = l[t];
+        }
+}
+__device__ __forceinline__ void write_planes(const double (&)[4], unsigned short*, long, int, int) {}
 
 }  // namespace
 }  // namespace moao

@@ -185,18 +185,27 @@ int trsmN_rec(const Tall<T>& p, long j0, long nn) {
             return rc;
         return MOAO_OK;
     }
-    // Segments in one launch, up to the rows where the launches' reuse of their operands wins.  n =
+    // Segments in one launch (with split-BF16 updates too: inside a segment they run in FP32), up to the rows where the launches' reuse of their operands wins.  n =
     // 2,048, launches -> segments, us: FP64 16 rows 1303 -> 1200, 1000 1362 -> 1248, 4000 1874 -> 1747,
     // 8000 2513 -> 2494, 16000 3841 -> 3910; FP32 16 rows 1116 -> 1023, 16000 2659 -> 2599, 32000 4165 ->
     // 4134.
     long rows_all = 0;
     for (const auto& g : G) rows_all += g.rows;
-    if (!p.sw && nn <= kSegment && nn % kLeaf == 0 && rows_all <= (sizeof(T) == 8 ? 8192 : 16384)) {
+    if (nn <= kSegment && nn % kLeaf == 0 && rows_all <= (sizeof(T) == 8 ? 8192 : 16384)) {
         for (size_t q = 0; q < G.size();) {
             SegRows<T> rows[kSegGroups];
             int ns = 0;
             for (; q < G.size() && ns < kSegGroups; ++q)
-                if (G[q].rows > 0) rows[ns++] = {G[q].p + j0 * G[q].ld, G[q].ld, G[q].rows};
+                if (G[q].rows > 0) {
+                    rows[ns] = {G[q].p + j0 * G[q].ld, G[q].ld, G[q].rows, nullptr, 0, 0};
+                    if (p.sw) {
+                        const Planes x = p.sw->x_rows(j0);
+                        rows[ns].cp = const_cast<unsigned short*>(x.hi);
+                        rows[ns].cpld = x.ld;
+                        rows[ns].cpps = x.ps;
+                    }
+                    ++ns;
+                }
             if (ns)
                 if (int rc = trsm_segment<T>(rows, ns, p.a(j0, j0), p.lda, p.inv(j0), (int)nn,
                                              p.skip, p.s))

@@ -66,6 +66,10 @@ __global__ void __launch_bounds__(512) trsm_segment_kernel(SegArgs<T> a) {
         T* X = g.X + row + (long)leaf * kLeaf * g.ld;
 #pragma unroll
         for (int t = 0; t < 4; ++t) X[(long)(16 * w + M::row(lane, t)) * g.ld] = x[t];
+        if constexpr (sizeof(T) == 4)  // a lane's 4 columns are 4 consecutive k of a plane row
+            if (g.cp)
+                write_planes(x, g.cp + (long)row * g.cpld, g.cpps, leaf * kLeaf + 16 * w + 4 * lq,
+                             (leaf + 1) * kLeaf);
     };
 
     // 128 k of op(B) for the wave's columns: lane (column li, k = 16 c + 4 lq ..) of column-major B;

@@ -14,6 +14,9 @@ struct SegRows {
     T* X;
     long ld;
     int rows;
+    // FP32, optional: the split-BF16 planes of the result (gemm.hpp's Planes), column 0 at cp
+    unsigned short* cp;
+    long cpld, cpps;
 };
 
 // L: the segment's diagonal block of the factor (leading dimension lda, lower triangle), inv: the
