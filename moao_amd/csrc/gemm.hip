@@ -1180,7 +1180,15 @@ int launch(const GemmArgs<T>& g, hipStream_t stream) {
     }
     // the K x N slab loads address 128 columns with 32-bit byte offsets
     const bool kn_offsets_fit = (long)BN * g.ldb * (long)sizeof(T) < (1L << 31);
-    if (g.transb < 2 && (g.transb == 1 || kn_offsets_fit)) {
+    // the direct kernel's lane offsets are 32-bit bytes: A reaches 3 columns and 31 rows from its
+    // base, B^T 3 columns and 127 rows.  Past those the slice kernel, whose columns have 64-bit bases.
+    auto lanes_reach = [](long ld, int rows) {
+        return ld < (1L << 32) && (3 * ld + rows) * (long)sizeof(T) < (1L << 32);
+    };
+    bool direct_offsets_fit = g.transb == 1 ? lanes_reach(g.ldb, BN - 1) : kn_offsets_fit;
+    for (int i = 0; i < g.nseg; ++i)
+        direct_offsets_fit = direct_offsets_fit && lanes_reach(g.seg[i].lda, 31);
+    if (g.transb < 2 && direct_offsets_fit) {
         if (const int rows = direct_rows(g, cells)) {
             grid.x = (maxM + rows - 1) / rows;
             auto k = g.transb == 1 ? (rows == 16 ? gemm_direct_kernel<T, 1, 1, 4>

@@ -1,0 +1,235 @@
+// Runs the library's host code without a GPU: this program defines the HIP functions that the
+// library calls, and the loader binds the library to them.  Device memory is a range of addresses
+// that nothing may touch, allocations are counted and may be refused, launches are printed with
+// the kernel's name and grid.  Copies to the host deliver zeros.
+#include <cxxabi.h>
+#include <hip/hip_runtime_api.h>
+
+#include <algorithm>
+#include <atomic>
+#include <chrono>
+#include <cmath>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <mutex>
+#include <new>
+#include <string>
+#include <thread>
+#include <vector>
+
+#include "gemm.hpp"
+#include "moao_hip.h"
+#include "recon.hpp"
+#include "stages.hpp"
+
+namespace {
+
+std::map<const void*, std::string>& kernels() {
+    static std::map<const void*, std::string> k;
+    return k;
+}
+std::mutex mu;
+bool show = true;          // print launches
+long launches = 0;
+size_t limit = SIZE_MAX;   // bytes a single stream-ordered allocation may ask for
+struct Pool {
+    size_t live = 0, peak = 0;
+    std::map<void*, size_t> blocks;
+};
+Pool pool, heap;           // stream-ordered, hipMalloc
+char* next_address = reinterpret_cast<char*>(1L << 44);
+
+hipError_t take(Pool& p, void** ptr, size_t bytes) {
+    std::lock_guard<std::mutex> g(mu);
+    *ptr = next_address;
+    next_address += (bytes + 4095) & ~size_t(4095);
+    p.blocks[*ptr] = bytes;
+    p.live += bytes;
+    p.peak = std::max(p.peak, p.live);
+    return hipSuccess;
+}
+hipError_t give(Pool& p, void* ptr) {
+    std::lock_guard<std::mutex> g(mu);
+    auto it = p.blocks.find(ptr);
+    if (ptr && it == p.blocks.end()) {
+        std::printf("free of an unknown block\n");
+        std::exit(3);
+    }
+    if (ptr) {
+        p.live -= it->second;
+        p.blocks.erase(it);
+    }
+    return hipSuccess;
+}
+
+// bytes of the C++ heap in use by what runs between the two readings of heap_peak
+std::atomic<long> cpp_live{0}, cpp_peak{0};
+
+}  // namespace
+
+void* operator new(size_t n) {
+    void* p = std::malloc(n + 16);
+    if (!p) throw std::bad_alloc();
+    *static_cast<size_t*>(p) = n;
+    const long live = cpp_live += (long)n;
+    long peak = cpp_peak;
+    while (live > peak && !cpp_peak.compare_exchange_weak(peak, live)) {
+    }
+    return static_cast<char*>(p) + 16;
+}
+void operator delete(void* q) noexcept {
+    if (!q) return;
+    char* p = static_cast<char*>(q) - 16;
+    cpp_live -= (long)*reinterpret_cast<size_t*>(p);
+    std::free(p);
+}
+void operator delete(void* q, size_t) noexcept { operator delete(q); }
+
+extern "C" {
+
+void** __hipRegisterFatBinary(const void*) { static void* h; return &h; }
+void __hipUnregisterFatBinary(void**) {}
+void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
+void __hipRegisterFunction(void**, const void* host, char*, const char* name, unsigned, void*,
+                           void*, void*, void*, int*) {
+    int rc = 0;
+    char* d = abi::__cxa_demangle(name, nullptr, nullptr, &rc);
+    std::string s = rc == 0 ? d : name;
+    std::free(d);
+    // "void moao::(anonymous namespace)::kernel<args>(parameters)" -> "kernel<args>"
+    if (s.compare(0, 5, "void ") == 0) s.erase(0, 5);
+    const std::string ns = "moao::(anonymous namespace)::";
+    if (s.compare(0, ns.size(), ns) == 0) s.erase(0, ns.size());
+    int depth = 0;
+    for (size_t k = 0; k < s.size(); ++k) {
+        if (s[k] == '<') ++depth;
+        if (s[k] == '>') --depth;
+        if (s[k] == '(' && depth == 0) {
+            s.resize(k);
+            break;
+        }
+    }
+    kernels()[host] = s;
+}
+hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t);
+static thread_local dim3 cfg_grid, cfg_block;
+hipError_t __hipPushCallConfiguration(dim3 grid, dim3 block, size_t, hipStream_t) {
+    cfg_grid = grid;
+    cfg_block = block;
+    return hipSuccess;
+}
+hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* shared, hipStream_t* s) {
+    *grid = cfg_grid;
+    *block = cfg_block;
+    *shared = 0;
+    *s = nullptr;
+    return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void* f, dim3 g, dim3 b, void**, size_t, hipStream_t) {
+    std::lock_guard<std::mutex> l(mu);
+    ++launches;
+    if (!g.x || !g.y || !g.z || g.y > 65535 || g.z > 65535 || b.x * b.y * b.z > 1024) {
+        std::printf("impossible launch of %s\n", kernels()[f].c_str());
+        std::exit(3);
+    }
+    if (show) std::printf("launch %s %u %u %u\n", kernels()[f].c_str(), g.x, g.y, g.z);
+    return hipSuccess;
+}
+hipError_t hipMalloc(void** p, size_t n) { return take(heap, p, n); }
+hipError_t hipFree(void* p) { return give(heap, p); }
+hipError_t hipMallocAsync(void** p, size_t n, hipStream_t) {
+    const bool ok = n <= limit;
+    if (show) std::printf("async %zu %s\n", n, ok ? "given" : "refused");
+    return ok ? take(pool, p, n) : hipErrorOutOfMemory;
+}
+hipError_t hipFreeAsync(void* p, hipStream_t) { return give(pool, p); }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+    *p = std::malloc(n);
+    return *p ? hipSuccess : hipErrorOutOfMemory;
+}
+hipError_t hipHostFree(void* p) {
+    std::free(p);
+    return hipSuccess;
+}
+hipError_t hipMemcpy(void* d, const void*, size_t n, hipMemcpyKind k) {
+    if (k == hipMemcpyDeviceToHost) std::memset(d, 0, n);
+    return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind k, hipStream_t) {
+    return hipMemcpy(d, s, n, k);
+}
+hipError_t hipMemcpy2DAsync(void*, size_t, const void*, size_t, size_t, size_t, hipMemcpyKind,
+                            hipStream_t) {
+    return hipSuccess;
+}
+hipError_t hipMemset(void*, int, size_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipDeviceSynchronize() { return hipSuccess; }
+hipError_t hipGetLastError() { return hipSuccess; }
+const char* hipGetErrorString(hipError_t) { return "refused"; }
+hipError_t hipGetDeviceCount(int* n) {
+    *n = 1;
+    return hipSuccess;
+}
+hipError_t hipGetDevice(int* d) {
+    *d = 0;
+    return hipSuccess;
+}
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600* p, int) {
+    std::memset(p, 0, sizeof *p);
+    std::strcpy(p->gcnArchName, "gfx950");
+    return hipSuccess;
+}
+hipError_t hipGetSymbolAddress(void** p, const void*) {
+    *p = reinterpret_cast<void*>(1L << 43);
+    return hipSuccess;
+}
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
+    static std::atomic<long> k{1};
+    *s = reinterpret_cast<hipStream_t>(k++ << 8);
+    return hipSuccess;
+}
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* c) {
+    *c = hipStreamCaptureStatusNone;
+    return hipSuccess;
+}
+hipError_t hipMemGetInfo(size_t* f, size_t* t) {
+    *f = *t = size_t(256) << 30;
+    return hipSuccess;
+}
+hipError_t hipDeviceGetDefaultMemPool(hipMemPool_t* p, int) {
+    *p = nullptr;
+    return hipSuccess;
+}
+hipError_t hipMemPoolSetAttribute(hipMemPool_t, hipMemPoolAttr, void*) { return hipSuccess; }
+
+}  // extern "C"
+
+namespace {
+
+double* at(long k) { return reinterpret_cast<double*>((1L << 42) + (k << 36)); }
+
+// <f64|f32> transb M N K lda ldb
+int run_gemm(char** a) {
+    const int tb = std::atoi(a[1]), M = std::atoi(a[2]), N = std::atoi(a[3]), K = std::atoi(a[4]);
+    const long lda = std::atol(a[5]), ldb = std::atol(a[6]);
+    if (std::string(a[0]) == "f64")
+        return moao_hip_dgemm_dev(tb, M, N, K, 1.0, at(1), lda, at(2), ldb, 1.0, at(3), M, nullptr);
+    return moao_hip_sgemm_dev(tb, M, N, K, 1.0f, (float*)at(1), lda, (float*)at(2), ldb, 1.0f,
+                              (float*)at(3), M, nullptr);
+}
+
+}  // namespace
+
+int main(int argc, char** argv) {
+    const std::string cmd = argc > 1 ? argv[1] : "";
+    int rc = 2;
+    if (const char* l = std::getenv("ASYNC_LIMIT")) limit = std::strtoull(l, nullptr, 10);
+    if (cmd == "gemm" && argc == 9) rc = run_gemm(argv + 2);
+    std::printf("rc %d\n", rc);
+    return rc == 2;
+}

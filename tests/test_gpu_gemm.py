@@ -235,3 +235,35 @@ def test_few_rows_of_the_split_bf16_product(transb):
                 got = dC.to_host()
                 assert np.array_equal(got[:r], want[:r])
                 assert np.array_equal(got[r:], C[r:])
+
+
+@pytest.mark.parametrize("dtype,transb,lda,ldb", [
+    (np.float64, 1, 179_000_000, 20), (np.float64, 0, 179_000_000, 20),
+    (np.float64, 1, 20, 179_000_000), (np.float32, 1, 358_000_000, 21)])
+def test_small_product_of_very_tall_buffers(dtype, transb, lda, ldb):
+    """20 x 20 x 5 products whose operands are the first rows of buffers so tall that 3 columns span
+    more than 4 GiB: offsets of 32 bits would read other rows.  Tolerance: K products of values
+    below 1, each rounded once and added once."""
+    from moao_amd.lib import check, lib
+    import ctypes
+    print(f"[gemm-tall] {dtype.__name__} transb={transb} lda={lda} ldb={ldb}", flush=True)
+    rng = np.random.default_rng(5)
+    M = N = 20
+    K = 5
+
+    def tall(rows, cols, ld):
+        a = np.asfortranarray(rng.uniform(-1, 1, (rows, cols)).astype(dtype))
+        d = DeviceArray((ld, cols), dtype)
+        for c in range(cols):
+            check(lib().moao_hip_memcpy_h2d(ctypes.c_void_p(d.ptr + c * ld * a.itemsize),
+                                            a[:, c].copy().ctypes.data, rows * a.itemsize), "h2d")
+        return a, d
+    A, dA = tall(M, K, lda)
+    B, dB = tall(N if transb == 1 else K, K if transb == 1 else N, ldb)
+    dC = DeviceArray.from_host(np.zeros((M, N), dtype, order="F"))
+    f = dgemm_dev if dtype == np.float64 else sgemm_dev
+    f(transb, M, N, K, 1.0, dA.ptr, lda, dB.ptr, ldb, 0.0, dC.ptr, M)
+    ref = A.astype(np.float64) @ (B.T if transb == 1 else B).astype(np.float64)
+    assert np.max(np.abs(dC.to_host() - ref)) <= 2 * K * np.finfo(dtype).eps
+    dA.free()
+    dB.free()
