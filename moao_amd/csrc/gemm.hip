@@ -1255,14 +1255,16 @@ int split_planes(const float* A, long lda, int rows, int cols, unsigned short* h
 }
 
 void sym_alloc(SymWork& w, long rows, long K, hipStream_t s) {
-    // in full where that stays below 4 GB, else as many columns at a time as do; for few rows
-    // the diagonal blocks
-    const long cols = rows < kSymRows ? 0 : std::min<long>(K, (1L << 29) / K / BN * BN);
-    const long elems = cols ? K * cols : (K + BN - 1) / BN * BN * BN;
-    if (hipMallocAsync(reinterpret_cast<void**>(&w.p), sizeof(double) * elems, s) != hipSuccess) {
+    // in full where that stays below 4 GB, else as many columns at a time as do; for few rows, or
+    // where that much is not to be had, the diagonal blocks
+    long cols = rows < kSymRows ? 0 : std::min<long>(K, (1L << 29) / K / BN * BN);
+    for (;; cols = 0) {
+        const long elems = cols ? K * cols : (K + BN - 1) / BN * BN * BN;
+        if (hipMallocAsync(reinterpret_cast<void**>(&w.p), sizeof(double) * elems, s) == hipSuccess)
+            break;
         w.p = nullptr;
         (void)hipGetLastError();
-        return;
+        if (!cols) return;
     }
     w.s = s;
     w.cols = (int)cols;

@@ -88,7 +88,8 @@ struct SymWork {
     SymWork& operator=(const SymWork&) = delete;
     ~SymWork();
 };
-// Allocates for products of `rows` rows with a K x K matrix; leaves w empty where it cannot.
+// Allocates for products of `rows` rows with a K x K matrix: the first that the pool has of the
+// matrix in full and its blocks; leaves w empty where it has neither.
 void sym_alloc(SymWork& w, long rows, long K, hipStream_t s);
 // The transb = 2 product, through w where it has room, else on the fallback kernel.
 int gemm_sym(const GemmArgs<double>& a, SymWork& w, hipStream_t stream);

@@ -56,3 +56,19 @@ def test_direct_kernel_keeps_to_its_32_bit_offsets(host, prec, transb):
     if transb == 1:
         assert kernel(20, B_FIT[prec]) == ["gemm_direct_kernel"]
         assert kernel(20, B_FIT[prec] + 1) == ["gemm_dl_kernel"]
+
+
+def test_symmetric_operand_without_room_for_all_of_it(host):
+    """The symmetric operand is written out in full where that scratch is to be had; else its diagonal
+    blocks serve, and only without those does the product take the register-staged kernel."""
+    K, full, blocks = 2000, 8 * 2000 * 2000, 8 * 128 * 2048
+    for lim, want in ((full, ["expand_sym_kernel", "gemm_dl_kernel"]),
+                      (full - 1, ["symdiag_kernel", "gemm_dl_kernel"]),
+                      (blocks, ["symdiag_kernel", "gemm_dl_kernel"]),
+                      (blocks - 1, ["gemm_kernel"])):
+        out = host("gemm", "f64", 2, 3000, K, K, 3000, K, ASYNC_LIMIT=lim)
+        got = kernels(out)
+        assert [k for k, _ in got] == want, (lim, out)
+        if lim < full and lim >= blocks:
+            assert got[-1][1][:2] == ["double", "2"]
+        assert out[-1] == ["rc", "0"]
