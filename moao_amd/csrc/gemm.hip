@@ -1254,24 +1254,37 @@ int split_planes(const float* A, long lda, int rows, int cols, unsigned short* h
     return MOAO_OK;
 }
 
+// Columns written out at a time: all where that stays below 4 GB, else as many as do; 0, the
+// diagonal blocks, for few rows.
+static long sym_cols(long rows, long K) {
+    return rows < kSymRows ? 0 : std::min<long>(K, (1L << 29) / K / BN * BN);
+}
+
+size_t sym_bytes(long rows, long K) {
+    const long cols = sym_cols(rows, K);
+    return sizeof(double) * (cols ? K * cols : (K + BN - 1) / BN * BN * BN);
+}
+
+void sym_place(SymWork& w, long rows, long K, void* mem, size_t bytes) {
+    w.p = static_cast<double*>(mem);
+    w.cols = bytes >= sym_bytes(rows, K) ? (int)sym_cols(rows, K) : 0;
+}
+
 void sym_alloc(SymWork& w, long rows, long K, hipStream_t s) {
-    // in full where that stays below 4 GB, else as many columns at a time as do; for few rows, or
-    // where that much is not to be had, the diagonal blocks
-    long cols = rows < kSymRows ? 0 : std::min<long>(K, (1L << 29) / K / BN * BN);
-    for (;; cols = 0) {
-        const long elems = cols ? K * cols : (K + BN - 1) / BN * BN * BN;
-        if (hipMallocAsync(reinterpret_cast<void**>(&w.p), sizeof(double) * elems, s) == hipSuccess)
-            break;
-        w.p = nullptr;
+    for (const size_t bytes : {sym_bytes(rows, K), sym_least_bytes(K)}) {
+        void* mem = nullptr;
+        if (hipMallocAsync(&mem, bytes, s) == hipSuccess) {
+            sym_place(w, rows, K, mem, bytes);
+            w.s = s;
+            w.own = true;
+            return;
+        }
         (void)hipGetLastError();
-        if (!cols) return;
     }
-    w.s = s;
-    w.cols = (int)cols;
 }
 
 SymWork::~SymWork() {
-    if (p) (void)hipFreeAsync(p, s);
+    if (own) (void)hipFreeAsync(p, s);
 }
 
 int gemm_sym(const GemmArgs<double>& a, SymWork& w, hipStream_t stream) {

@@ -76,11 +76,13 @@ struct GemmArgs {
 // out in full, so that they run on the kernel for op(B) = B^T; with fewer, full copies of its 128 x
 // 128 diagonal blocks, with which a kernel reads the lower triangle in place, columns above the
 // diagonal and rows below it.  K = 18,688, in place -> in full: 256 rows 4.1 -> 5.3 ms, 512 rows
-// 9.8 -> 7.6, 8 x 2,336 rows 213 -> 187.  Stream-ordered, for one matrix and one caller's scope.
+// 9.8 -> 7.6, 8 x 2,336 rows 213 -> 187.  For one matrix and one caller's scope; stream-ordered
+// (sym_alloc) or in the caller's memory (sym_place).
 constexpr long kSymRows = 448;
 struct SymWork {
     double* p = nullptr;
     hipStream_t s = nullptr;
+    bool own = false;   // from sym_alloc
     int cols = 0;       // columns written out at a time; 0: diagonal blocks
     bool held = false;  // the whole matrix, or its blocks, are there
     SymWork() = default;
@@ -91,6 +93,11 @@ struct SymWork {
 // Allocates for products of `rows` rows with a K x K matrix: the first that the pool has of the
 // matrix in full and its blocks; leaves w empty where it has neither.
 void sym_alloc(SymWork& w, long rows, long K, hipStream_t s);
+// Bytes that serve products of `rows` rows best, and the least that serve them (the blocks).
+size_t sym_bytes(long rows, long K);
+inline size_t sym_least_bytes(long K) { return sym_bytes(1, K); }
+// The same in `bytes` of device memory at mem, at least sym_least_bytes(K), for work on one stream.
+void sym_place(SymWork& w, long rows, long K, void* mem, size_t bytes);
 // The transb = 2 product, through w where it has room, else on the fallback kernel.
 int gemm_sym(const GemmArgs<double>& a, SymWork& w, hipStream_t stream);
 

@@ -236,9 +236,9 @@ struct MixedWs {
 // Leading dimension of the split-BF16 planes of an order-n solve.
 static long plane_ld(long n) { return (n + 63) / 64 * 64; }
 
-// Byte offsets of the workspace pieces (MixedWs order, then the symmetric diagonal blocks and,
-// for the BF16 mode, the planes of L in both orientations and of the right-hand sides) and the
-// total size.
+// Byte offsets of the workspace pieces (MixedWs order, then for the BF16 mode the planes of L in
+// both orientations and of the right-hand sides, last the scratch of the residuals' symmetric
+// operand, which may be longer) and the least total size.
 static size_t mixed_layout(long n, long m, int p, int mode, std::vector<size_t>* offs) {
     const long xr = m + p;
     const long q = std::max(p, 1);
@@ -269,11 +269,17 @@ static size_t mixed_layout(long n, long m, int p, int mode, std::vector<size_t>*
         take(sizeof(unsigned short) * 2 * n * ld);   // L, plane row = column
         take(sizeof(unsigned short) * 2 * xr * ld);  // right-hand sides
     }
+    take(sym_least_bytes(n));
     return off;
 }
 
 size_t mixed_workspace_bytes(long n, long m, const moao_tomo_view* lowrank, int mode) {
     return mixed_layout(n, m, lowrank_ranges(lowrank, n).p(), mode, nullptr);
+}
+
+size_t mixed_spare_bytes(long n, long m) {
+    const size_t best = sym_bytes(m, n), least = sym_least_bytes(n);
+    return best > least ? best - least : 0;
 }
 
 int reconstructor_mixed_dev(long n, long m, const double* Cmm, long ldCmm, double* Ctm, long ldCtm,
@@ -432,10 +438,10 @@ int reconstructor_mixed_dev(long n, long m, const double* Cmm, long ldCmm, doubl
         std::fprintf(stderr, "[mixed] |Z|=%.6e |Z2|=%.6e |R0|=%.6e\n", a, b2, c2);
     }
 
-    // --- 4. refinement (the residual's symmetric operand Cmm written out in full where there is
-    // room)
+    // --- 4. refinement (the residual's symmetric operand Cmm written out in full where the
+    // workspace has room)
     SymWork sym;
-    sym_alloc(sym, m, n, s);
+    sym_place(sym, m, n, b + offs.back(), ws_bytes - offs.back());
     double rel = 0;
     int it = 0;
     int status = MOAO_OK;
@@ -492,15 +498,19 @@ int moao_hip_reconstructor_mixed_dev(long nmeas, long nmeasts, const double* dCm
         moao::set_error("reconstructor_mixed: invalid arguments");
         return MOAO_ERR_ARG;
     }
-    // workspace of this call only, from the stream-ordered pool
+    // workspace of this call only, from the stream-ordered pool; the least where more is not to be had
     hipStream_t s = moao::pick_stream(stream);
-    const size_t bytes = moao::mixed_workspace_bytes(nmeas, nmeasts, lowrank, mode);
+    const size_t least = moao::mixed_workspace_bytes(nmeas, nmeasts, lowrank, mode);
+    size_t bytes = least + moao::mixed_spare_bytes(nmeas, nmeasts);
     void* ws = nullptr;
-    if (hipMallocAsync(&ws, bytes, s) != hipSuccess) {
+    while (hipMallocAsync(&ws, bytes, s) != hipSuccess) {
         (void)hipGetLastError();
-        moao::set_error("reconstructor_mixed: workspace allocation of " + std::to_string(bytes) +
-                        " B failed");
-        return MOAO_ERR_NOMEM;
+        if (bytes == least) {
+            moao::set_error("reconstructor_mixed: workspace allocation of " +
+                            std::to_string(bytes) + " B failed");
+            return MOAO_ERR_NOMEM;
+        }
+        bytes = least;
     }
     int rc = moao::reconstructor_mixed_dev(nmeas, nmeasts, dCmm, ldCmm, dCtm, ldCtm, lowrank, mode,
                                            tol, max_iter, resid, iters, ws, bytes, s);

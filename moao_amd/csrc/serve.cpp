@@ -4,7 +4,8 @@
 // atmospheric profile).  A serving deployment instead receives solves for new profiles and for
 // systems of uneven size while earlier ones are still on the device.  Here:
 //   * submit() builds the request's Tomo on the caller's thread (host work, no GPU), which fixes
-//     n and m and so the request's HBM footprint, and queues it;
+//     n and m and so the request's HBM footprint, and queues it (a mixed solve runs faster with
+//     more: it gets that where no other request can want the memory);
 //   * `slots` worker threads, each with its own HIP stream and scratch, take requests from the
 //     queue as soon as a slot is free AND the footprint fits in the byte budget (first fit in
 //     arrival order; a request passed over max_bypass times blocks later ones until it fits, so
@@ -79,7 +80,9 @@ struct Request {
     long ldR = 0;
     long n = 0, m = 0;
     size_t solve_bytes = 0;  // scratch of the solve (inverse leaves or mixed workspace)
-    size_t footprint = 0;
+    size_t footprint = 0;    // bytes it is admitted with
+    size_t spare = 0;        // bytes beyond them that a mixed solve makes use of
+    size_t held = 0;         // bytes it runs with
     int bypassed = 0;
     bool done = false;
     moao_serve_result res{};
@@ -133,6 +136,14 @@ struct moao_server {
         }
         return nullptr;
     }
+    // Bytes an admitted request runs with: its spare ones too where that leaves every idle slot
+    // room for the largest request in sight.  Called with mu held.
+    size_t grant(const moao::Request& r) const {
+        size_t most = r.footprint;
+        for (const moao::Request* q : queue) most = std::max(most, q->footprint);
+        const size_t idle = slots.size() - running - 1, left = budget - in_use - r.footprint;
+        return r.footprint + (left >= r.spare && (left - r.spare) / most >= idle ? r.spare : 0);
+    }
     void worker(int k);
     int run(moao::Request& r, moao::Slot& s);
     int run_body(moao::Request& r, moao::Slot& s);
@@ -149,10 +160,14 @@ int moao_server::run_body(moao::Request& r, moao::Slot& sl) {
     hipStream_t s = sl.stream;
     const long n = r.n, m = r.m;
     char* block = nullptr;
-    if (hipMallocAsync(reinterpret_cast<void**>(&block), r.footprint, s) != hipSuccess) {
+    size_t held = r.held;
+    while (hipMallocAsync(reinterpret_cast<void**>(&block), held, s) != hipSuccess) {
         (void)hipGetLastError();
-        set_error("serve: device allocation of " + std::to_string(r.footprint) + " B failed");
-        return MOAO_ERR_NOMEM;
+        if (held == r.footprint) {
+            set_error("serve: device allocation of " + std::to_string(r.footprint) + " B failed");
+            return MOAO_ERR_NOMEM;
+        }
+        held = r.footprint;  // the spare bytes are not to be had
     }
     double* Cmm = reinterpret_cast<double*>(block);
     double* Ctm = reinterpret_cast<double*>(block + al256(sizeof(double) * n * n));
@@ -211,7 +226,7 @@ int moao_server::run_body(moao::Request& r, moao::Slot& sl) {
             int iters = 0;
             rc = reconstructor_mixed_dev(n, m, Cmm, n, Ctm, m, &r.view, r.mode, r.tol, r.max_iter,
                                          &resid,
-                                         &iters, scratch, r.solve_bytes, s);
+                                         &iters, scratch, r.solve_bytes + (held - r.footprint), s);
             r.res.resid = resid;
             r.res.iters = iters;
         }
@@ -250,7 +265,8 @@ void moao_server::worker(int k) {
         moao::Request* r = nullptr;
         cv_work.wait(lk, [&] { return stop || (r = pick()) != nullptr; });
         if (!r) return;  // stop with nothing admissible
-        in_use += r->footprint;
+        r->held = r->res.footprint = grant(*r);
+        in_use += r->held;
         peak_bytes = std::max(peak_bytes, in_use);
         ++running;
         peak_running = std::max(peak_running, running);
@@ -261,7 +277,7 @@ void moao_server::worker(int k) {
         lk.lock();
         r->res.t_end = now();
         r->res.status = rc;
-        in_use -= r->footprint;
+        in_use -= r->held;
         --running;
         ++completed;
         r->done = true;
@@ -356,9 +372,9 @@ int moao_serve_submit(moao_server* s, const moao_serve_request* q, long* ticket)
                                           : moao::mixed_workspace_bytes(r->n, r->m, &r->view, r->mode);
     r->footprint = moao::al256(sizeof(double) * r->n * r->n) +
                    moao::al256(sizeof(double) * r->m * r->n) + moao::al256(r->solve_bytes);
+    if (r->mode != MOAO_FP64) r->spare = moao::mixed_spare_bytes(r->n, r->m);
     r->res.n = r->n;
     r->res.m = r->m;
-    r->res.footprint = r->footprint;
     r->res.t_submit = t_submit;
     std::lock_guard<std::mutex> g(s->mu);
     if (r->footprint > s->budget) {

@@ -15,6 +15,7 @@
 #include <map>
 #include <mutex>
 #include <new>
+#include <set>
 #include <string>
 #include <thread>
 #include <vector>
@@ -32,7 +33,7 @@ std::map<const void*, std::string>& kernels() {
 }
 std::mutex mu;
 bool show = true;          // print launches
-long launches = 0;
+std::set<std::string> launched;
 size_t limit = SIZE_MAX;   // bytes a single stream-ordered allocation may ask for
 struct Pool {
     size_t live = 0, peak = 0;
@@ -129,7 +130,7 @@ hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* shared, hi
 }
 hipError_t hipLaunchKernel(const void* f, dim3 g, dim3 b, void**, size_t, hipStream_t) {
     std::lock_guard<std::mutex> l(mu);
-    ++launches;
+    launched.insert(kernels()[f]);
     if (!g.x || !g.y || !g.z || g.y > 65535 || g.z > 65535 || b.x * b.y * b.z > 1024) {
         std::printf("impossible launch of %s\n", kernels()[f].c_str());
         std::exit(3);
@@ -223,6 +224,49 @@ int run_gemm(char** a) {
                               (float*)at(3), M, nullptr);
 }
 
+// n m <1 FP32 | 2 BF16>: a mixed solve in the least and in the best workspace; launches of both
+int run_mixed(char** a) {
+    const long n = std::atol(a[0]), m = std::atol(a[1]);
+    const int mode = std::atoi(a[2]);
+    const size_t least = moao::mixed_workspace_bytes(n, m, nullptr, mode);
+    std::printf("least %zu spare %zu\n", least, moao::mixed_spare_bytes(n, m));
+    for (const size_t ws : {least, least + moao::mixed_spare_bytes(n, m)}) {
+        std::printf("workspace %zu\n", ws);
+        if (int rc = moao::reconstructor_mixed_dev(n, m, at(1), n, at(2), m, nullptr, mode, 1e-11, 5,
+                                                   nullptr, nullptr, at(3), ws, nullptr))
+            return rc;
+    }
+    return moao_hip_reconstructor_mixed_dev(n, m, at(1), n, at(2), m, nullptr, mode, 1e-11, 5,
+                                            nullptr, nullptr, nullptr);
+}
+
+// sys atm mode slots budget requests: what the requests were said to hold and what they took
+int run_serve(char** a) {
+    show = false;
+    moao_serve_config cfg{std::atoi(a[3]), std::strtoull(a[4], nullptr, 10), 0};
+    moao_server* srv = nullptr;
+    if (int rc = moao_serve_create(&cfg, &srv)) return rc;
+    moao_serve_request q{};
+    q.sys_file = a[0];
+    q.atm_file = a[1];
+    q.mode = std::atoi(a[2]);
+    std::vector<long> tickets(std::atoi(a[5]));
+    for (long& t : tickets)
+        if (int rc = moao_serve_submit(srv, &q, &t)) return rc;
+    for (long t : tickets) {
+        moao_serve_result r{};
+        const int rc = moao_serve_wait(srv, t, &r);
+        std::printf("request status %d n %ld m %ld footprint %zu\n", rc, r.n, r.m, r.footprint);
+    }
+    moao_serve_counters c{};
+    moao_serve_stats(srv, &c);
+    std::printf("peak %zu taken %zu left %zu kept %zu\n", c.peak_bytes, pool.peak, pool.live,
+                heap.live);
+    for (auto& k : launched) std::printf("launched %s\n", k.c_str());
+    moao_serve_destroy(srv);
+    return 0;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -230,6 +274,8 @@ int main(int argc, char** argv) {
     int rc = 2;
     if (const char* l = std::getenv("ASYNC_LIMIT")) limit = std::strtoull(l, nullptr, 10);
     if (cmd == "gemm" && argc == 9) rc = run_gemm(argv + 2);
+    if (cmd == "mixed" && argc == 5) rc = run_mixed(argv + 2);
+    if (cmd == "serve" && argc == 8) rc = run_serve(argv + 2);
     std::printf("rc %d\n", rc);
     return rc == 2;
 }

@@ -72,3 +72,63 @@ def test_symmetric_operand_without_room_for_all_of_it(host):
         if lim < full and lim >= blocks:
             assert got[-1][1][:2] == ["double", "2"]
         assert out[-1] == ["rc", "0"]
+
+
+def _words(lines, first):
+    return [{w[k]: int(w[k + 1]) for k in range(len(w) % 2, len(w) - 1, 2)}
+            for w in lines if w[0] == first]
+
+
+@pytest.mark.parametrize("mode", [1, 2])
+@pytest.mark.parametrize("n,m", [(700, 300), (1500, 448), (2000, 900)])
+def test_mixed_solve_allocates_nothing_but_its_workspace(host, mode, n, m):
+    """The workspace that mixed_workspace_bytes names is all that a mixed solve takes: its residuals
+    run with the symmetric operand's diagonal blocks there, and with all of it in the larger
+    workspace; the entry that makes its own asks for the larger one, then for the least."""
+    out = host("mixed", n, m, mode)
+    least, spare = (_words([out[0]], out[0][0])[0][k] for k in ("least", "spare"))
+    assert spare == (max(0, 8 * n * n - 8 * 128 * -(-n // 128) * 128) if m >= 448 else 0)
+    parts = [k for k, w in enumerate(out) if w[0] == "workspace"]
+    asked = [w for w in out if w[0] == "async"]
+    assert asked == [["async", str(least + spare), "given"]]
+    assert out.index(asked[0]) > parts[1]
+    names = [[k for k, _ in kernels(out[a:b])] for a, b in
+             ((parts[0], parts[1]), (parts[1], out.index(asked[0])), (out.index(asked[0]), None))]
+    full = "expand_sym_kernel" if spare else "symdiag_kernel"
+    assert "symdiag_kernel" in names[0] and "gemm_kernel" not in names[0]
+    assert full in names[1] and full in names[2]
+    if spare:
+        out = host("mixed", n, m, mode, ASYNC_LIMIT=least)
+        assert [w[2] for w in out if w[0] == "async"] == ["refused", "given"]
+        assert out[-1] == ["rc", "0"]
+        out = host("mixed", n, m, mode, ASYNC_LIMIT=least - 1)
+        assert out[-1] == ["rc", "-3"]
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_served_requests_hold_what_they_say(host, tmp_path, mode):
+    """All device memory that the requests take from the pool is in their footprints and so in the
+    budget; a mixed solve's spare bytes are given with a wide budget and not at the cost of another
+    request's place, and a budget of one plain request still serves it."""
+    from moao_amd import systems
+    s, a = systems.make_system(str(tmp_path), systems.SystemSpec(diam=8.0, nssp=24, nlgs=2, nngs=1,
+                                                                 nlayer=2, seed=3))
+    def serve(slots, budget, requests):
+        out = host("serve", s, a[0], mode, slots, budget, requests)
+        assert all(w[:3] == ["request", "status", "0"] for w in out if w[0] == "request"), out
+        return (_words(out, "request"), _words(out, "peak")[0],
+                {w[1].split("<")[0] for w in out if w[0] == "launched"})
+    req, mem, names = serve(1, 0, 1)
+    assert req[0]["m"] >= 448  # rows from which the residuals use the whole operand
+    assert mem["taken"] <= mem["peak"] == req[0]["footprint"]
+    assert ("expand_sym_kernel" in names) == (mode != 0)
+    wide = req[0]["footprint"]
+    n = req[0]["n"]
+    plain = wide - (8 * n * n - 8 * 128 * -(-n // 128) * 128 if mode else 0)
+    for slots, budget in ((1, plain), (1, max(plain, wide - 1)), (2, 2 * plain),
+                          (4, wide + 3 * plain - (1 if mode else 0))):
+        req, mem, names = serve(slots, budget, 6)
+        assert mem["taken"] <= mem["peak"] <= budget
+        assert all(r["footprint"] in (plain, wide) for r in req)
+        if slots < 4:
+            assert all(r["footprint"] == plain for r in req)
