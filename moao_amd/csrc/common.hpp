@@ -36,7 +36,11 @@ struct DevBuf {
 
 // What matcov uploads for a call (pinned host staging and its device copy) and, behind it on the
 // device, the covariance tables it computes there.  Grows on demand, used by one call at a time.
+// With `space`, device memory of the caller's that is free during the call, the covariance tables
+// go there, and the call does without where they don't fit.
 struct MatcovTables {
+    void* space = nullptr;
+    size_t space_bytes = 0;
     DevBuf dev;
     unsigned char* host = nullptr;
     size_t host_bytes = 0;

@@ -849,10 +849,11 @@ int matcov_tile_launch(double* d_data, int nrows, int ncols, int xoffset, int yo
                 }
             }
         // A table entry takes 9 structure functions a layer, an element on its own 3 or 4: tables
-        // where they are the smaller work (a tile of a few hundred elements is not), 256 MiB at most.
+        // where they are the smaller work (a tile of a few hundred elements is not), 256 MiB at most
+        // or what the caller has room for.
         const double W = 2.0 * lat.ext - 1;
-        if (slots.size() * W * W * 9 < 3.5 * nrows * ncols &&
-            slots.size() * W * W * 24 <= (256 << 20)) {
+        const double room = tables && tables->space ? tables->space_bytes : 256 << 20;
+        if (slots.size() * W * W * 9 < 3.5 * nrows * ncols && slots.size() * W * W * 24 <= room) {
             for (size_t k = 0; k < slots.size(); ++k)
                 cls[(slots[k] >> 8) * Nw + (slots[k] & 0xff)] = (int)k;
         } else {
@@ -969,7 +970,7 @@ int matcov_tile_launch(double* d_data, int nrows, int ncols, int xoffset, int yo
     a.v0 = (const double*)P(iV0);
     a.cls = (const int*)P(iCls);
     a.slots = (const int*)P(iSl);
-    a.ptab = (double*)(d + tables->upload);
+    a.ptab = (double*)(tables->space ? tables->space : d + tables->upload);
     a.Nw = Nw;
     a.ext = lat.ext;
 

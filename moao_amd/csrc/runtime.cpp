@@ -60,7 +60,7 @@ int MatcovTables::ensure(size_t upload_bytes, size_t table_bytes) {
         }
         host_bytes = upload;
     }
-    return dev.ensure(upload + table_bytes);
+    return dev.ensure(upload + (space ? 0 : table_bytes));
 }
 
 void MatcovTables::release() {

@@ -94,7 +94,7 @@ constexpr long kGraphMaxN = 16384;  // FP64 solves up to this order run as captu
 struct Slot {
     hipStream_t stream = nullptr;
     hipStream_t capture = nullptr;       // idle stream the slot records its graphs on
-    MatcovTables tables;                 // matcov upload and covariance tables (kept)
+    MatcovTables tables;                 // matcov upload (small, kept)
     std::unique_ptr<SolveGraph> graph;   // the graph of this slot's last captured solve
     struct {
         long n = 0, m = 0;
@@ -172,6 +172,9 @@ int moao_server::run_body(moao::Request& r, moao::Slot& sl) {
     double* Cmm = reinterpret_cast<double*>(block);
     double* Ctm = reinterpret_cast<double*>(block + al256(sizeof(double) * n * n));
     char* scratch = block + al256(sizeof(double) * n * n) + al256(sizeof(double) * m * n);
+    // the solve's scratch is free while matcov runs: its covariance tables go there
+    sl.tables.space = scratch;
+    sl.tables.space_bytes = held - (scratch - block);
     int rc = MOAO_OK;
     int hinfo = 0;
     do {

@@ -132,3 +132,18 @@ def test_served_requests_hold_what_they_say(host, tmp_path, mode):
         assert all(r["footprint"] in (plain, wide) for r in req)
         if slots < 4:
             assert all(r["footprint"] == plain for r in req)
+
+
+def test_covariance_tables_of_a_request_are_in_its_block(host, tmp_path):
+    """A slot keeps the upload of a request's system (subapertures' positions, noise and places: some
+    120 bytes each here, and the structure function's table of 64 KB), not the covariance
+    tables of its sensor pairs, which lie in the request's own block."""
+    from moao_amd import systems
+    s, a = systems.make_system(str(tmp_path), systems.SystemSpec(diam=8.0, nssp=24, nlgs=8, nngs=0,
+                                                                 nlayer=2, seed=4))
+    out = host("serve", s, a[0], 0, 1, 0, 2)
+    req, mem = _words(out, "request"), _words(out, "peak")[0]
+    tables = 36 * 3 * 8 * (2 * 24 - 1) ** 2  # 8 sensors' pairs, xx, yy and xy, 47 x 47 differences
+    assert ["launched", "lattice_table"] in out and ["launched", "lattice_fill"] in out
+    assert mem["kept"] <= 120 * req[0]["n"] // 2 * 9 // 8 + 70_000 + 16_384 < tables
+    assert mem["taken"] <= mem["peak"] == req[0]["footprint"]
