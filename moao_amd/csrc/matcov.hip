@@ -702,15 +702,16 @@ Lattices find_lattices(const moao_tomo_view* t, const std::vector<long>& off,
         const double x0 = *std::min_element(X, X + N), y0 = *std::min_element(Y, Y + N);
         fx.resize(N);
         fy.resize(N);
-        double far = 0, most = 0;
+        double most = 0;
+        bool ok = true;  // comparisons that a NaN fails
         for (long i = 0; i < N; ++i) {
             const double x = (X[i] - x0) / pitch[w], y = (Y[i] - y0) / pitch[w];
             fx[i] = std::floor(x + 0.5);
             fy[i] = std::floor(y + 0.5);
-            far = std::max(far, std::max(std::fabs(x - fx[i]), std::fabs(y - fy[i])));
+            ok = ok & (std::fabs(x - fx[i]) < 1e-6) & (std::fabs(y - fy[i]) < 1e-6);
             most = std::max(most, std::max(fx[i], fy[i]));
         }
-        bool ok = far < 1e-6 && most < 1024;
+        ok = ok && most < 1024;
         for (int l = 0; l < L && ok; ++l) {
             const double s = t->sspSizeL[w * L + l];
             if (!(s > 0)) continue;

@@ -240,6 +240,26 @@ int run_mixed(char** a) {
                                             nullptr, nullptr, nullptr);
 }
 
+// sys atm type [field index value]...: matcov of a whole matrix, with values of the system replaced
+int run_matcov(char** a, int n) {
+    moao_tomo* t = nullptr;
+    if (int rc = moao_tomo_create(a[0], a[1], &t)) return rc;
+    moao_tomo_set_target(t, 0);
+    moao_tomo_view v;
+    moao_tomo_get_view(t, &v);
+    const int type = std::atoi(a[2]);
+    for (int k = 3; k + 2 < n; k += 3) {
+        const std::string f = a[k];
+        const double* p = f == "X" ? v.X : f == "Y" ? v.Y : f == "u" ? v.u : f == "v" ? v.v
+                        : f == "sspSizeL" ? v.sspSizeL : f == "L0" ? v.L0 : nullptr;
+        const_cast<double*>(p)[std::atol(a[k + 1])] = std::atof(a[k + 2]);
+    }
+    const int cols = (int)moao_tomo_nmeas(t), rows = type == 1 ? cols : (int)moao_tomo_nmeasts(t);
+    const int rc = moao_hip_matcov_tile_dev(at(1), rows, cols, 0, 0, rows, &v, type, nullptr);
+    moao_tomo_destroy(t);
+    return rc;
+}
+
 // sys atm mode slots budget requests: what the requests were said to hold and what they took
 int run_serve(char** a) {
     show = false;
@@ -275,6 +295,7 @@ int main(int argc, char** argv) {
     if (const char* l = std::getenv("ASYNC_LIMIT")) limit = std::strtoull(l, nullptr, 10);
     if (cmd == "gemm" && argc == 9) rc = run_gemm(argv + 2);
     if (cmd == "mixed" && argc == 5) rc = run_mixed(argv + 2);
+    if (cmd == "matcov" && argc >= 5) rc = run_matcov(argv + 2, argc - 2);
     if (cmd == "serve" && argc == 8) rc = run_serve(argv + 2);
     std::printf("rc %d\n", rc);
     return rc == 2;

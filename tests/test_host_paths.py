@@ -147,3 +147,25 @@ def test_covariance_tables_of_a_request_are_in_its_block(host, tmp_path):
     assert ["launched", "lattice_table"] in out and ["launched", "lattice_fill"] in out
     assert mem["kept"] <= 120 * req[0]["n"] // 2 * 9 // 8 + 70_000 + 16_384 < tables
     assert mem["taken"] <= mem["peak"] == req[0]["footprint"]
+
+
+@pytest.mark.parametrize("field", ["X", "Y"])
+@pytest.mark.parametrize("index", [0, 7])
+def test_sensor_with_a_nan_position_is_no_grid(host, tmp_path, field, index):
+    """A NaN among a sensor's positions takes the sensor out of the covariance tables, also where no
+    layer's positions can show it (a sensor that sees no layer): its place on a grid would be an
+    index without bounds."""
+    from moao_amd import systems
+    s, a = systems.make_system(str(tmp_path), systems.SystemSpec(diam=8.0, nssp=16, nlgs=3, nngs=0,
+                                                                 nlayer=2, seed=3))
+    unseen = ["sspSizeL", 0, 0.0, "sspSizeL", 1, 0.0]
+    names = [k for k, _ in kernels(host("matcov", s, a[0], 1, *unseen))]
+    assert names == ["lattice_table", "lattice_fill", "pair_kernel"]  # sensor 0 is a grid of its own
+    tables = _grids(host("matcov", s, a[0], 1, *unseen))
+    assert tables == 1 + 3  # sensor 0 with itself, sensors 1 and 2 with each other
+    assert _grids(host("matcov", s, a[0], 1, *unseen, field, index, "nan")) == 3
+
+
+def _grids(lines):
+    """Sensor pairs with a covariance table."""
+    return [int(w[-2]) for w in lines if w[:2] == ["launch", "lattice_table"]][0]
