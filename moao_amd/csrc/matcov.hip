@@ -75,8 +75,11 @@ constexpr int kSub = 64, kSubBits = 6, kLo = -10, kHi = 11;
 constexpr int kCoef = 6;
 constexpr int kTabN = (kHi - kLo) * kSub + 2;
 constexpr double kTBorder = kXlim * kXlim;
-// Arguments below the table and those within rounding of the border take the direct formulas.
-constexpr double kTMin = 1.0 / (1 << -kLo), kTBand = 1e-9;
+// Arguments below the table, those within rounding of the border, infinities and NaN take the direct
+// formulas.  kHiMin, kHiInf: high words of 2^kLo and of infinity (below kHiMin and from kHiInf on
+// is one unsigned comparison).
+constexpr unsigned kHiMin = (unsigned)(1023 + kLo) << 20, kHiInf = 0x7ff00000u;
+constexpr double kTBand = 1e-9;
 
 constexpr int kRows = 64;       // rows per workgroup (one wave tall)
 constexpr int kWaves = 8;       // waves per workgroup; each takes MatcovArgs::cw columns
@@ -178,7 +181,8 @@ __device__ __forceinline__ void vk_table(const double* tab, const double (&x)[N]
 #pragma unroll
     for (int n = 0; n < N; ++n) {
         t[n] = fma(x[n], x[n], y[n] * y[n]) * (lk * lk);
-        direct[n] = !(t[n] >= kTMin) || fabs(t[n] - kTBorder) < kTBand;
+        direct[n] = (unsigned)__double2hiint(t[n]) - kHiMin >= kHiInf - kHiMin ||
+                    fabs(t[n] - kTBorder) < kTBand;
         any = any || direct[n];
     }
 #pragma unroll

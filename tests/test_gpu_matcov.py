@@ -231,3 +231,36 @@ def test_cmm_tiles_at_and_above_the_diagonal(tmp_path, xo, yo):
     low = np.arange(xo, xo + 40)[:, None] >= np.arange(yo, yo + 30)[None, :]
     assert np.array_equal(buf[low], C[xo:xo + 40, yo:yo + 30][low])
     assert np.all(buf[~low] == -1.0)
+
+
+def _poke(t, field, index, value):
+    """Overwrites one value of the library's model (the view points into it)."""
+    getattr(t.view(), field)[index] = value
+
+
+@pytest.mark.parametrize("field,value", [("u", np.inf), ("v", -np.inf), ("u", np.nan), ("u", 1e200),
+                                         ("L0", 0.0), ("L0", 1e-160)])
+def test_separations_out_of_range(tmp_path, field, value):
+    """Infinite positions, positions whose square overflows and an outer scale of zero give NaN where
+    the reference's formulas do, an outer scale whose inverse square overflows gives their values: Cmm,
+    Ctm and a small tile (evaluated without covariance tables).  Finite elements within 1e-12 of
+    Ctt's largest, as above (Ctt of the unchanged system)."""
+    from moao_amd import systems
+    s, a = systems.make_system(str(tmp_path), systems.SystemSpec(diam=8.0, nssp=8, nlgs=2, nngs=1,
+                                                                 nlayer=2, seed=8))
+    t, o = Tomo(s, a[0]), OTomo.from_files(s, a[0])
+    t.set_target(0)
+    o.set_target(0)
+    scale = np.max(np.abs(om.ctt(o)))
+    k = 0 if field == "L0" else 5
+    _poke(t, field, k, value)
+    (o.L0diff if field == "L0" else getattr(o, field).reshape(-1))[k] = value
+    print(f"[matcov-inf] {field} = {value}", flush=True)
+    for g, r in ((np.tril(gm.cmm(t)), np.tril(om.cmm(o))), (gm.ctm(t), om.ctm(o))):
+        bad = ~np.isfinite(r)
+        assert bad.any() == (value != 1e-160)
+        assert np.array_equal(np.isnan(g), np.isnan(r))
+        assert np.max(np.abs(g - r)[~bad], initial=0.0) <= 1e-12 * scale
+    tile, whole = np.zeros((9, 7), order="F"), gm.ctm(t)
+    gm.matcov_tile(tile, 9, 7, 0, 0, 9, t, gm.CTM)
+    assert np.array_equal(tile, whole[:9, :7], equal_nan=True)
