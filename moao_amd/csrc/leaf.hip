@@ -105,6 +105,23 @@ __device__ __forceinline__ void gather_rows(double v, double (&r)[4]) {
     for (int q = 0; q < 4; ++q) __builtin_memcpy(&r[q], o[q], 8);
 }
 
+// Whether the unnormalised elimination below takes pivot d as it is, 2^-1000 <= d < 2^1000: it needs
+// reciprocals (they overflow below 2^-1023) where the reciprocal square root has the whole range.
+// One unsigned comparison of the high words, which negative numbers, infinities and NaN fail.
+__device__ __forceinline__ bool easy_pivot(double d) {
+    constexpr unsigned lo = (1023u - 1000) << 20, hi = (1023u + 1000) << 20;
+    return (unsigned)__double2hiint(d) - lo < hi - lo;
+}
+
+// Exponent e that brings diagonal element li of a block (accumulator layout, see diag_factor) to
+// 2^(2 e) A[li][li] in [1/2, 2); 0 where the element is not a positive number.
+__device__ __forceinline__ int diag_exponent(f64x4 a, int li, int lq) {
+    const int t = li >> 2;
+    const double own = t & 2 ? (t & 1 ? a[3] : a[2]) : (t & 1 ? a[1] : a[0]);
+    const double d = __shfl(own, li + 16 * (li & 3));  // lane row li % 4 holds column li in a[t]
+    return d > 0.0 && d < __builtin_inf() ? -(__builtin_amdgcn_frexp_exp(d) >> 1) : 0;
+}
+
 // A 16 x 16 block A = L L^T and D = inv(L) in one wave.  c in MFMA accumulator layout: lane
 // (li, lq) = (l % 16, l / 16) holds A[li][lq + 4t] in c[t] (lower triangle used).  Unnormalised
 // elimination of [A | I], four columns at a time: columns 4t .. 4t+3 are register t of the four
@@ -149,6 +166,43 @@ __device__ __forceinline__ void diag_factor(f64x4 c, int li, int lq, double (&lo
         });
         x = __builtin_amdgcn_mfma_f64_16x16x4f64(own(w), x[t], x, 0, 0, 0);
     });
+}
+
+// L of the block to S (leading dimension LD) and its inverse to Db, both up to order bs.
+__device__ __forceinline__ void store_block(const double (&lo)[4], const double (&piv)[4], f64x4 x,
+                                            int li, int lq, double* S, double* Db, int bs) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        const double rs = rsqrt_nr(piv[t]);
+        const int col = lq + 4 * t;
+        if (li < bs && col <= li) S[li + col * LD] = lo[t] * rs;
+        Db[col * kB + li] = col < bs && li <= col ? x[t] * rs : 0.0;
+    }
+}
+
+// A block with pivots that are not easy: once more with its diagonal scaled to about 1, c row and
+// column li by 2^ex, so L's row li by 2^ex and inv(L)'s column li by 2^-ex.  The first pivot that is
+// not positive (NaN included), then nothing is stored; else kB.
+__device__ __noinline__ int hard_block(f64x4 c, int li, int lq, double* S, double* Db, int bs) {
+    const int ex = diag_exponent(c, li, lq);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) c[t] = ldexp(c[t], ex + __shfl(ex, lq + 4 * t));
+    double lo[4], piv[4];
+    f64x4 x;
+    diag_factor(c, li, lq, lo, piv, x);
+    int first = kB;
+#pragma unroll
+    for (int t = 3; t >= 0; --t)
+        for (int q = 3; q >= 0; --q)
+            if (__ballot(lq == q && !(piv[t] > 0.0))) first = 4 * t + q;
+    if (first < kB) return first;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        lo[t] = ldexp(lo[t], -ex);
+        x[t] = ldexp(x[t], ex);
+    }
+    store_block(lo, piv, x, li, lq, S, Db, bs);
+    return kB;
 }
 
 // 16 x 16 block product on MFMA: acc += X[r0:r0+16, k0:k0+16*nc] * Y[k0:k0+16*nc, c0:c0+16]
@@ -329,25 +383,16 @@ __global__ void __launch_bounds__(NTL) leaf_potrf_inv(TS* A, long lda, int nb, T
             double lo[4], piv[4];
             f64x4 x;
             diag_factor(c, li, lq, lo, piv, x);
-            const bool good = piv[0] > 0.0 && piv[1] > 0.0 && piv[2] > 0.0 && piv[3] > 0.0;
-            if (__ballot(!good)) {
-                int first = kB;  // the first pivot that is not positive (NaN included)
-#pragma unroll
-                for (int t = 3; t >= 0; --t)
-                    for (int q = 3; q >= 0; --q)
-                        if (__ballot(lq == q && !(piv[t] > 0.0))) first = 4 * t + q;
-                if (lane == 0) {
+            const bool easy = easy_pivot(piv[0]) && easy_pivot(piv[1]) && easy_pivot(piv[2]) &&
+                              easy_pivot(piv[3]);
+            if (__ballot(!easy)) {
+                const int first = hard_block(c, li, lq, &S_(kb, kb), Db, bs);
+                if (first < kB && lane == 0) {
                     fail = 1;
                     atomicCAS(info, 0, j0 + kb + first + 1);
                 }
             } else {
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const double rs = rsqrt_nr(piv[t]);
-                    const int col = lq + 4 * t;
-                    if (li < bs && col <= li) S_(kb + li, kb + col) = lo[t] * rs;
-                    Db[col * kB + li] = col < bs && li <= col ? x[t] * rs : 0.0;
-                }
+                store_block(lo, piv, x, li, lq, &S_(kb, kb), Db, bs);
             }
         }
         lds_barrier();

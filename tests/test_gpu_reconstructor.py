@@ -363,3 +363,25 @@ def test_backward_solve_of_many_rows_equals_that_of_few():
     assert reconstructor(n, big, C.copy(order="F"), n, R, big, 1) == 0
     assert reconstructor(n, few, C.copy(order="F"), n, r, few, 1) == 0
     assert np.array_equal(R[:few], r)
+
+
+@pytest.mark.parametrize("n", [5, 16, 70, 128, 200])
+@pytest.mark.parametrize("low,high", [(-520, -520), (-520, 0), (0, 511), (511, 511), (-400, 400)])
+def test_pivots_at_the_ends_of_the_range(n, low, high):
+    """Pivots down to 2^-1040 (subnormal, no reciprocal in range) and up to 2^1022 (its reciprocal is
+    subnormal), all alike or beside each other: A = D T T^T D with D powers of two and T unit lower
+    triangular with one entry of +-1 left of the diagonal in a row, so L = D T and R = C (T T^T)^-1
+    D^-1 for B = C D hold to a few roundings of each sum of n terms of at most max |T^-1| <= 1."""
+    print(f"[recon] pivots 2^{2 * low} .. 2^{2 * high}, n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    T = np.eye(n)
+    for i in range(1, n):
+        T[i, rng.integers(0, i)] = rng.choice([-1.0, 1.0])
+    d = np.ldexp(1.0, np.where(np.arange(n) % 3 == 1, low, high))
+    Cg = np.asfortranarray(np.tril(d[:, None] * (T @ T.T) * d))
+    C = rng.integers(-3, 4, (9, n)).astype(np.float64)
+    Bg = np.asfortranarray(C * d)
+    assert reconstructor(n, 9, Cg, n, Bg, 9, 1) == 0
+    assert np.max(np.abs(np.tril(Cg) / d[:, None] - T)) <= 1e-12
+    want = np.linalg.solve(T.T, np.linalg.solve(T, C.T)).T
+    assert np.max(np.abs(Bg * d - want)) <= 1e-12 * n * np.max(np.abs(C))
