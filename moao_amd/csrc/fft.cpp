@@ -11,14 +11,18 @@ namespace moao {
 template <typename R>
 int fft_twiddles(int N, typename Cplx<R>::type** d_table, hipStream_t s) {
     using C = typename Cplx<R>::type;
-    std::vector<C> h(N);
+    int log = 0;
+    while (1 << log < N) ++log;
+    std::vector<C> h;  // N - (first radix) values
     const double pi = 3.14159265358979323846;
-    for (int e = 0; e < N; ++e) {
-        const double a = -2.0 * pi * (double)e / (double)N;
-        h[e] = C{(R)std::cos(a), (R)std::sin(a)};
-    }
-    MOAO_HIP_TRY(hipMalloc((void**)d_table, sizeof(C) * N));
-    MOAO_HIP_TRY(hipMemcpyAsync(*d_table, h.data(), sizeof(C) * N, hipMemcpyHostToDevice, s));
+    for (int ns = fft_radix(log, 1); ns < N; ns *= fft_radix(log, ns))
+        for (int m = 1; m < fft_radix(log, ns); ++m)
+            for (int k = 0; k < ns; ++k) {
+                const double a = -2.0 * pi * m * k / ((double)ns * fft_radix(log, ns));
+                h.push_back(C{(R)std::cos(a), (R)std::sin(a)});
+            }
+    MOAO_HIP_TRY(hipMalloc((void**)d_table, sizeof(C) * h.size()));
+    MOAO_HIP_TRY(hipMemcpyAsync(*d_table, h.data(), sizeof(C) * h.size(), hipMemcpyHostToDevice, s));
     MOAO_HIP_TRY(hipStreamSynchronize(s));
     return MOAO_OK;
 }

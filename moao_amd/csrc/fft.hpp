@@ -15,6 +15,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 namespace moao {
 
 template <typename R>
@@ -24,7 +26,16 @@ struct Cplx<float> { using type = float2; };
 template <>
 struct Cplx<double> { using type = double2; };
 
-// Twiddle table W_N^e = exp(-2 pi i e / N), e < N, built on the host in FP64 and rounded once.
+// Values per lane of a transform of 2^log: 8 where the radices come out even (8.4, 8.8, 8.8.8), else
+// 16; and the radix of its stage over sub-transforms of length ns.
+constexpr int fft_values(int log) { return log == 5 || log == 6 || log == 9 ? 8 : 16; }
+constexpr int fft_radix(int log, int ns) {
+    return fft_values(log) < (1 << log) / ns ? fft_values(log) : (1 << log) / ns;
+}
+
+// Twiddles of a transform of N values, stage by stage: exp(-2 pi i m k / (ns P)) for m = 1 .. P - 1 and
+// k < ns (k fast: neighbouring lanes read neighbouring entries), computed on the host in FP64 and
+// rounded once.
 template <typename R>
 int fft_twiddles(int N, typename Cplx<R>::type** d_table, hipStream_t s);
 
@@ -32,8 +43,7 @@ template <typename R, int LOG>
 struct RowFft {
     using C = typename Cplx<R>::type;
     static constexpr int N = 1 << LOG;
-    // 8 values per lane where the radices come out even (8.4, 8.8, 8.8.8), else 16
-    static constexpr int E = LOG == 5 || LOG == 6 || LOG == 9 ? 8 : 16;
+    static constexpr int E = fft_values(LOG);
     static constexpr int T = N / E;
     // 4 rows per workgroup; 2 where 4 would not fit the 160 KB of LDS
     static constexpr int kRows = sizeof(R) == 8 && LOG == 12 ? 2 : 4;
@@ -49,6 +59,10 @@ struct RowFft {
     template <int DIR>
     static __device__ __forceinline__ C mul_i(C a) {  // a * (DIR * i)
         return DIR > 0 ? C{-a.y, a.x} : C{a.y, -a.x};
+    }
+    template <int DIR>
+    static __device__ __forceinline__ C conj_if(C a) {  // a's conjugate for the backward direction
+        return DIR > 0 ? C{a.x, -a.y} : a;
     }
     template <int DIR>
     static __device__ __forceinline__ void dft4(C& a, C& b, C& c, C& d) {
@@ -99,87 +113,126 @@ struct RowFft {
         }
     }
 
-    // Twiddles of one stage: W^(m k), m < P, from the entries m = 1, 2, 3 and the multiples of 4
-    static constexpr int radix(int ns) { return E < N / ns ? E : N / ns; }
+    static constexpr int radix(int ns) { return fft_radix(LOG, ns); }
+    // A run takes its twiddles from the table, a stage's while the row crosses LDS on the way to it, or
+    // from registers filled before the run.  There a lane keeps, of a stage's factors m = 1 .. P - 1,
+    // those with m = 1, 2, 3 and the multiples of 4 and multiplies out the others: at N = 2048 14
+    // loads and not 29, but with the roundings of the products.  With those in every run the FP32
+    // PSF is 8, 2 and 3% (N = 512, 1024, 2048) further from the exact one than by radix-4 stages
+    // with table entries alone; with the table in its last two runs 0.4 +- 0.6% further, 0.6 and 0.4%
+    // nearer.
+    struct Table {
+        const C* w;
+    };
     static constexpr int entries(int p) { return p == 16 ? 6 : p == 8 ? 4 : p - 1; }
+    static constexpr int factor(int k) { return k < 3 ? k + 1 : 4 * k - 8; }
     static constexpr int tw_count(int ns) {
         return ns >= N ? 0
                        : (ns > 1 ? E / radix(ns) * entries(radix(ns)) : 0) + tw_count(ns * radix(ns));
     }
-    static constexpr int kTw = tw_count(1);
-    template <int NS = 1, int AT = 0>
-    static __device__ __forceinline__ void load_twiddles(C (&w)[kTw], int t,
-                                                         const C* __restrict__ tw) {
+    struct Kept {
+        C w[tw_count(1)];
+    };
+    // AT, FROM: where the stage's entries start in Kept and in the table
+    template <int NS = 1, int AT = 0, int FROM = 0>
+    static __device__ __forceinline__ void keep(Kept& kept, const Table& tw, int t) {
         if constexpr (NS < N) {
             constexpr int P = radix(NS), Q = E / P, M = NS > 1 ? entries(P) : 0;
 #pragma unroll
-            for (int q = 0; q < Q; ++q) {
-                const int k = ((t + q * T) & (NS - 1)) * (N / (NS * P));
+            for (int q = 0; q < Q; ++q)
 #pragma unroll
-                for (int m = 0; m < M; ++m) w[AT + q * M + m] = tw[(m < 3 ? m + 1 : 4 * m - 8) * k];
-            }
-            load_twiddles<NS * P, AT + Q * M>(w, t, tw);
+                for (int k = 0; k < M; ++k)
+                    kept.w[AT + q * M + k] =
+                        tw.w[FROM + (factor(k) - 1) * NS + ((t + q * T) & (NS - 1))];
+            keep<NS * P, AT + Q * M, FROM + (NS > 1 ? (P - 1) * NS : 0)>(kept, tw, t);
+        }
+    }
+    // A run's twiddles: the table's own, or kept ones.  FP64 keeps them always (its PSF is nearer to
+    // the exact one than by radix-4 stages all the same, and 8 directions at N = 1024 take 98 us
+    // with the table, 93 without).
+    template <bool TABLE>
+    static __device__ __forceinline__ auto twiddles(const C* tw, int t) {
+        if constexpr (TABLE && sizeof(R) == 4) {
+            return Table{tw};
+        } else {
+            Kept kept;
+            keep(kept, Table{tw}, t);
+            return kept;
         }
     }
 
     // Stage over sub-transforms of length NS, then the later ones.  Butterfly j = t + q T takes
-    // elements j + m N/P, m < P.
-    template <int DIR, int NS, int AT>
-    static __device__ __forceinline__ void stage(C (&v)[E], C* lds, int t, int row,
-                                                 const C (&tw)[kTw]) {
-        if constexpr (NS < N) {
-            constexpr int P = radix(NS), Q = E / P, M = NS > 1 ? entries(P) : 0;
-            if constexpr (NS * P < N) __syncthreads();  // the last reads of lds are done
+    // elements j + m N/P times factor m, m < P; from the table f holds factor m at q (P - 1) + m - 1.
+    template <int DIR, int NS, int AT, int FROM, typename W, int L>
+    static __device__ __forceinline__ void stage(C (&v)[E], C* lds, int t, int row, const W& tw,
+                                                 const C (&f)[L]) {
+        constexpr bool kTable = std::is_same<W, Table>::value;
+        constexpr int P = radix(NS), Q = E / P, M = NS > 1 ? entries(P) : 0;
+        if constexpr (NS * P < N) __syncthreads();  // the last reads of lds are done
 #pragma unroll
-            for (int q = 0; q < Q; ++q) {
-                const int j = t + q * T;
-                C x[P];
+        for (int q = 0; q < Q; ++q) {
+            const int j = t + q * T;
+            C x[P];
 #pragma unroll
-                for (int m = 0; m < P; ++m) x[m] = v[q + m * Q];
-                if constexpr (NS > 1) {
-                    C w[P];
+            for (int m = 0; m < P; ++m) x[m] = v[q + m * Q];
+            if constexpr (NS > 1) {
+                C w[P];
+                if constexpr (kTable) {
 #pragma unroll
-                    for (int m = 0; m < M; ++m) {
-                        C& c = w[m < 3 ? m + 1 : 4 * m - 8];
-                        c = tw[AT + q * M + m];
-                        if (DIR > 0) c.y = -c.y;
-                    }
+                    for (int m = 1; m < P; ++m) w[m] = conj_if<DIR>(f[q * (P - 1) + m - 1]);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < M; ++k) w[factor(k)] = conj_if<DIR>(tw.w[AT + q * M + k]);
 #pragma unroll
                     for (int m = 5; m < P; ++m)
                         if (m % 4) w[m] = mul(w[m & ~3], w[m & 3]);
-#pragma unroll
-                    for (int m = 1; m < P; ++m) x[m] = mul(x[m], w[m]);
                 }
-                dft<P, DIR>(x);
-                if constexpr (NS * P < N) {
-                    const int o = (j / NS) * NS * P + (j & (NS - 1));
 #pragma unroll
-                    for (int m = 0; m < P; ++m) {
-                        const int i = o + m * NS;
-                        lds[(i + i / E) * kRows + row] = x[m];
-                    }
-                } else {
-#pragma unroll
-                    for (int m = 0; m < P; ++m) v[q + m * Q] = x[m];
-                }
+                for (int m = 1; m < P; ++m) x[m] = mul(x[m], w[m]);
             }
+            dft<P, DIR>(x);
             if constexpr (NS * P < N) {
-                __syncthreads();
+                const int o = (j / NS) * NS * P + (j & (NS - 1));
 #pragma unroll
-                for (int e = 0; e < E; ++e) {
-                    const int i = t + T * e;
-                    v[e] = lds[(i + i / E) * kRows + row];
+                for (int m = 0; m < P; ++m) {
+                    const int i = o + m * NS;
+                    lds[(i + i / E) * kRows + row] = x[m];
                 }
-                stage<DIR, NS * P, AT + Q * M>(v, lds, t, row, tw);
+            } else {
+#pragma unroll
+                for (int m = 0; m < P; ++m) v[q + m * Q] = x[m];
             }
+        }
+        if constexpr (NS * P < N) {
+            constexpr int NS2 = NS * P, P2 = radix(NS2), Q2 = E / P2;
+            C f2[kTable ? Q2 * (P2 - 1) : 1];
+            if constexpr (kTable) {
+                // at an address that the compiler takes for another run to run: what it kept from one
+                // run for the next would fill the registers of the work between them
+                int k = t;
+                asm volatile("" : "+v"(k));
+#pragma unroll
+                for (int q = 0; q < Q2; ++q)
+#pragma unroll
+                    for (int m = 1; m < P2; ++m)
+                        f2[q * (P2 - 1) + m - 1] =
+                            tw.w[FROM + (m - 1) * NS2 + ((k + q * T) & (NS2 - 1))];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const int i = t + T * e;
+                v[e] = lds[(i + i / E) * kRows + row];
+            }
+            stage<DIR, NS2, AT + Q * M, FROM + (P2 - 1) * NS2>(v, lds, t, row, tw, f2);
         }
     }
     // v[e] = element t + T e of the row, before and after; unnormalised; every thread of the
-    // workgroup calls it.
-    template <int DIR>
-    static __device__ __forceinline__ void run(C (&v)[E], C* lds, int t, int row,
-                                               const C (&tw)[kTw]) {
-        stage<DIR, 1, 0>(v, lds, t, row, tw);
+    // workgroup calls it.  tw: a Table or a Kept.
+    template <int DIR, typename W>
+    static __device__ __forceinline__ void run(C (&v)[E], C* lds, int t, int row, const W& tw) {
+        const C none[1] = {};
+        stage<DIR, 1, 0, 0>(v, lds, t, row, tw, none);
     }
 };
 

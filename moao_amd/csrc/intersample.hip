@@ -334,8 +334,8 @@ __global__ __launch_bounds__((RowFft<R, LOG>::kThreads), (RowFft<R, LOG>::kWaves
         lds[u] = C{(R)z[0], (R)z[1]};
     }
     __syncthreads();
-    C v[F::E], tw[F::kTw];
-    F::load_twiddles(tw, t, g.tw);
+    C v[F::E];
+    const auto tw = F::template twiddles<false>(g.tw, t);
 #pragma unroll
     for (int e = 0; e < F::E; ++e) {
         const int tj = map_index(t + F::T * e, g.first, g.step, g.ncov);
@@ -353,6 +353,12 @@ __global__ __launch_bounds__((RowFft<R, LOG>::kThreads), (RowFft<R, LOG>::kWaves
     }
 }
 
+// Whether the middle runs (map_cols, the first of dphi_rows) take their twiddles from the table.  The
+// kept ones take registers beside the row's: N = 1024, FP32, 8 directions, kept -> table 16.5 ->
+// 14.3 us in map_cols; N = 2048, where a run's loads are more, 40 -> 44.
+template <typename F>
+constexpr bool middle_from_table = F::N <= 1024;
+
 // Bound by its writes (67 MB at N = 2048 and 4 pairs, 40 us): columns j <= N/2, transform along x,
 // product with abs2fi, transform back.  mid[j] = H(N/2, j).
 template <typename R, int LOG>
@@ -367,8 +373,8 @@ __global__ __launch_bounds__((RowFft<R, LOG>::kThreads), (RowFft<R, LOG>::kWaves
     const int2 b = tile_line<F>();
     const int j = b.x * K + row, p = b.y;
     A += ((size_t)p * NB + b.x) * K * g.ncov + row;
-    C v[F::E], tw[F::kTw];
-    F::load_twiddles(tw, t, g.tw);
+    C v[F::E];
+    const auto tw = F::template twiddles<middle_from_table<F>>(g.tw, t);
     R wt[F::E];
 #pragma unroll
     for (int e = 0; e < F::E; ++e) {
@@ -431,8 +437,8 @@ __global__ __launch_bounds__((RowFft<R, LOG>::kThreads), (RowFft<R, LOG>::kWaves
     const int t = threadIdx.x / K, row = threadIdx.x % K;
     const int2 b = tile_line<F>();
     const int r = b.x * K + row, p = b.y;
-    C v[E], tw[F::kTw];
-    F::load_twiddles(tw, t, g.tw);
+    C v[E];
+    const auto tw = F::template twiddles<middle_from_table<F>>(g.tw, t);
     load_line<F>(v, H + p * grid_size<F>(), t, r);
     mid += (size_t)p * (N / 2 + 1);
     double na = 0, nb = 0;
@@ -472,8 +478,7 @@ __global__ __launch_bounds__((RowFft<R, LOG>::kThreads), (RowFft<R, LOG>::kWaves
     // read again, not kept across the exponentials: the registers decide the occupancy
     int again = t;
     asm volatile("" : "+v"(again));
-    F::load_twiddles(tw, again, g.tw);
-    F::template run<1>(x, lds, t, row, tw);
+    F::template run<1>(x, lds, t, row, F::template twiddles<true>(g.tw, again));
     store_line<F>(x, H2 + p * grid_size<F>(), t, r);
 }
 
@@ -490,8 +495,8 @@ __global__ __launch_bounds__((RowFft<R, LOG>::kThreads), (RowFft<R, LOG>::kWaves
     const int t = threadIdx.x / K, row = threadIdx.x % K;
     const int2 b = tile_line<F>();
     const int r = b.x * K + row, p = b.y;
-    C v[E], tw[F::kTw];
-    F::load_twiddles(tw, t, g.tw);
+    C v[E];
+    const auto tw = F::template twiddles<true>(g.tw, t);
     load_line<F>(v, H2 + p * grid_size<F>(), t, r);
     F::template run<1>(v, lds, t, row, tw);
     // Through LDS by rows, so that every store is a contiguous kilobyte of one image row; lane
