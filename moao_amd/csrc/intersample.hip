@@ -32,6 +32,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <deque>
 #include <vector>
 
 #include "common.hpp"
@@ -653,28 +654,36 @@ bool make_plan(const long* idx, long nidx, int ncov, Plan* plan) {
         long i;
         int place, len;
     };
-    std::vector<Flat> flat;
-    for (long i = 0, next = -1; i < nidx; ++i) {
+    // by entries as soon as the runs are too many; the list grows in pieces, not by doubling
+    const long most = nidx <= kEntryMax ? nidx / kRunFrom : nidx;
+    std::deque<Flat> flat;
+    for (long i = 0, next = -1; i < nidx && !P.entries; ++i) {
         const long b = idx[i] - 1;
         if (b < 0 || b >= nmap) return false;
         P.div[b] += 1;
         const int p = place[b];
         if (p == next && flat.back().len < 64 && p % bins)
             ++flat.back().len;
-        else
+        else if ((long)flat.size() < most)
             flat.push_back({i, p, 1});
+        else
+            P.entries = true;
         next = p + 1;
     }
-    if (nidx < kRunFrom * (long)flat.size() && nidx <= kEntryMax) {
-        P.entries = true;
+    if (P.entries) {
+        flat.clear();
+        std::vector<int> at(nmap, 0);  // entries of a bin, then where its next one goes
+        for (long i = 0; i < nidx; ++i) {
+            const long b = idx[i] - 1;
+            if (b < 0 || b >= nmap) return false;
+            ++at[b];
+        }
         P.run_of.assign(nmap + 1, 0);
-        for (const Flat& r : flat)
-            for (int k = 0; k < r.len; ++k) ++P.run_of[r.place + k + 1];
+        for (long b = 0; b < nmap; ++b) P.div[b] = P.run_of[place[b] + 1] = at[b];
         for (long b = 0; b < nmap; ++b) P.run_of[b + 1] += P.run_of[b];
+        for (long b = 0; b < nmap; ++b) at[b] = P.run_of[place[b]];
         P.item_of.resize(nidx);
-        std::vector<int> at(P.run_of.begin(), P.run_of.end() - 1);
-        for (const Flat& r : flat)
-            for (int k = 0; k < r.len; ++k) P.item_of[at[r.place + k]++] = (int)r.i + k;
+        for (long i = 0; i < nidx; ++i) P.item_of[at[idx[i] - 1]++] = (int)i;
         return true;
     }
     // slabs: at least two rounds of loads per wave; runs are cut where slabs meet

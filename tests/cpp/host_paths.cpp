@@ -287,6 +287,33 @@ int run_serve(char** a) {
     return 0;
 }
 
+// np N <0 in order | 1 shuffled>: the plan of a PSF whose index lists every pair of np x np actuators
+int run_create(char** a) {
+    const long np = std::atol(a[0]), N = std::atol(a[1]), nact = np * np, ncov = 2 * np - 1;
+    std::vector<long> idx(nact * nact);
+    for (long i = 0; i < nact; ++i)
+        for (long j = 0; j < nact; ++j)
+            idx[i * nact + j] = (i / np - j / np + np - 1) * ncov + i % np - j % np + np;
+    if (std::atoi(a[2])) {
+        unsigned long x = 88172645463325252ul;
+        for (size_t k = idx.size() - 1; k > 0; --k) {
+            x ^= x << 13, x ^= x >> 7, x ^= x << 17;
+            std::swap(idx[k], idx[x % (k + 1)]);
+        }
+    }
+    const std::vector<double> w(N * N, 1.0);
+    cpp_peak = cpp_live.load();
+    const long before = cpp_live;
+    const auto t = std::chrono::steady_clock::now();
+    moao_isample* S = nullptr;
+    const int rc = moao_hip_intersample_create(idx.size(), np, N, idx.data(), w.data(), w.data(), 1, &S);
+    const double s = std::chrono::duration<double>(std::chrono::steady_clock::now() - t).count();
+    std::printf("plan entries %zu heap %ld device %zu us %.0f\n", idx.size(), cpp_peak - before,
+                heap.live, s * 1e6);
+    moao_hip_intersample_destroy(S);
+    return rc;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -296,6 +323,7 @@ int main(int argc, char** argv) {
     if (cmd == "gemm" && argc == 9) rc = run_gemm(argv + 2);
     if (cmd == "mixed" && argc == 5) rc = run_mixed(argv + 2);
     if (cmd == "matcov" && argc >= 5) rc = run_matcov(argv + 2, argc - 2);
+    if (cmd == "plan" && argc == 5) rc = run_create(argv + 2);
     if (cmd == "serve" && argc == 8) rc = run_serve(argv + 2);
     std::printf("rc %d\n", rc);
     return rc == 2;

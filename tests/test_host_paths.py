@@ -169,3 +169,15 @@ def test_sensor_with_a_nan_position_is_no_grid(host, tmp_path, field, index):
 def _grids(lines):
     """Sensor pairs with a covariance table."""
     return [int(w[-2]) for w in lines if w[:2] == ["launch", "lattice_table"]][0]
+
+
+def test_plan_of_an_irregular_index_takes_little_more_than_its_lists(host):
+    """A PSF plan of an index in random order lists its entries (4 bytes each); no list of
+    single-entry runs (16 bytes each and more while it grows) is built on the way.  An index in order
+    takes a run per row of actuators."""
+    pairs = 30 ** 4
+    out = host("plan", 30, 512, 1)
+    assert out[-1] == ["rc", "0"]
+    heap = _words(out, "plan")[0]["heap"]
+    assert 4 * pairs <= heap <= 8 * pairs + 8 * 4 * 59 ** 2
+    assert _words(host("plan", 30, 512, 0), "plan")[0]["heap"] <= 2 * pairs
