@@ -284,3 +284,66 @@ def test_symmetric_operand_in_full_and_in_place_give_the_same_bits(K):
         dgemm_dev(2, M, K, K, 1.0, dA.ptr, 1000, dB.ptr, K, 0.0, dC.ptr, M)
         out.append(dC.to_host())
     assert np.array_equal(out[0][:447], out[1])
+
+
+# Launches of 128-row tiles (tests/test_host_paths.py holds them to that; the shapes of CASES and of
+# test_tiles_at_the_edge run on 64-row tiles): as (type, transb, M, N, K).
+TILES_128 = [(np.float64, 1, 4609 + d, 4737 - d, 2056 + k) for d, k in
+             ((0, 0), (30, 1), (32, 7), (63, 3), (64, 5), (126, 4))] + \
+            [(np.float64, 0, 7425, 7423, 8195), (np.float64, 0, 7551, 7393, 8200),
+             (np.float32, 1, 5921, 5889, 520), (np.float32, 1, 5951, 5999, 525),
+             (np.float32, 0, 4673, 4735, 2049), (np.float32, 0, 4735, 4673, 2061)]
+
+
+@pytest.mark.parametrize("dtype,transb,M,N,K", TILES_128)
+def test_128_row_tiles_at_the_edge(dtype, transb, M, N, K):
+    """128-row tiles whose last row and column tiles hold 1 to 127 rows and columns (waves that leave
+    out half or all of their MFMAs) and whose K ends inside a slice or with one.  The first and the
+    last rows and some between against numpy in 64 bits; tolerance: K products of values below 1,
+    each rounded once and added once, and the two operations of alpha and beta."""
+    print(f"[gemm-128] {dtype.__name__} transb={transb} {M} x {N} x {K}", flush=True)
+    rng = np.random.default_rng(M)
+
+    def uniform(r, c):
+        return np.asfortranarray(rng.uniform(-1, 1, (r, c)).astype(dtype))
+    A, C = uniform(M, K), uniform(M, N)
+    B = uniform(N, K) if transb == 1 else uniform(K, N)
+    dA, dB, dC = (DeviceArray.from_host(x) for x in (A, B, C))
+    f = dgemm_dev if dtype == np.float64 else sgemm_dev
+    f(transb, M, N, K, 0.5, dA.ptr, M, dB.ptr, B.shape[0], 1.0, dC.ptr, M)
+    rows = np.unique(np.r_[:3, 60:68, 126:131, M // 2:M // 2 + 3, M - 130:M])
+    op = (B.T if transb == 1 else B).astype(np.float64)
+    ref = 0.5 * (A[rows].astype(np.float64) @ op) + C[rows]
+    err = np.max(np.abs(dC.to_host()[rows] - ref))
+    assert err <= 2 * (K + 2) * np.finfo(dtype).eps
+
+
+# Products of few rows and of so many that the slice kernels take them, with ragged columns and a K
+# that ends past whole chunks of the direct kernel (checked there too).
+RAGGED, RAGGED_ROWS = (97, 131), (1, 15, 16, 17, 33, 300, 4097, 9000, 66000)
+
+
+@pytest.mark.parametrize("transb", [0, 1])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_few_ragged_rows_equal_the_rows_of_a_slice_product(transb, dtype):
+    """The direct kernel's rows have the bits of the slice kernel's."""
+    print(f"[gemm-direct] {dtype.__name__} transb={transb} ragged", flush=True)
+    f = dgemm_dev if dtype == np.float64 else sgemm_dev
+    rng = np.random.default_rng(17 + transb)
+    N, K = RAGGED
+    big = RAGGED_ROWS[-1]
+    ldb = (N if transb == 1 else K) + 1
+    A = np.asfortranarray(rng.standard_normal((big, K)).astype(dtype))
+    B = np.asfortranarray(rng.standard_normal((ldb, N if transb == 0 else K)).astype(dtype))
+    C = np.asfortranarray(rng.standard_normal((big, N)).astype(dtype))
+    dA, dB = DeviceArray.from_host(A), DeviceArray.from_host(B)
+    for beta in (0.0, 1.0):
+        dC = DeviceArray.from_host(C)
+        f(transb, big, N, K, -1.25, dA.ptr, big, dB.ptr, ldb, beta, dC.ptr, big)
+        want = dC.to_host()
+        for r in RAGGED_ROWS[:-1]:
+            dC = DeviceArray.from_host(C)
+            f(transb, r, N, K, -1.25, dA.ptr, big, dB.ptr, ldb, beta, dC.ptr, big)
+            got = dC.to_host()
+            assert np.array_equal(got[:r], want[:r])
+            assert np.array_equal(got[r:], C[r:])

@@ -3,6 +3,7 @@ and reports which kernels a call launches and what it allocates."""
 import os
 import subprocess
 
+import numpy as np
 import pytest
 
 from conftest import ROOT
@@ -181,3 +182,21 @@ def test_plan_of_an_irregular_index_takes_little_more_than_its_lists(host):
     heap = _words(out, "plan")[0]["heap"]
     assert 4 * pairs <= heap <= 8 * pairs + 8 * 4 * 59 ** 2
     assert _words(host("plan", 30, 512, 0), "plan")[0]["heap"] <= 2 * pairs
+
+
+def test_gpu_gemm_shapes_reach_their_kernels(host):
+    """The shapes that tests/test_gpu_gemm.py gives to the 128-row tiles, to the direct kernel and to the
+    slice kernels go there."""
+    from test_gpu_gemm import RAGGED, RAGGED_ROWS, TILES_128
+    for dtype, transb, M, N, K in TILES_128:
+        p, t = ("f64", "double") if dtype == np.float64 else ("f32", "float")
+        (name, args), = kernels(host("gemm", p, transb, M, N, K, M, N if transb else K))
+        assert name == "gemm_dl_kernel" and args[:2] == [t, str(transb)] and args[3] == "128", \
+            (dtype, transb, M, N, K, name, args)
+    N, K = RAGGED
+    for p in ("f64", "f32"):
+        for transb in (0, 1):
+            got = [kernels(host("gemm", p, transb, r, N, K, 66000, 200))[0] for r in RAGGED_ROWS]
+            assert {k for k, _ in got[:-1]} == {"gemm_direct_kernel"}
+            assert {a[2] for _, a in got[:-1]} == {"1", "2"}  # 16- and 32-row workgroups
+            assert got[-1][0] == "gemm_dl_kernel"
