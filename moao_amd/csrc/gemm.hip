@@ -43,7 +43,7 @@ constexpr int NT = 256;
 #endif
 constexpr int kStages = MOAO_GEMM_STAGES;  // direct-to-LDS pipeline depth (slices in flight + 1)
 
-// TB: 0 = B is K x N, 1 = B is N x K (op = transpose), 2 = B symmetric K x K, lower stored.
+// TB: 0 = B is K x N, 2 = B symmetric K x K, lower stored (op(B) = B^T never falls back).
 // Loads are branch-free: addresses are clamped into the matrix and out-of-range values zeroed
 // by a select, so the compiler issues every load of a slice back to back.
 // WMB: 16-row MFMA blocks per wave along M (4: 128-row tile; 2: 64-row tile for launches
@@ -103,7 +103,7 @@ __global__ void __launch_bounds__(NT, WMB == 4 ? 2 : 4) gemm_kernel(GemmArgs<T> 
     const unsigned bcoloff = (unsigned)min(n0 + lrow, Nc) * (unsigned)sizeof(T);  // bytes
     const bool bcol_ok = n0 + lrow < N;
 
-    int bpat = TB == 1 ? 1 : 0;  // layout of the slice held in rb
+    int bpat = 0;  // layout of the slice held in rb
     auto load = [&](int k0) {
         ma = mb = 0;
 #pragma unroll
@@ -113,7 +113,7 @@ __global__ void __launch_bounds__(NT, WMB == 4 ? 2 : 4) gemm_kernel(GemmArgs<T> 
             ra[r] = *(const T*)((const char*)col + aoff);
             ma |= (unsigned)(arow_ok && k < K) << r;
         }
-        int pat = TB == 1 ? 1 : 0;
+        int pat = 0;
         if (TB == 2) {
             if (k0 + BK - 1 < n0) pat = 1;            // slice wholly above the diagonal
             else if (k0 >= n0 + BN - 1) pat = 0;      // wholly below
@@ -1215,20 +1215,19 @@ int launch(const GemmArgs<T>& g, hipStream_t stream) {
             return MOAO_OK;
         }
     } after{g, stream};
-    // the direct-to-LDS slice kernel, else the fallback
-    const bool dl = g.transb == 1 || (kn_offsets_fit && (g.transb == 0 || g.symdiag));
+    // the direct-to-LDS slice kernel, else the fallback (diagonal blocks are for FP64 only)
+    const bool blocks = sizeof(T) == 8 && g.symdiag;
+    const bool dl = g.transb == 1 || (kn_offsets_fit && (g.transb == 0 || blocks));
     const bool half = dl ? half_tiles(g, cells) : small;
     if (half) grid.x = (maxM + 63) / 64;
-    void (*k)(GemmArgs<T>);
+    auto* k = half ? gemm_dl_kernel<T, 0, kStages, 64> : gemm_dl_kernel<T, 0, kStages, 128>;
     if (!dl)
         k = g.transb == 0 ? (half ? gemm_kernel<T, 0, 2> : gemm_kernel<T, 0, 4>)
                           : (half ? gemm_kernel<T, 2, 2> : gemm_kernel<T, 2, 4>);
-    else if (g.transb == 2)
-        k = gemm_dl_kernel<T, 2, kStages, 64>;
     else if (g.transb == 1)
         k = half ? gemm_dl_kernel<T, 1, kStages, 64> : gemm_dl_kernel<T, 1, kStages, 128>;
-    else
-        k = half ? gemm_dl_kernel<T, 0, kStages, 64> : gemm_dl_kernel<T, 0, kStages, 128>;
+    if constexpr (sizeof(T) == 8)
+        if (dl && g.transb == 2) k = gemm_dl_kernel<T, 2, kStages, 64>;
     hipLaunchKernelGGL(k, grid, dim3(NT), 0, stream, g);
     MOAO_HIP_TRY(hipGetLastError());
     return after.run();
