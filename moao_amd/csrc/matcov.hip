@@ -76,9 +76,8 @@ constexpr int kCoef = 6;
 constexpr int kTabN = (kHi - kLo) * kSub + 2;
 constexpr double kTBorder = kXlim * kXlim;
 // Arguments below the table, those within rounding of the border, infinities and NaN take the direct
-// formulas.  kHiMin, kHiInf: high words of 2^kLo and of infinity (below kHiMin and from kHiInf on
-// is one unsigned comparison).
-constexpr unsigned kHiMin = (unsigned)(1023 + kLo) << 20, kHiInf = 0x7ff00000u;
+// formulas: interval numbers below 0 and from kInfinite on (one unsigned comparison).
+constexpr int kInfinite = (2047 - 1023 - kLo) << kSubBits;
 constexpr double kTBand = 1e-9;
 
 constexpr int kRows = 64;       // rows per workgroup (one wave tall)
@@ -178,18 +177,19 @@ __device__ __forceinline__ void vk_table(const double* tab, const double (&x)[N]
                                          double (&f)[N]) {
     bool direct[N], any = false;
     double t[N];
+    int iv[N];
 #pragma unroll
     for (int n = 0; n < N; ++n) {
         t[n] = fma(x[n], x[n], y[n] * y[n]) * (lk * lk);
-        direct[n] = (unsigned)__double2hiint(t[n]) - kHiMin >= kHiInf - kHiMin ||
-                    fabs(t[n] - kTBorder) < kTBand;
+        iv[n] = (int)((unsigned)__double2hiint(t[n]) >> (20 - kSubBits)) -
+                ((1023 + kLo) << kSubBits);
+        direct[n] = (unsigned)iv[n] >= (unsigned)kInfinite || fabs(t[n] - kTBorder) < kTBand;
         any = any || direct[n];
     }
 #pragma unroll
     for (int n = 0; n < N; ++n) {
         const unsigned hi = (unsigned)__double2hiint(t[n]);
-        int k = (int)(hi >> (20 - kSubBits)) - ((1023 + kLo) << kSubBits);
-        k = max(min(k + (t[n] > kTBorder ? 1 : 0), kTabN - 1), 0);
+        const int k = max(min(iv[n] + (t[n] > kTBorder ? 1 : 0), kTabN - 1), 0);
         const double w = __hiloint2double((int)((hi & ((1u << (20 - kSubBits)) - 1)) | 0x3ff00000u),
                                           __double2loint(t[n]));
         const double z = w - (1.0 + 0.5 / kSub);
