@@ -220,7 +220,6 @@ struct MixedWs {
     double* E;     // m x n residual / correction
     double* Ctm0;  // m x n copy of the right-hand side for the residuals
     double* W;     // p x n
-    double* P;     // kSumParts x (m or p) x p partial sums of range_sums
     double* Z;     // m x p
     double* Z2;    // m x p
     double* Sinv;  // p x p
@@ -254,7 +253,6 @@ static size_t mixed_layout(long n, long m, int p, int mode, std::vector<size_t>*
     take(sizeof(double) * m * n);
     take(sizeof(double) * m * n);
     take(sizeof(double) * q * n);
-    take(sizeof(double) * kSumParts * std::max(m, (long)q) * q);
     take(sizeof(double) * m * q);
     take(sizeof(double) * m * q);
     take(sizeof(double) * q * q);
@@ -307,15 +305,15 @@ int reconstructor_mixed_dev(long n, long m, const double* Cmm, long ldCmm, doubl
     MixedWs w{(float*)(b + offs[0]), (float*)(b + offs[1]), (float*)(b + offs[2]),
               (double*)(b + offs[3]), (double*)(b + offs[4]), (double*)(b + offs[5]),
               (double*)(b + offs[6]), (double*)(b + offs[7]), (double*)(b + offs[8]),
-              (double*)(b + offs[9]), (double*)(b + offs[10]), (double*)(b + offs[11]),
-              (int*)(b + offs[12]), (int*)(b + offs[13]), (int*)(b + offs[14])};
+              (double*)(b + offs[9]), (double*)(b + offs[10]), (int*)(b + offs[11]),
+              (int*)(b + offs[12]), (int*)(b + offs[13])};
     const int N = (int)n, M = (int)m;
     SplitWs sw{};
     const SplitWs* swp = nullptr;
     if (split) {
         const long ld = plane_ld(n);
-        sw = SplitWs{(unsigned short*)(b + offs[15]), (unsigned short*)(b + offs[16]),
-                     (unsigned short*)(b + offs[17]), ld, n * ld, n * ld, xr * ld};
+        sw = SplitWs{(unsigned short*)(b + offs[14]), (unsigned short*)(b + offs[15]),
+                     (unsigned short*)(b + offs[16]), ld, n * ld, n * ld, xr * ld};
         swp = &sw;
     }
 
@@ -378,13 +376,17 @@ int reconstructor_mixed_dev(long n, long m, const double* Cmm, long ldCmm, doubl
     if (int rc = trsm_right_lower_notrans<float>(n, w.C0, n, w.invL, all, s, nullptr, swp))
         return rc;
 
-    // Z = X U (rows x p, leading dimension rows)
-    auto times_u = [&](const double* X, long ldx, int rows, double* Z) -> int {
-        hipLaunchKernelGGL(range_sums, dim3((rows + 63) / 64, p, kSumParts), dim3(256), 0, s, X,
-                           ldx, rows, w.ends, w.P, p);
+    // Z = X U (rows x p, leading dimension rows); the parts' sums in `room` bytes at P, memory of the
+    // workspace that is free meanwhile, as many parts as it holds
+    auto times_u = [&](const double* X, long ldx, int rows, double* Z, void* P, size_t room) -> int {
         const long cells = (long)rows * p;
-        hipLaunchKernelGGL(range_sums_add, dim3((unsigned)((cells + 255) / 256)), dim3(256), 0, s,
-                           w.P, cells, kSumParts, Z);
+        const int parts = (int)std::min<size_t>(kSumParts, room / (sizeof(double) * cells));
+        double* to = parts > 1 ? static_cast<double*>(P) : Z;
+        hipLaunchKernelGGL(range_sums, dim3((rows + 63) / 64, p, std::max(parts, 1)), dim3(256), 0, s,
+                           X, ldx, rows, w.ends, to, p);
+        if (parts > 1)
+            hipLaunchKernelGGL(range_sums_add, dim3((unsigned)((cells + 255) / 256)), dim3(256), 0,
+                               s, to, cells, parts, Z);
         MOAO_HIP_TRY(hipGetLastError());
         return MOAO_OK;
     };
@@ -394,7 +396,7 @@ int reconstructor_mixed_dev(long n, long m, const double* Cmm, long ldCmm, doubl
     if (p) {
         hipLaunchKernelGGL(cvt_f32_f64, grid2(p, N), dim3(256), 0, s, w.X32 + m, xr, w.W, p, p, N);
         MOAO_HIP_TRY(hipGetLastError());
-        if (int rc = times_u(w.W, p, p, w.WU)) return rc;
+        if (int rc = times_u(w.W, p, p, w.WU, w.E, sizeof(double) * m * n)) return rc;
         std::vector<double> S((size_t)p * p);
         MOAO_HIP_TRY(hipMemcpyAsync(S.data(), w.WU, sizeof(double) * p * p, hipMemcpyDeviceToHost,
                                     s));
@@ -412,10 +414,10 @@ int reconstructor_mixed_dev(long n, long m, const double* Cmm, long ldCmm, doubl
         MOAO_HIP_TRY(hipMemcpyAsync(w.Sinv, Sinv.data(), sizeof(double) * p * p,
                                     hipMemcpyHostToDevice, s));
     }
-    // Y (FP64) -> X; X -= (X U) S^{-1} W
+    // Y (FP64) -> X; X -= (X U) S^{-1} W; the FP32 right-hand sides, of which Y is the copy, are free
     auto woodbury = [&](double* X, long ldx) -> int {
         if (!p) return MOAO_OK;
-        if (int rc = times_u(X, ldx, M, w.Z)) return rc;
+        if (int rc = times_u(X, ldx, M, w.Z, w.X32, sizeof(float) * xr * n)) return rc;
         auto g = gemm_args<double>(M, p, p, 1.0, w.Z, m, w.Sinv, p, 0, 0.0, w.Z2, m);
         if (int rc = gemm_f64(g, s)) return rc;
         g = gemm_args<double>(M, N, p, -1.0, w.Z2, m, w.W, p, 0, 1.0, X, ldx);

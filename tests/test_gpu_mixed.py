@@ -121,3 +121,16 @@ def test_mixed_reports_nonconvergence(tmp_path):
     rc, res, its = reconstructor_mixed_dev(C.shape[0], B.shape[0], dC.ptr, C.shape[0], dB.ptr,
                                            B.shape[0], t, 1e-15, 0, allow_noconv=True)
     assert rc == MOAO_ERR_NOCONV and its == 0 and res > 1e-15
+
+
+@pytest.mark.parametrize("mode", MODES)
+@pytest.mark.parametrize("nssp,nlgs", [(2, 1), (2, 3), (3, 4), (6, 2), (10, 5)])
+def test_mixed_smallest_systems(tmp_path, nssp, nlgs, mode):
+    """Systems of a few subapertures, whose right-hand sides leave room for one to a few of the
+    eight parts that the low-rank sums are cut into; bars as above."""
+    print(f"[mixed] nssp {nssp} nlgs {nlgs} mode {mode}", flush=True)
+    spec = systems.SystemSpec(diam=8.0, nssp=nssp, nlgs=nlgs, nngs=0, nlayer=2, seed=3)
+    s, atms = systems.make_system(str(tmp_path), spec)
+    err, res, its = _run(Tomo(s, atms[0]), mode=mode)
+    print(f"    err={err:.2e} resid={res:.2e} steps={its}", flush=True)
+    assert res <= 1e-11 and err <= 1e-6

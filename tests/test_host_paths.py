@@ -200,3 +200,20 @@ def test_gpu_gemm_shapes_reach_their_kernels(host):
             assert {k for k, _ in got[:-1]} == {"gemm_direct_kernel"}
             assert {a[2] for _, a in got[:-1]} == {"1", "2"}  # 16- and 32-row workgroups
             assert got[-1][0] == "gemm_dl_kernel"
+
+
+def test_footprint_of_a_mixed_request_piece_by_piece(host, tmp_path):
+    """Cmm, Ctm, the FP32 factor and right-hand sides with U^T, the leaves' inverses, residual and saved
+    Ctm, the Woodbury terms, norms, range ids, status and ranges, and the symmetric operand's
+    diagonal blocks: nothing for sums that find room in what is idle."""
+    from moao_amd import systems
+    s, a = systems.make_system(str(tmp_path), systems.SystemSpec(diam=8.0, nssp=12, nlgs=4, nngs=0,
+                                                                 nlayer=2, seed=3))
+    req = _words(host("serve", s, a[0], 1, 1, 0, 1), "request")[0]
+    n, m, p = req["n"], req["m"], 8
+    assert m < 448  # no larger workspace
+    leaves = -(-n // 128)
+    pieces = [8 * n * n, 8 * m * n, 4 * n * n, 4 * (m + p) * n, 4 * leaves * 128 * 128, 8 * m * n,
+              8 * m * n, 8 * p * n, 8 * m * p, 8 * m * p, 8 * p * p, 8 * p * p, 8 * 1024, 4 * n, 16,
+              4 * 2 * p, 8 * 128 * 128 * leaves]
+    assert req["footprint"] == sum(-(-b // 256) * 256 for b in pieces)
