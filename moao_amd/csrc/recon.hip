@@ -185,10 +185,10 @@ int trsmN_rec(const Tall<T>& p, long j0, long nn) {
             return rc;
         return MOAO_OK;
     }
-    // Segments in one launch (with split-BF16 updates too: inside a segment they run in FP32), up to the rows where the launches' reuse of their operands wins.  n =
-    // 2,048, launches -> segments, us: FP64 16 rows 1303 -> 1200, 1000 1362 -> 1248, 4000 1874 -> 1747,
-    // 8000 2513 -> 2494, 16000 3841 -> 3910; FP32 16 rows 1116 -> 1023, 16000 2659 -> 2599, 32000 4165 ->
-    // 4134.
+    // Segments in one launch (with split-BF16 updates too: inside a segment they run in FP32), up to
+    // the rows where the launches' reuse of their operands wins.  n = 2,048, launches -> segments, us:
+    // FP64 16 rows 1303 -> 1200, 1000 1362 -> 1248, 4000 1874 -> 1747, 8000 2513 -> 2494, 16000 3841 ->
+    // 3910; FP32 16 rows 1116 -> 1023, 16000 2659 -> 2599, 32000 4165 -> 4134.
     long rows_all = 0;
     for (const auto& g : G) rows_all += g.rows;
     if (nn <= kSegment && nn % kLeaf == 0 && rows_all <= (sizeof(T) == 8 ? 8192 : 16384)) {

@@ -2,9 +2,9 @@
 
 FP64 tolerance: |C - C_ref| <= 1e-13 * (|A| |op(B)| + |beta C|) elementwise-bound scale; FP32:
 2e-5 relative to the same scale, widened in proportion to K beyond 700 (sums of K products of
-O(1) numbers).  Shapes cover both tile sizes (launches of >= 512 128-row tiles and smaller
-ones), ragged M, N and K (K not a multiple of the 8-deep slice), and transb = 0, 1 and 2
-(symmetric B read from its lower triangle).
+O(1) numbers).  Shapes cover the direct kernel, both tile sizes of the slice kernels (128-row
+tiles: TILES_128), ragged M, N and K (K not a multiple of the 8-deep slice), and transb = 0, 1
+and 2 (symmetric B read from its lower triangle).
 """
 import numpy as np
 import pytest
@@ -16,8 +16,7 @@ pytestmark = pytest.mark.gpu
 
 CASES = [(128, 128, 16, 1, 0.0), (130, 77, 33, 1, 1.0), (300, 129, 200, 0, -1.0),
          (1, 1, 1, 0, 0.5), (257, 383, 700, 1, 1.0), (64, 500, 5, 0, 0.0),
-         # >= 512 tiles of 128 rows: the 128-row kernels; 561 tiles leave a short last wave
-         # whose tiles run as K chunks plus a reduction
+         # more than 512 tiles of 128 rows, which run as 64-row tiles
          (4133, 3900, 300, 1, 1.0), (4133, 3900, 301, 0, -1.0), (4133, 2100, 301, 0, 1.0),
          # symmetric B (K == N)
          (50, 300, 300, 2, 1.0), (257, 129, 129, 2, 0.0), (7, 16, 16, 2, 1.0),
@@ -181,8 +180,8 @@ def test_direct_in_place_panel():
 @pytest.mark.parametrize("M,N,K", [(3073, 2945, 257), (3103, 3009, 260), (3105, 2943, 8),
                                    (3136, 2977, 7), (3137, 3041, 264), (3199, 3039, 129)])
 def test_tiles_at_the_edge(M, N, K):
-    """op(B) = B^T launches of 128-row tiles whose last row and column tiles hold 1, 31, 33, 64, 65 or
-    127 rows and columns (waves that leave out their MFMAs) and whose K ends inside a slice.
+    """op(B) = B^T launches of 64-row tiles whose last 128 rows and columns hold 1, 31, 33, 64, 65 or 127
+    of them (waves that leave out their MFMAs) and whose K ends inside a slice.
     Tolerance: K products of values below 1, each rounded once and added once."""
     print(f"[gemm] edge tiles {M} x {N} x {K}", flush=True)
     rng = np.random.default_rng(M)

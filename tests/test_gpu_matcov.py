@@ -154,7 +154,7 @@ def test_whole_matrix_pair_kernel_is_bit_identical_to_element_tiles(tmp_path):
 @pytest.mark.parametrize("L0", [0.3, 2.0, 10.66, 25.0, 400.0, 1e5])
 def test_structure_function_range(tmp_path, L0):
     """Outer scales that take the structure function's arguments q = 2 pi r / L0 through the whole
-    range of its table and past both ends (q < 1/256, q > 45), and near the border of its two
+    range of its table and past both ends (q < 1/32, q > 45), and near the border of its two
     branches (r = 3/4 L0: 8 m for L0 = 10.66): Cmm, Ctm and Ctt within 1e-12 of the largest entry
     of the oracle's, as for the fixtures (second differences amplify the last-ulp differences)."""
     from moao_amd import systems

@@ -330,9 +330,9 @@ def test_leaf_edges(n):
                                       (384, 16, 1), (385, 20, 1), (450, 31, 3), (511, 16, 1), (512, 48, 1),
                                       (513, 16, 1), (640, 7, 1), (1100, 40, 2), (1409, 16, 1)])
 def test_backward_solve_segments(n, m, ngal):
-    """The backward solve's segments of two, three and four leaves, the last one whole or down to a
-    single column, rows at the edges of the 16-row workgroups and more targets than one launch
-    takes: backward error of R in both precisions (bars as above), and every target as alone."""
+    """The backward solve's segments of two, three and four whole leaves, columns that end in a leaf cut
+    down to a single column (those are single products, before and after segments), rows at the
+    edges of the 16-row workgroups and more targets than one launch takes: backward error of R in both precisions (bars as above), and every target as alone."""
     from moao_amd.reconstructor import sreconstructor
     print(f"[recon] segments n={n} m={m} ngal={ngal}", flush=True)
     rng = np.random.default_rng(n + m)
