@@ -82,8 +82,9 @@ int cee_cvv_batched_dev(long n, long m, long nact, long ngal, const double* Cmm,
     auto Cee_ = [&](long g) { return Cee + g * ldCee * m; };
     auto Cvv_ = [&](long g) { return Cvv + g * ldCvv * nact; };
     auto Tmp_ = [&](long g) { return Tmp + g * ldTmp * m; };
-    // Stream-ordered scratch, so calls on different streams never share it: Cmm in full (step 2;
-    // without it that step runs on the fallback kernel) and step 1's product.
+    // Stream-ordered scratch, so calls on different streams never share it: Cmm in full or its
+    // diagonal blocks (step 2; without either that step runs on the fallback kernel) and step 1's
+    // product.
     SymWork sym;
     sym_alloc(sym, m * std::min<long>(ngal, kMaxSeg), n, s);
     struct Scratch {

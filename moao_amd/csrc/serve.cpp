@@ -244,6 +244,7 @@ int moao_server::run_body(moao::Request& r, moao::Slot& sl) {
             }
         }
     } while (false);
+    sl.tables.space = nullptr;  // the block goes
     if (rc) r.error = moao_last_error();
     hipError_t e1 = hipFreeAsync(block, s);
     hipError_t e2 = hipStreamSynchronize(s);

@@ -156,3 +156,22 @@ def test_repeated_shapes_replay_graphs(tmp_path):
         assert reconstructor_dev(n, m, dC.ptr, n, dB.ptr, m, 1) == 0
         synchronize()
         assert np.array_equal(r["R"], dB.to_host())
+
+
+def test_mixed_request_in_its_least_workspace(tmp_path):
+    """With a budget of the least footprint a mixed request's residuals read the symmetric operand in
+    place, with a wide one they take it written out: the same R, bit for bit."""
+    spec = systems.SystemSpec(diam=8.0, nssp=24, nlgs=2, nngs=1, lgs_ring_diam_as=60.0,
+                              ngs_field_diam_as=60.0, nlayer=2, r0=0.15, seed=23)
+    s, atms = systems.make_system(str(tmp_path), spec)
+    t = Tomo(s, atms[0])
+    n, m = t.nmeas(), t.nmeasts()
+    assert m >= 448  # rows from which the operand is written out
+    print(f"[serve] mixed n={n} m={m} in its least workspace", flush=True)
+    with Server(slots=1) as srv:
+        wide = srv.wait(srv.submit(s, atms[0], 0, MOAO_MIXED_FP32, n_m=(n, m)))
+    least = wide["footprint"] - (8 * n * n - 8 * 128 * 128 * -(-n // 128))
+    with Server(slots=1, hbm_budget=least) as srv:
+        res = srv.wait(srv.submit(s, atms[0], 0, MOAO_MIXED_FP32, n_m=(n, m)))
+        assert srv.stats()["peak_bytes"] == res["footprint"] == least
+    assert res["status"] == 0 and np.array_equal(res["R"], wide["R"])
